@@ -1,6 +1,10 @@
 // Device kernels of liblina_hip (gfx950 / CDNA4, wave64).
 //
-// Row kernels (SpMV, multicolour SOR, Jacobi) share one structure:
+// Row kernels (SpMV, multicolour SOR, Jacobi) come in two forms.  Matrices
+// whose rows of a wavefront are of about one length (the finest levels, the
+// Galerkin levels, most transfers) are streamed from a sliced copy (Slices,
+// k_sell_*): one wavefront per slice, one or more lanes per row, no LDS and no
+// barrier.  The others (irregular coarsest levels) keep this structure:
 //
 //   phase 1  all 256 lanes of a workgroup stream the value and column arrays
 //            of a block of consecutive rows (<= 2048 entries, coalesced, each
@@ -282,6 +286,252 @@ __global__ __launch_bounds__(TPB) void k_spmv(int nblk, const int2* __restrict__
         if (!block_live(bspec, active, bb)) continue;
         spmv_block<VT, XT, MODE, LPR>(bb, bk, rp, ci, cs, cbase, v, x, b, y, part, w, epi, prod);
         __syncthreads();  // prod is restaged by the next block
+    }
+}
+
+// ------------------------------------------------------- sliced row kernels
+//
+// What bounds them: the stream of values and codes (6 or 10 bytes an entry)
+// plus the gathers of x, which a slice's layout makes nearly contiguous.  The
+// block form below spends its time elsewhere: a dependent chain of block
+// bounds, entries, gathers, LDS stage, barrier and row sums per workgroup.
+// Products with matrices of the shape of (MI355X, block form -> slices):
+// 2.1M rows x 14, FP32 57 -> 37 us, FP64 76 -> 65 us; 403k x 14, FP32 12.9 ->
+// 8.6 us; 148k x 38, FP32 12.0 -> 8.7 us; 20k x 117, FP32 6.8 -> 5.0 us;
+// 16k x 7, FP64 3.6 -> 2.8 us.
+// T = 1 adds a row's products one after another in column order, as the block
+// form's LPR = 1 does (the same bits); T > 1 adds T interleaved partial sums
+// with a fixed xor tree.
+
+// the lane's place in slice s: its row (of nr), entry offset t and row data
+struct SliceLane {
+    int row, t, len, p0, steps, T, b0, b1;
+    size_t base;
+    bool ok;
+};
+
+template <typename VT>
+__device__ __forceinline__ SliceLane slice_lane(const Slices<VT>& S, int s, const int* __restrict__ rp) {
+    SliceLane L;
+    const int lane = threadIdx.x % WAVE;
+    // one slice a wavefront: its head comes by one scalar load
+    const SliceHead h = S.head[__builtin_amdgcn_readfirstlane(s)];
+    const int lr = 6 - S.lt;  // log2 of the rows a slice holds
+    L.T = 1 << S.lt;
+    L.t = lane >> lr;
+    L.row = h.row0 + (lane & ((1 << lr) - 1));
+    L.ok = L.row < h.row1;
+    L.steps = L.ok ? h.steps : 0;  // lanes past the slice's rows load nothing
+    L.base = (size_t)h.step0 * WAVE + lane;
+    L.b0 = h.b0;
+    L.b1 = h.b1;
+    L.p0 = L.len = 0;
+    if (L.ok) {
+        L.p0 = rp[L.row];
+        L.len = rp[L.row + 1] - L.p0;
+    }
+    return L;
+}
+
+// f(e, a, a * x_col) for the lane's entries e of its row, ascending.  U steps
+// are in flight: their values and codes, then their gathers; steps past the
+// slice's end load its last step again (in bounds).
+template <int U, bool NT, typename VT, typename XT, typename F>
+__device__ __forceinline__ void slice_entries(const Slices<VT>& S, const SliceLane& L, const int* __restrict__ ci,
+                                              const XT* __restrict__ x, F&& f) {
+    const VT* vp = S.v + L.base;
+    const uint16_t* cp = S.cs + L.base;
+    for (int j = 0; j < L.steps; j += U) {
+        VT a[U];
+        int c[U];
+        XT xv[U];
+        if (L.b0 >= 0) {
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int jj = min(j + u, L.steps - 1) * WAVE;
+                const int o = (int)ld_stream<NT>(cp + jj);
+                a[u] = ld_stream<NT>(vp + jj);
+                c[u] = ((o & 0x8000) ? L.b1 : L.b0) + (o & 0x7fff);
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int e = (j + u) * L.T + L.t;
+                c[u] = e < L.len ? ci[L.p0 + e] : 0;
+                a[u] = ld_stream<NT>(vp + min(j + u, L.steps - 1) * WAVE);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) xv[u] = x[c[u]];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int e = (j + u) * L.T + L.t;
+            if (e < L.len) f(e, (XT)a[u], (XT)a[u] * xv[u]);
+        }
+    }
+}
+
+// the sum over a row's T lanes, in every one of them
+template <typename XT>
+__device__ __forceinline__ XT slice_sum(XT v, int T) {
+    for (int o = WAVE / 2; o >= WAVE / T; o >>= 1) v += __shfl_xor(v, o, WAVE);
+    return v;
+}
+
+template <typename VT, typename XT, int MODE, int U, bool NT>
+__global__ __launch_bounds__(TPB) void k_sell_spmv(const Slices<VT> S, const int* __restrict__ rp,
+                                                   const int* __restrict__ ci, const XT* __restrict__ x,
+                                                   const XT* __restrict__ b, XT* __restrict__ y,
+                                                   double* __restrict__ part, const XT* __restrict__ w,
+                                                   const Epi<VT, XT> epi, const int2* __restrict__ bspec,
+                                                   const double* __restrict__ active) {
+    const int bb = xcd_block(blockIdx.x, gridDim.x);
+    const int s = bb * SLICES_PER_BLOCK + threadIdx.x / WAVE;
+    double mine = 0.0;
+    if (s < S.ns && block_live(bspec, active, s)) {
+        const SliceLane L = slice_lane(S, s, rp);
+        XT base = (XT)0;
+        if (L.ok && L.t == 0) base = spmv_base<MODE>(L.row, b, y);
+        XT sum = (XT)0;
+        slice_entries<U, NT>(S, L, ci, x, [&](int, XT, XT p) { sum += p; });
+        sum = slice_sum(sum, L.T);
+        if (L.ok && L.t == 0) {
+            const XT out = spmv_out<VT, XT, MODE>(sum, base, L.row, y, epi);
+            if (part) mine = (double)out * (double)(w ? w[L.row] : out);
+        }
+    }
+    if (part) {
+        const double t = block_sum(mine);
+        if (threadIdx.x == 0) part[bb] = t;
+    }
+}
+
+// one colour of multicolour SOR on the slices [s0, s0 + ns) of the
+// colour-permuted copy (k_mcsor's arithmetic); the diagonal is picked out of
+// the stream
+template <typename VT, typename XT, int U, bool NT>
+__global__ __launch_bounds__(TPB) void k_sell_mcsor(const Slices<VT> S, int s0, int ns, const int* __restrict__ rp,
+                                                    const int* __restrict__ ci, const int* __restrict__ dpos,
+                                                    const int* __restrict__ perm, const XT* __restrict__ f,
+                                                    XT* __restrict__ x, XT omega, const int2* __restrict__ bspec,
+                                                    const double* __restrict__ active) {
+    const int k = xcd_block(blockIdx.x, gridDim.x) * SLICES_PER_BLOCK + threadIdx.x / WAVE;
+    if (k >= ns || !block_live(bspec, active, s0 + k)) return;
+    const SliceLane L = slice_lane(S, s0 + k, rp);
+    int i = 0, dj = -1;
+    XT fi = (XT)0, xi = (XT)0;
+    if (L.ok) {
+        i = perm[L.row];
+        dj = dpos[L.row] - L.p0;
+        fi = f[i];
+        xi = x[i];
+    }
+    // T = 1: f_i - a_i1 x_1 - ... in order; else f_i + (-(sum of the products))
+    XT acc = L.T == 1 ? fi : (XT)0, d = (XT)0;
+    slice_entries<U, NT>(S, L, ci, (const XT*)x, [&](int e, XT a, XT p) {
+        if (e == dj) d = a;
+        else acc -= p;
+    });
+    if (L.T > 1) {
+        acc = fi + slice_sum(acc, L.T);
+        d = slice_sum(d, L.T);
+    }
+    if (L.ok && L.t == 0) x[i] = ((XT)1 - omega) * xi + omega * acc / d;
+}
+
+// Jacobi sweep x = J(xo) (k_jacobi's arithmetic)
+template <typename VT, typename XT, int KIND, int U, bool NT>
+__global__ __launch_bounds__(TPB) void k_sell_jacobi(const Slices<VT> S, const int* __restrict__ rp,
+                                                     const int* __restrict__ ci, const int* __restrict__ dpos,
+                                                     const VT* __restrict__ l1, const XT* __restrict__ f,
+                                                     const XT* __restrict__ xo, XT* __restrict__ x, int nlim,
+                                                     const int2* __restrict__ bspec,
+                                                     const double* __restrict__ active) {
+    const int s = xcd_block(blockIdx.x, gridDim.x) * SLICES_PER_BLOCK + threadIdx.x / WAVE;
+    if (s >= S.ns || !block_live(bspec, active, s)) return;
+    const SliceLane L = slice_lane(S, s, rp);
+    const int r = L.row;
+    int dj = -1;
+    XT fr = (XT)0, xr = (XT)0;
+    VT lr = (VT)1;
+    if (L.ok) {
+        fr = f[r];
+        xr = xo[r];
+        if (KIND == JAC_REF) dj = dpos[r] - L.p0;
+        else lr = l1[r];
+    }
+    XT acc = L.T == 1 ? fr : (XT)0, d = (XT)0;
+    slice_entries<U, NT>(S, L, ci, xo, [&](int e, XT a, XT p) {
+        if (KIND == JAC_REF && e == dj) d = a;
+        else acc -= p;
+    });
+    if (L.T > 1) {
+        acc = fr + slice_sum(acc, L.T);
+        if (KIND == JAC_REF) d = slice_sum(d, L.T);
+    }
+    if (L.ok && L.t == 0) {
+        if (KIND == JAC_REF) x[r] = r < nlim ? acc / d : xr;
+        else x[r] = xr + acc / lr;
+    }
+}
+
+// bases and codes of one slice per wavefront: base 0 is the smallest column,
+// base 1 the smallest one more than 32767 beyond it; b0 = -1 when the
+// columns need a third
+__global__ __launch_bounds__(TPB) void k_slice_columns(int ns, int lt, SliceHead* __restrict__ head,
+                                                       const int* __restrict__ rp, const int* __restrict__ ci,
+                                                       uint16_t* __restrict__ cs) {
+    const int s = blockIdx.x * SLICES_PER_BLOCK + threadIdx.x / WAVE;
+    if (s >= ns) return;
+    const int lane = threadIdx.x % WAVE;
+    const int step0 = head[s].step0, steps = head[s].steps, row1 = head[s].row1;
+    const int lr = 6 - lt, T = 1 << lt, t = lane >> lr, row = head[s].row0 + (lane & ((1 << lr) - 1));
+    int p0 = 0, len = 0;
+    if (row < row1) {
+        p0 = rp[row];
+        len = rp[row + 1] - p0;
+    }
+    constexpr int NONE = 0x7fffffff;
+    auto wave_min = [](int v) {
+        for (int o = WAVE / 2; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o, WAVE));
+        return v;
+    };
+    int lo = NONE, hi = NONE, far = 0;
+    for (int e = t; e < len; e += T) lo = min(lo, ci[p0 + e]);
+    lo = wave_min(lo);
+    if (lo == NONE) lo = 0;  // no entries
+    for (int e = t; e < len; e += T)
+        if (ci[p0 + e] - lo > 32767) hi = min(hi, ci[p0 + e]);
+    hi = wave_min(hi);
+    if (hi == NONE) hi = lo;
+    for (int e = t; e < len; e += T)
+        if (ci[p0 + e] - lo > 32767 && ci[p0 + e] - hi > 32767) far = -1;
+    far = wave_min(far);
+    if (lane == 0) {
+        head[s].b0 = far < 0 ? -1 : lo;
+        head[s].b1 = far < 0 ? -1 : hi;
+    }
+    for (int j = 0; j < steps; j++) {
+        const int e = j * T + t;
+        int code = 0;
+        if (far == 0 && e < len) {
+            const int c = ci[p0 + e];
+            code = c - lo <= 32767 ? c - lo : 0x8000 | (c - hi);
+        }
+        cs[((size_t)step0 + j) * WAVE + lane] = (uint16_t)code;
+    }
+}
+
+template <typename VT>
+__global__ __launch_bounds__(TPB) void k_slice_values(const Slices<VT> S, const int* __restrict__ rp,
+                                                      const VT* __restrict__ v, VT* __restrict__ out) {
+    const int s = blockIdx.x * SLICES_PER_BLOCK + threadIdx.x / WAVE;
+    if (s >= S.ns) return;
+    const SliceLane L = slice_lane(S, s, rp);
+    const int steps = S.head[s].steps;
+    for (int j = 0; j < steps; j++) {
+        const int e = j * L.T + L.t;
+        out[L.base + (size_t)j * WAVE] = e < L.len ? v[L.p0 + e] : (VT)0;
     }
 }
 
@@ -2098,6 +2348,39 @@ static inline int grid_for(int n, int cap = 4096) {
         default: { constexpr int L = 32; __VA_ARGS__; break; } \
     }
 
+// a sliced kernel's steps in flight and load kind
+#define LINA_SLICE_DISPATCH(S, ...)                                                                       \
+    if ((S).nt) {                                                                                         \
+        constexpr bool NT = true;                                                                         \
+        if ((S).unroll == 4) { constexpr int U = 4; __VA_ARGS__; }                                        \
+        else if ((S).unroll == 7) { constexpr int U = 7; __VA_ARGS__; }                                   \
+        else { constexpr int U = 8; __VA_ARGS__; }                                                        \
+    } else {                                                                                              \
+        constexpr bool NT = false;                                                                        \
+        if ((S).unroll == 4) { constexpr int U = 4; __VA_ARGS__; }                                        \
+        else if ((S).unroll == 7) { constexpr int U = 7; __VA_ARGS__; }                                   \
+        else { constexpr int U = 8; __VA_ARGS__; }                                                        \
+    }
+
+static inline int slice_blocks(int ns) { return (ns + SLICES_PER_BLOCK - 1) / SLICES_PER_BLOCK; }
+
+template <typename VT>
+void slice_columns(hipStream_t st, const DMat<VT>& D) {
+    if (D.sl.ns == 0) return;
+    hipLaunchKernelGGL(k_slice_columns, dim3(slice_blocks(D.sl.ns)), dim3(TPB), 0, st, D.sl.ns, D.sl.lt, D.sl.head,
+                       D.rp, D.ci, D.sl.cs);
+}
+template void slice_columns<double>(hipStream_t, const DMat<double>&);
+template void slice_columns<float>(hipStream_t, const DMat<float>&);
+
+template <typename VT>
+void slice_values(hipStream_t st, const DMat<VT>& D) {
+    if (D.sl.ns == 0) return;
+    hipLaunchKernelGGL((k_slice_values<VT>), dim3(slice_blocks(D.sl.ns)), dim3(TPB), 0, st, D.sl, D.rp, D.v, D.sl.v);
+}
+template void slice_values<double>(hipStream_t, const DMat<double>&);
+template void slice_values<float>(hipStream_t, const DMat<float>&);
+
 // workgroups of a row-kernel launch: one per row block, or a persistent grid
 // of at most LINA_SPMV_GRID workgroups (rounded down to a multiple of 8; read
 // from the environment once, 0: off)
@@ -2112,10 +2395,27 @@ static int row_grid(int nblk) {
 
 template <typename VT, typename XT>
 int spmv(hipStream_t st, const DMat<VT>& A, const XT* x, const XT* b, XT* y, int mode, double* part, const XT* w,
-         const Epi<VT, XT>* epi) {
-    if (A.nblk == 0) return 0;
-    dim3 g(row_grid(A.nblk)), t(TPB);
+         const Epi<VT, XT>* epi, bool blocks) {
+    if (A.n == 0) return 0;
     const Epi<VT, XT> e = epi ? *epi : Epi<VT, XT>{};
+    if (A.sl.ns && !(blocks && A.nblk)) {
+        const int wg = slice_blocks(A.sl.ns);
+#define LINA_SELL_MODE(M)                                                                                           \
+    LINA_SLICE_DISPATCH(A.sl, hipLaunchKernelGGL((k_sell_spmv<VT, XT, M, U, NT>), dim3(wg), dim3(TPB), 0, st, \
+                                                 A.sl, A.rp, A.ci, x, b, y, part, w, e, A.bspec, A.active))
+        switch (mode) {
+            case MODE_SET: LINA_SELL_MODE(MODE_SET); break;
+            case MODE_OUTER: LINA_SELL_MODE(MODE_OUTER); break;
+            case MODE_RES: LINA_SELL_MODE(MODE_RES); break;
+            case MODE_ADD: LINA_SELL_MODE(MODE_ADD); break;
+            case MODE_ADDB: LINA_SELL_MODE(MODE_ADDB); break;
+            case MODE_SETX: LINA_SELL_MODE(MODE_SETX); break;
+            default: return -1;
+        }
+#undef LINA_SELL_MODE
+        return wg;
+    }
+    dim3 g(row_grid(A.nblk)), t(TPB);
 #define LINA_SPMV_MODE(M)                                                                                       \
     LINA_LPR_DISPATCH(A.lpr, hipLaunchKernelGGL((k_spmv<VT, XT, M, L>), g, t, 0, st, A.nblk, A.bk, A.rp, A.ci, \
                                                 A.cs, A.cb, A.v, x, b, y, part, w, e, A.bspec, A.active))
@@ -2132,23 +2432,30 @@ int spmv(hipStream_t st, const DMat<VT>& A, const XT* x, const XT* b, XT* y, int
     return A.nblk;
 }
 template int spmv<double, double>(hipStream_t, const DMat<double>&, const double*, const double*, double*, int,
-                                  double*, const double*, const Epi<double, double>*);
+                                  double*, const double*, const Epi<double, double>*, bool);
 
 // the outer CG's y = A x (MODE_OUTER, FP64) with HIP events recorded by the
 // launch itself at the kernel's start and end (hipExtLaunchKernel), so that
 // their interval is the kernel's own duration
 int spmv_outer_timed(hipStream_t st, const DMat<double>& A, const double* x, double* y, double* part,
-                     const double* w, hipEvent_t e0, hipEvent_t e1) {
-    if (A.nblk == 0) return 0;
-    dim3 g(row_grid(A.nblk)), t(TPB);
+                     const double* w, hipEvent_t e0, hipEvent_t e1, bool blocks) {
+    if (A.n == 0) return 0;
     const Epi<double, double> e{};
+    if (A.sl.ns && !(blocks && A.nblk)) {
+        const int wg = slice_blocks(A.sl.ns);
+        LINA_SLICE_DISPATCH(A.sl, hipExtLaunchKernelGGL((k_sell_spmv<double, double, MODE_OUTER, U, NT>), dim3(wg),
+                                                        dim3(TPB), 0, st, e0, e1, 0, A.sl, A.rp, A.ci, x,
+                                                        (const double*)nullptr, y, part, w, e, A.bspec, A.active))
+        return wg;
+    }
+    dim3 g(row_grid(A.nblk)), t(TPB);
     LINA_LPR_DISPATCH(A.lpr, hipExtLaunchKernelGGL((k_spmv<double, double, MODE_OUTER, L>), g, t, 0, st, e0, e1, 0,
                                                    A.nblk, A.bk, A.rp, A.ci, A.cs, A.cb, A.v, x,
                                                    (const double*)nullptr, y, part, w, e, A.bspec, A.active))
     return A.nblk;
 }
 template int spmv<float, float>(hipStream_t, const DMat<float>&, const float*, const float*, float*, int, double*,
-                                const float*, const Epi<float, float>*);
+                                const float*, const Epi<float, float>*, bool);
 
 template <typename XT>
 int dot_part(hipStream_t st, int n, const XT* a, const XT* b, double* part) {
@@ -2334,6 +2641,12 @@ template <typename VT, typename XT>
 void mcsor_colour(hipStream_t st, const DMat<VT>& Ac, int blk0, int nblk, const int* perm, const XT* f, XT* x,
                   XT omega) {
     if (nblk <= 0) return;
+    if (Ac.sl.ns) {
+        LINA_SLICE_DISPATCH(Ac.sl, hipLaunchKernelGGL((k_sell_mcsor<VT, XT, U, NT>), dim3(slice_blocks(nblk)), dim3(TPB),
+                                                      0, st, Ac.sl, blk0, nblk, Ac.rp, Ac.ci, Ac.dpos, perm, f, x,
+                                                      omega, Ac.bspec, Ac.active))
+        return;
+    }
     LINA_LPR_DISPATCH(Ac.lpr, hipLaunchKernelGGL((k_mcsor<VT, XT, L>), dim3(nblk), dim3(TPB), 0, st, nblk, blk0,
                                                  Ac.bk, Ac.rp, Ac.ci, Ac.cs, Ac.cb, Ac.v, Ac.dpos, perm, f, x, omega, Ac.bspec,
                                                  Ac.active))
@@ -2387,8 +2700,18 @@ template void sor_lex<float, float>(hipStream_t, const DMat<float>&, int, const 
 
 template <typename VT, typename XT>
 void jacobi(hipStream_t st, const DMat<VT>& A, int kind, const XT* f, const XT* xo, XT* x, int nlim) {
-    if (A.nblk == 0) return;
-    dim3 g(A.nblk), t(TPB);
+    if (A.n == 0) return;
+    const dim3 g(A.sl.ns ? slice_blocks(A.sl.ns) : A.nblk), t(TPB);
+    if (A.sl.ns) {
+        if (kind == JAC_REF) {
+            LINA_SLICE_DISPATCH(A.sl, hipLaunchKernelGGL((k_sell_jacobi<VT, XT, JAC_REF, U, NT>), g, t, 0, st, A.sl,
+                                                         A.rp, A.ci, A.dpos, A.l1, f, xo, x, nlim, A.bspec, A.active))
+        } else {
+            LINA_SLICE_DISPATCH(A.sl, hipLaunchKernelGGL((k_sell_jacobi<VT, XT, JAC_L1, U, NT>), g, t, 0, st, A.sl,
+                                                         A.rp, A.ci, A.dpos, A.l1, f, xo, x, nlim, A.bspec, A.active))
+        }
+        return;
+    }
     if (kind == JAC_REF) {
         LINA_LPR_DISPATCH(A.lpr, hipLaunchKernelGGL((k_jacobi<VT, XT, JAC_REF, L>), g, t, 0, st, A.nblk, A.bk, A.rp,
                                                     A.ci, A.cs, A.cb, A.v, A.dpos, A.l1, f, xo, x, nlim, A.bspec,

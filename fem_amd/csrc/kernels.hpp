@@ -57,14 +57,41 @@ enum {
     S_COUNT = 16
 };
 
-// device CSR with its LDS row-block schedule
+// Sliced copy of a matrix, the form the row kernels stream where its padding
+// is small (plan_slices): a slice is up to 64 / T consecutive rows, one
+// wavefront.  Step j of a slice holds 64 entries at v[64 (step0 + j) + lane]:
+// lane = t (64 / T) + i is entry j T + t of the slice's row i (zero and code 0
+// past the row's end), so that every load of values and codes is one
+// contiguous run and neighbouring lanes gather neighbouring entries of x.
+// Columns are 16-bit codes against the slice's two bases as in DMat::cs;
+// b0 < 0: the slice's columns are read from the CSR's ci.
+struct alignas(32) SliceHead {
+    int row0 = 0, row1 = 0;    // its rows [row0, row1)
+    int step0 = 0, steps = 0;
+    int b0 = 0, b1 = 0;
+    int pad[2] = {0, 0};
+};
+template <typename VT>
+struct Slices {
+    int ns = 0;          // slices (0: no sliced copy)
+    int lt = 0;          // log2 T
+    int unroll = 8;      // steps in flight per lane: 4, 7 or 8
+    bool nt = false;     // nontemporal loads of the streamed arrays
+    size_t steps = 0;    // of all slices
+    SliceHead* head = nullptr;
+    uint16_t* cs = nullptr;
+    VT* v = nullptr;
+};
+
+// device CSR with its sliced copy or its LDS row-block schedule
 template <typename VT>
 struct DMat {
     int n = 0, ncols = 0, nnz = 0;
     int* rp = nullptr;
     int* ci = nullptr;
     VT* v = nullptr;
-    int nblk = 0;
+    Slices<VT> sl;
+    int nblk = 0;        // row blocks (0: only the sliced copy)
     int2* bk = nullptr;  // nblk+1 (first row, first entry) pairs of the row blocks
     // 16-bit column codes: a block's columns form at most two clusters, each
     // spanning < 32768, with base columns cb[block] = (b0, b1); an entry's
@@ -73,8 +100,8 @@ struct DMat {
     uint16_t* cs = nullptr;
     int2* cb = nullptr;
     double idx_bytes = 0;  // column index bytes the row kernels read (host-side accounting)
-    // batches: the first and last system of each row block's rows, and the
-    // systems' active flags; a block whose systems are all inactive is skipped
+    // batches: the first and last system of each row block's (slice's) rows,
+    // and the systems' active flags; a block whose systems are all inactive is skipped
     int2* bspec = nullptr;
     const double* active = nullptr;
     int lpr = 1;         // lanes reducing one row from LDS: 1 (sequential), 4, 8, 16, 32
@@ -109,14 +136,31 @@ inline int lanes_per_row(double mean_len) {
     return 32;
 }
 
-// returns the number of block partials written to part (if part != nullptr)
+// wavefronts (slices) of a row-kernel workgroup over a sliced matrix
+constexpr int SLICES_PER_BLOCK = 4;
+// the column codes and bases of D.sl (rows and steps set) from D's CSR
+template <typename VT>
+void slice_columns(hipStream_t st, const DMat<VT>& D);
+// D.sl.v from D.v (after every change of D.v; nothing without a sliced copy)
+template <typename VT>
+void slice_values(hipStream_t st, const DMat<VT>& D);
+
+// the larger workgroup count of a row kernel over A's forms
+template <typename VT>
+inline int row_blocks(const DMat<VT>& A) {
+    const int s = (A.sl.ns + SLICES_PER_BLOCK - 1) / SLICES_PER_BLOCK;
+    return s > A.nblk ? s : A.nblk;
+}
+
+// returns the number of block partials written to part (if part != nullptr);
+// blocks: the row-block form where A has both
 template <typename VT, typename XT>
 int spmv(hipStream_t st, const DMat<VT>& A, const XT* x, const XT* b, XT* y, int mode, double* part, const XT* w,
-         const Epi<VT, XT>* epi = nullptr);
+         const Epi<VT, XT>* epi = nullptr, bool blocks = false);
 // MODE_OUTER y = A x in FP64 with events recorded at the kernel's own start
 // and end (the outer CG's timed launches)
 int spmv_outer_timed(hipStream_t st, const DMat<double>& A, const double* x, double* y, double* part,
-                     const double* w, hipEvent_t e0, hipEvent_t e1);
+                     const double* w, hipEvent_t e0, hipEvent_t e1, bool blocks = false);
 // block partials of a.b: at most DOT_PART_MAX of them (the grid's cap)
 constexpr int DOT_PART_MAX = 1024;
 template <typename XT>
@@ -199,6 +243,7 @@ int pcg_xr(hipStream_t st, int n, double* X, double* R, const double* P, const d
 void axpy_s(hipStream_t st, int n, double* x, const double* y, const double* scal, int slot_a, int slot_b,
             double sign);
 void axpby(hipStream_t st, int n, double a, double* x, double b, const double* y);
+// one colour: its row blocks (slices of a sliced copy) [blk0, blk0 + nblk)
 template <typename VT, typename XT>
 void mcsor_colour(hipStream_t st, const DMat<VT>& Ac, int blk0, int nblk, const int* perm, const XT* f, XT* x,
                   XT omega);

@@ -170,7 +170,7 @@ static bool tri_pack(const Csr& T, bool upper, bool pattern_only, const std::vec
     return true;
 }
 
-// blocks: also the LDS row blocks of the SpMV (the factors need only the CSR)
+// blocks: also the slices or LDS row blocks of the SpMV (the factors need only the CSR)
 static dev::DMat<double> upload_csr(const Csr& A, DevBuffers& B, hipStream_t st, bool blocks = true) {
     dev::DMat<double> D;
     D.n = A.n;
@@ -180,6 +180,7 @@ static dev::DMat<double> upload_csr(const Csr& A, DevBuffers& B, hipStream_t st,
     D.ci = kupload(A.ci, B, st);
     D.v = kupload(A.v, B, st);
     if (!blocks) return D;
+    if (slice_matrix(A, D, B, st)) return D;
     // LDS row blocks for the SpMV (same builder rule as the AMG levels)
     std::vector<int> starts;
     build_blocks(A, 0, A.n, dev::block_nnz<double>(), starts);
@@ -345,6 +346,7 @@ void IluSystem::refactor_p(const Csr& A) {
         // A_ keeps the pattern; its values are not refreshed (only dA_'s are)
         hip_check(hipMemcpyAsync(dA_.v, A.v.data(), A.v.size() * sizeof(double), hipMemcpyHostToDevice, stream_),
                   "h2d");
+        dev::slice_values<double>(stream_, dA_);
     }
     numeric();
 }
@@ -354,6 +356,7 @@ bool IluSystem::refactor_device(const double* d_val) {
     const int nnz = A_.nnz();
     if (dvpos_) dev::permute_idx(stream_, nnz, dvpos_, d_val, dA_.v);
     else hip_check(hipMemcpyAsync(dA_.v, d_val, (size_t)nnz * sizeof(double), hipMemcpyDeviceToDevice, stream_), "d2d");
+    dev::slice_values<double>(stream_, dA_);
     numeric();
     return true;
 }
@@ -550,7 +553,7 @@ void IluSystem::upload(bool pattern_levels_in) {
         vYu_ = kalloc<double>(n, B);
         pack_values();
     }
-    part_ = kalloc<double>(std::max(4096, dA_.nblk + 16) * 40, B);
+    part_ = kalloc<double>(std::max(4096, dev::row_blocks(dA_) + 16) * 40, B);
     scal_ = kalloc<double>(64, B);
     fail_ = kalloc<int>(1, B);
     dev::fill(st, 64, scal_, 0.0);

@@ -163,9 +163,6 @@ static long column_codes(const Csr& A, const std::vector<int>& starts_with_end, 
     return coded;
 }
 
-// share: a copy of A with other values uploaded before; its row pointers and
-// column indices are reused, and its 16-bit offsets too when its schedule
-// (share_starts) is the same
 // first and last system (seg: a batch's row offsets per system) of each row
 // block's rows; row r of A is row row_ids[r] of the level (ascending in a block)
 static std::vector<int2> block_systems(const std::vector<int>& starts_with_end, const std::vector<int>& seg,
@@ -184,13 +181,141 @@ static std::vector<int2> block_systems(const std::vector<int>& starts_with_end, 
     return bs;
 }
 
+// The slices of a matrix (dev::Slices) or none: groups: row offsets that no
+// slice may straddle (a colour-permuted copy's colours; empty: one group).
+//
+// T lanes a row.  free_order false: the block form's lanes_per_row, so that a
+// row's products are added in its order (the same bits); with blocks given and
+// T = 1 each workgroup also keeps the rows of one block, so that a product's
+// block partials (P.Q of the outer CG) are the block form's.  free_order true:
+// one lane for short rows (means up to 24 entries) unless that leaves most of
+// the chip idle (below 1,024 wavefronts), then four of at least 3 entries
+// each; for longer rows as many as make 4,096 wavefronts (16 per compute unit:
+// 20k rows x 117 entries takes 14.0 us with 313 wavefronts, 5.0 us with 5,000;
+// 148k x 38 is flat from 2,300 to 9,200, 8.7 us, and 10 us beyond), at least 6
+// entries a lane.
+//
+// No slices where more than twice the entries would be read: those are the
+// coarsest levels with a few rows many times the mean, which the block form
+// splits evenly.
+struct SlicePlan {
+    std::vector<dev::SliceHead> head;
+    std::vector<int> group;  // first slice of each group, then the slice count
+    int lt = 0;
+    size_t steps = 0;
+};
+
+SlicePlan plan_slices(const Csr& A, const std::vector<int>& groups, bool free_order,
+                      const std::vector<int>* blocks = nullptr) {
+    SlicePlan p;
+    const long nnz = A.nnz();
+    if (A.n == 0 || nnz == 0) return p;
+    const double mean = (double)nnz / A.n;
+    if (free_order) {
+        const double waves = (double)A.n / std::max((int)groups.size() - 1, 1) / 64;
+        auto more = [&]() { p.lt = p.lt == 0 ? 2 : p.lt + 1; };  // 1, 4, 8, 16 as in the block form
+        if (mean > 24)
+            while (p.lt < 4 && waves * (1 << p.lt) < 4096 && mean >= (p.lt == 0 ? 24 : 6 << (p.lt + 1))) more();
+        else if (waves < 1024 && mean >= 12)
+            more();
+    } else {
+        while ((1 << p.lt) < dev::lanes_per_row(mean)) p.lt++;
+    }
+    const std::vector<int> whole = {0, A.n};
+    const bool per_block = blocks && p.lt == 0;
+    const std::vector<int>& g = per_block ? *blocks : groups.empty() ? whole : groups;
+    const int ng = (int)g.size() - 1, T = 1 << p.lt, R = 64 / T;
+    size_t steps = 0;
+    for (int q = 0; q < ng; q++) {
+        p.group.push_back((int)p.head.size());
+        for (int r = g[q]; r < g[q + 1]; r += R) {
+            dev::SliceHead h;
+            h.row0 = r;
+            h.row1 = std::min(r + R, g[q + 1]);
+            h.step0 = (int)steps;
+            int w = 0;
+            for (int i = r; i < h.row1; i++) w = std::max(w, A.rp[i + 1] - A.rp[i]);
+            h.steps = (w + T - 1) / T;
+            steps += h.steps;
+            p.head.push_back(h);
+        }
+        while (per_block && p.head.size() % dev::SLICES_PER_BLOCK) {
+            dev::SliceHead h;
+            h.row0 = h.row1 = g[q + 1];
+            h.step0 = (int)steps;
+            p.head.push_back(h);
+        }
+    }
+    p.group.push_back((int)p.head.size());
+    p.steps = steps;
+    // entries read: lanes past a slice's rows load nothing
+    size_t read = 0;
+    for (const dev::SliceHead& h : p.head) read += (size_t)h.steps * T * (h.row1 - h.row0);
+    if (read > 2 * (size_t)nnz) {  // 64 steps < 2^32: step0 fits an int
+        p.head.clear();
+        p.group.clear();
+    }
+    return p;
+}
+
+// steps in flight per lane: all of a short row, else the count that wastes
+// least of its last round (7 for the 7 and 14 entries of the P1 stencils:
+// 2.1M rows x 14 in FP64, 69 us with 8, 65 us with 7)
+static int slice_unroll(double mean_steps) {
+    const int w = (int)std::ceil(mean_steps);
+    if (w <= 4) return 4;
+    return (w + 6) / 7 * 7 < (w + 7) / 8 * 8 ? 7 : 8;
+}
+
+// D.sl from the plan (D's CSR uploaded); share: the other precision's copy,
+// whose layout and codes are reused.  Large streams are loaded nontemporally:
+// FP64 from 64 MB (read once per Krylov iteration; 2.1M rows x 14, 79 -> 69
+// us, 1.05M x 7, 22.0 -> 20.4 us), FP32 from 128 MB (2.1M x 14, 40 -> 37 us;
+// smaller ones stay in the last-level cache between sweeps and lose: 403k x
+// 14, 8.6 -> 9.1 us).
+template <typename VT, typename OT>
+static void make_slices(const SlicePlan& p, dev::DMat<VT>& D, DevBuffers& B, hipStream_t st,
+                        const dev::DMat<OT>* share) {
+    dev::Slices<VT>& S = D.sl;
+    S = dev::Slices<VT>();
+    if (p.head.empty()) return;
+    S.ns = (int)p.head.size();
+    S.lt = p.lt;
+    S.steps = p.steps;
+    S.unroll = slice_unroll((double)S.steps / S.ns);
+    S.nt = S.steps * 64 * (sizeof(VT) + 2) >= (sizeof(VT) == 8 ? 64u << 20 : 128u << 20);
+    S.v = dalloc<VT>(S.steps * 64, B);
+    if (share) {
+        S.head = share->sl.head;
+        S.cs = share->sl.cs;
+    } else {
+        S.head = dupload(p.head, B, st);
+        S.cs = dalloc<uint16_t>(S.steps * 64, B);
+        dev::slice_columns<VT>(st, D);
+    }
+    dev::slice_values<VT>(st, D);
+    D.lpr = 1 << p.lt;
+    D.idx_bytes = 2.0 * D.nnz + 24.0 * S.ns;  // 32 bytes a head, 8 of them counted as its bounds
+}
+
+// slices of a matrix without groups and systems (krylov.cpp's operators)
+bool slice_matrix(const Csr& A, dev::DMat<double>& D, DevBuffers& B, hipStream_t st) {
+    const SlicePlan p = plan_slices(A, {}, false);  // the ILU's Krylov loops take no partials from it
+    make_slices<double, double>(p, D, B, st, nullptr);
+    return D.sl.ns > 0;
+}
+
+// plan: the slices (none: empty), starts_with_end: the row blocks (none:
+// empty); share: a copy of A with other values uploaded before; its row
+// pointers and column indices are reused, its slice layout when its plan
+// (share_plan) has the same rows, its 16-bit offsets when its block schedule
+// (share_starts) is the same
 template <typename VT, typename OT = double>
-static void upload_mat(const Csr& A, const std::vector<int>& starts_with_end, dev::DMat<VT>& D, DevBuffers& B,
-                       hipStream_t st, const dev::DMat<OT>* share = nullptr,
-                       const std::vector<int>* share_starts = nullptr, const int* row_ids = nullptr,
-                       const std::vector<int>* seg = nullptr) {
+static void upload_mat(const Csr& A, const SlicePlan& plan, const std::vector<int>& starts_with_end,
+                       dev::DMat<VT>& D, DevBuffers& B, hipStream_t st, const dev::DMat<OT>* share = nullptr,
+                       const SlicePlan* share_plan = nullptr, const std::vector<int>* share_starts = nullptr,
+                       const int* row_ids = nullptr, const std::vector<int>* seg = nullptr) {
     validate(A, starts_with_end, dev::block_nnz<VT>());
-    D.bspec = seg ? dupload(block_systems(starts_with_end, *seg, row_ids), B, st) : nullptr;
     D.active = nullptr;
     D.n = A.n;
     D.ncols = A.ncols;
@@ -199,27 +324,41 @@ static void upload_mat(const Csr& A, const std::vector<int>& starts_with_end, de
     D.ci = share ? share->ci : dupload(A.ci, B, st);
     std::vector<VT> v(A.v.begin(), A.v.end());
     D.v = dupload(v, B, st);
-    D.nblk = (int)starts_with_end.size() - 1;
-    if (D.nblk < 0) D.nblk = 0;
-    D.bk = dupload(block_pairs(A, starts_with_end), B, st);
-    if (share && share_starts && *share_starts == starts_with_end) {
-        D.cs = share->cs;
-        D.cb = share->cb;
-        D.idx_bytes = share->idx_bytes;
-    } else {
-        std::vector<uint16_t> cs;
-        std::vector<int2> cb;
-        const long coded = A.nnz() > 0 ? column_codes(A, starts_with_end, cs, cb) : 0;
-        D.cs = nullptr;
-        D.cb = nullptr;
-        D.idx_bytes = 4.0 * A.nnz();
-        if (coded > 0) {
-            D.cs = dupload(cs, B, st);
-            D.cb = dupload(cb, B, st);
-            D.idx_bytes = 2.0 * coded + 4.0 * (A.nnz() - coded) + 8.0 * D.nblk;
+    D.cs = nullptr;
+    D.cb = nullptr;
+    D.bspec = nullptr;
+    D.sl = dev::Slices<VT>();
+    D.nblk = std::max((int)starts_with_end.size() - 1, 0);
+    if (D.nblk > 0) {
+        D.bk = dupload(block_pairs(A, starts_with_end), B, st);
+        if (share && share_starts && *share_starts == starts_with_end) {
+            D.cs = share->cs;
+            D.cb = share->cb;
+            D.idx_bytes = share->idx_bytes;
+        } else {
+            std::vector<uint16_t> cs;
+            std::vector<int2> cb;
+            const long coded = A.nnz() > 0 ? column_codes(A, starts_with_end, cs, cb) : 0;
+            D.idx_bytes = 4.0 * A.nnz();
+            if (coded > 0) {
+                D.cs = dupload(cs, B, st);
+                D.cb = dupload(cb, B, st);
+                D.idx_bytes = 2.0 * coded + 4.0 * (A.nnz() - coded) + 8.0 * D.nblk;
+            }
         }
+        D.lpr = dev::lanes_per_row(A.n > 0 ? (double)A.nnz() / A.n : 0.0);
     }
-    D.lpr = dev::lanes_per_row(A.n > 0 ? (double)A.nnz() / A.n : 0.0);
+    if (!plan.head.empty()) {
+        const bool same = share && share_plan && share_plan->lt == plan.lt &&
+                          share_plan->head.size() == plan.head.size();
+        make_slices<VT, OT>(plan, D, B, st, same ? share : nullptr);
+    }
+    if (seg) {  // the systems of each slice, or of each block where there are no slices
+        std::vector<int> first;
+        for (const dev::SliceHead& k : plan.head) first.push_back(k.row0);
+        if (!first.empty()) first.push_back(A.n);
+        D.bspec = dupload(block_systems(first.empty() ? starts_with_end : first, *seg, row_ids), B, st);
+    }
     // diagonal positions (row r's own index: row_ids == nullptr) and l1 norms
     std::vector<int> dpos(A.n, -1);
     std::vector<VT> l1(A.n, (VT)0);
@@ -255,15 +394,33 @@ static std::vector<int> schedule(const Csr& A) {
     return starts;
 }
 
-// upload A as FP64 + FP32 copies sharing the index arrays (each with the row
-// blocks of its own value size); returns the larger block count
+// upload A as FP64 + FP32 copies sharing the index arrays; free32: the FP32
+// rows may be summed in any order (see Solver::fixed_order); partials: the
+// FP64 product's block partials are summed by a Krylov method (its row order is
+// kept then, and its partials' too without free32); returns the larger
+// workgroup count of a row kernel
 int upload_pair(const Csr& A0, dev::DMat<double>& D, dev::DMat<float>& F, DevBuffers& B, hipStream_t st,
-                const std::vector<int>* seg) {
+                const std::vector<int>* seg, bool free32, bool partials) {
     Csr A = drop_outside_zeros(A0);
-    const std::vector<int> s64 = schedule<double>(A), s32 = schedule<float>(A);
-    upload_mat<double, double>(A, s64, D, B, st, nullptr, nullptr, nullptr, seg);
-    upload_mat(A, s32, F, B, st, &D, &s64, nullptr, seg);
-    return std::max(D.nblk, F.nblk);
+    // the FP64 finest matrix (partials) keeps a row's column order
+    SlicePlan p64 = plan_slices(A, {}, !partials), p32 = plan_slices(A, {}, free32);
+    std::vector<int> s64, s32;
+    if (partials && !free32 && !seg && !p64.head.empty() && p64.lt == 0) {
+        // slices by row block where they fill their wavefronts (1.05M rows x
+        // 7: 256-row blocks), else the block form beside them (2.1M x 14, 146
+        // rows a block: 76 us, 87 us as slices of 64, 64 and 18 rows)
+        s64 = schedule<double>(A);
+        SlicePlan q = plan_slices(A, {}, false, &s64);
+        if (!q.head.empty() && A.n >= 0.9 * 64 * q.head.size()) {
+            p64 = std::move(q);
+            s64.clear();
+        }
+    }
+    if (p64.head.empty()) s64 = schedule<double>(A);
+    if (p32.head.empty()) s32 = schedule<float>(A);
+    upload_mat<double, double>(A, p64, s64, D, B, st, nullptr, nullptr, nullptr, nullptr, seg);
+    upload_mat(A, p32, s32, F, B, st, &D, &p64, &s64, nullptr, seg);
+    return std::max(dev::row_blocks(D), dev::row_blocks(F));
 }
 
 // level schedule of the lexicographic sweep: forward, level(i) = 1 + max over
@@ -336,7 +493,7 @@ constexpr int kLprCandidates[] = {1, 4, 8, 16, 32};
 
 template <typename VT, typename XT>
 int Solver::tune_spmv(dev::DMat<VT>& M, const XT* x, XT* y) {
-    if (M.nblk == 0) return M.lpr;
+    if (M.n == 0 || M.sl.ns) return M.lpr;  // slices: their lanes follow from the plan
     float best = 1e30f;
     int best_lpr = M.lpr;
     for (int lpr : kLprCandidates) {
@@ -359,7 +516,7 @@ int Solver::tune_spmv(dev::DMat<VT>& M, const XT* x, XT* y) {
 
 template <typename VT, typename XT>
 int Solver::tune_mcsor(DevLevel& d, dev::DMat<VT>& Ac, const XT* f, XT* x) {
-    if (Ac.nblk == 0 || d.ncolours == 0) return Ac.lpr;
+    if (Ac.n == 0 || d.ncolours == 0 || Ac.sl.ns) return Ac.lpr;
     float best = 1e30f;
     int best_lpr = Ac.lpr;
     const std::vector<int>& cb = sizeof(VT) == 8 ? d.colour_blk : d.colour_blk32;
@@ -455,7 +612,7 @@ void Solver::upload() {
         d.n = h.A.n;
         maxn = std::max(maxn, d.n);
         const std::vector<int>* segl = seg_off_.empty() ? nullptr : &seg_off_[l];
-        maxblk = std::max(maxblk, upload_pair(h.A, d.A, d.Af, B, st, segl));
+        maxblk = std::max(maxblk, upload_pair(h.A, d.A, d.Af, B, st, segl, !fixed_order(), l == depth - 1));
         d.x = dalloc<double>(d.n, B);
         d.f = dalloc<double>(d.n, B);
         d.r = dalloc<double>(d.n, B);
@@ -470,8 +627,9 @@ void Solver::upload() {
             up_[l].ci = h.A.ci;
         }
         if (l == 0) continue;
-        maxblk = std::max(maxblk, upload_pair(h.P, d.P, d.Pf, B, st, segl));
-        maxblk = std::max(maxblk, upload_pair(h.R, d.R, d.Rf, B, st, seg_off_.empty() ? nullptr : &seg_off_[l - 1]));
+        maxblk = std::max(maxblk, upload_pair(h.P, d.P, d.Pf, B, st, segl, !fixed_order(), false));
+        maxblk = std::max(maxblk, upload_pair(h.R, d.R, d.Rf, B, st, seg_off_.empty() ? nullptr : &seg_off_[l - 1],
+                                              !fixed_order(), false));
         // colour-permuted copy for the multicolour sweeps
         const std::vector<int>& col = colours_[l];
         int nc = ncolours_[l];
@@ -498,7 +656,7 @@ void Solver::upload() {
             }
             Ac.rp[r + 1] = (int)Ac.ci.size();
         }
-        // colour c's rows form the blocks [colour_blk[c], colour_blk[c+1])
+        // colour c's rows form the slices or blocks [colour_blk[c], colour_blk[c+1])
         auto colour_schedule = [&](int max_nnz, std::vector<int>& cb) {
             std::vector<int> starts;
             cb.assign(nc + 1, 0);
@@ -510,10 +668,14 @@ void Solver::upload() {
             starts.push_back(d.n);
             return starts;
         };
-        const std::vector<int> c64 = colour_schedule(dev::block_nnz<double>(), d.colour_blk);
-        const std::vector<int> c32 = colour_schedule(dev::block_nnz<float>(), d.colour_blk32);
-        upload_mat<double, double>(Ac, c64, d.Ac, B, st, nullptr, nullptr, perm.data(), segl);
-        upload_mat(Ac, c32, d.Acf, B, st, &d.Ac, &c64, perm.data(), segl);
+        const SlicePlan q64 = plan_slices(Ac, d.colour_rows, true), q32 = plan_slices(Ac, d.colour_rows, !fixed_order());
+        std::vector<int> c64, c32;
+        if (q64.head.empty()) c64 = colour_schedule(dev::block_nnz<double>(), d.colour_blk);
+        else d.colour_blk = q64.group;
+        if (q32.head.empty()) c32 = colour_schedule(dev::block_nnz<float>(), d.colour_blk32);
+        else d.colour_blk32 = q32.group;
+        upload_mat<double, double>(Ac, q64, c64, d.Ac, B, st, nullptr, nullptr, nullptr, perm.data(), segl);
+        upload_mat(Ac, q32, c32, d.Acf, B, st, &d.Ac, &q64, &c64, perm.data(), segl);
         d.perm = dupload(perm, B, st);
         d.ncolours = nc;
         if (track_) {
@@ -926,6 +1088,7 @@ bool Solver::refresh_values() {
         DevLevel& d = L_[l];
         put(d.A.v, A.v);
         dev::convert<double, float>(st, d.A.nnz, d.A.v, d.Af.v);
+        slice_pair(st, d.A, d.Af);
         put(d.A.l1, row_l1<double>(A));
         putf(d.Af.l1, row_l1<float>(A));
         if (l == 0) continue;
@@ -944,6 +1107,7 @@ bool Solver::refresh_values() {
         const int nnz = (int)Ac.v.size();
         put(d.Ac.v, std::move(Ac.v));
         dev::convert<double, float>(st, nnz, d.Ac.v, d.Acf.v);
+        slice_pair(st, d.Ac, d.Acf);
         if (d.sor_packed) {
             hip_check(hipStreamSynchronize(st), "sync");
             build_sor_packs(l, *bufs_, true);  // the packs hold values: rewritten in place
@@ -1572,6 +1736,7 @@ int Solver::pcg_dev(double* X, double* B, double tol, int max_iter, int stop, li
     // from the second iteration on, pcg_xr writes the preconditioner's entry
     // on the new R (its FP32 copy, initial guess and r0 test)
     const bool prep = entry_prepared_ok();
+    const bool fixed = prm_.precision == LINA_PREC_MIXED && fixed_order();
     auto enqueue = [&](int k) {
         int m = 0;
         precon(R, Z, R, &m, prep && k > 0);
@@ -1584,9 +1749,10 @@ int Solver::pcg_dev(double* X, double* B, double tol, int max_iter, int stop, li
             m = dev::dot_part<double>(st, n, P, Q, part_);
         } else {
             if (sampled(k))  // the events bracket the kernel itself
-                m = dev::spmv_outer_timed(st, top.A, P, Q, part_, P, evk_[k % 2][0], evk_[k % 2][1]);
+                m = dev::spmv_outer_timed(st, top.A, P, Q, part_, P, evk_[k % 2][0], evk_[k % 2][1], fixed);
             else
-                m = dev::spmv<double, double>(st, top.A, P, nullptr, Q, dev::MODE_OUTER, part_, P);  // Q = A P, P.Q
+                m = dev::spmv<double, double>(st, top.A, P, nullptr, Q, dev::MODE_OUTER, part_, P, nullptr,
+                                              fixed);  // Q = A P, P.Q
         }
         dev::finalize(st, m, part_, scal_, dev::S_PQ, 0);
         if (!prep) {
@@ -1721,11 +1887,11 @@ double spmv_bytes(double n, double nnz, int precision) {
 }
 
 // algorithmic bytes of one y = A x with the uploaded arrays: values, column
-// indices (2-byte codes + 8 bytes of bases per block, or 4 bytes), row
-// pointers, block pairs, x gathered once, y written once
+// indices (2-byte codes + 8 bytes of bases per slice or block, or 4 bytes),
+// row pointers, slice or block pairs, x gathered once, y written once
 template <typename VT>
 static double mat_bytes(const dev::DMat<VT>& A) {
-    return (double)sizeof(VT) * A.nnz + A.idx_bytes + 4.0 * (A.n + 1) + 8.0 * (A.nblk + 1) +
+    return (double)sizeof(VT) * A.nnz + A.idx_bytes + 4.0 * (A.n + 1) + 8.0 * ((A.sl.ns ? A.sl.ns : A.nblk) + 1) +
            (double)sizeof(VT) * (A.ncols + A.n);
 }
 
@@ -1742,7 +1908,7 @@ DevMatrix::DevMatrix(const Csr& A) : n_(A.n), nnz_(A.nnz()), bufs_(new DevBuffer
     hip_check(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking), "stream");
     hip_check(hipEventCreate(&ev0_), "event");
     hip_check(hipEventCreate(&ev1_), "event");
-    upload_pair(A, A_, Af_, *bufs_, stream_);
+    upload_pair(A, A_, Af_, *bufs_, stream_, nullptr, true, true);
     prp_ = A.rp;
     pci_ = A.ci;
     x_ = dalloc<double>(n_, *bufs_);
@@ -1758,6 +1924,7 @@ bool DevMatrix::update_values(const Csr& A0) {
     if (A.nnz() != A_.nnz) return false;
     hip_check(hipMemcpyAsync(A_.v, A.v.data(), A.v.size() * sizeof(double), hipMemcpyHostToDevice, stream_), "h2d");
     dev::convert<double, float>(stream_, A_.nnz, A_.v, Af_.v);
+    slice_pair(stream_, A_, Af_);
     hip_check(hipStreamSynchronize(stream_), "update");
     return true;
 }
@@ -1766,6 +1933,7 @@ bool DevMatrix::update_values_device(const double* d_val, long nnz) {
     if (nnz != (long)A_.nnz || nnz_ != nnz) return false;
     hip_check(hipMemcpyAsync(A_.v, d_val, nnz * sizeof(double), hipMemcpyDeviceToDevice, stream_), "d2d");
     dev::convert<double, float>(stream_, A_.nnz, A_.v, Af_.v);
+    slice_pair(stream_, A_, Af_);
     hip_check(hipStreamSynchronize(stream_), "update");
     return true;
 }

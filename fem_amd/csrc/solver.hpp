@@ -84,8 +84,8 @@ struct DevLevel {
     int ncolours = 0;
     int* perm = nullptr;
     std::vector<int> colour_rows;  // ncolours+1 row offsets into Ac
-    std::vector<int> colour_blk;   // ncolours+1 block offsets into Ac's blocks
-    std::vector<int> colour_blk32; // the same for Acf (FP32 blocks hold more entries)
+    std::vector<int> colour_blk;   // ncolours+1 offsets into Ac's slices or blocks
+    std::vector<int> colour_blk32; // the same for Acf
     // exact lexicographic sweeps
     int nlv_f = 0, nlv_b = 0;
     int *lvf_off = nullptr, *lvf_rows = nullptr, *lvb_off = nullptr, *lvb_rows = nullptr;
@@ -100,7 +100,14 @@ struct DevLevel {
 };
 
 int upload_pair(const Csr& A0, dev::DMat<double>& D, dev::DMat<float>& F, DevBuffers& B, hipStream_t st,
-                const std::vector<int>* seg = nullptr);
+                const std::vector<int>* seg, bool free32, bool partials);
+// a sliced copy of D (CSR of A uploaded) where worthwhile; false: none
+bool slice_matrix(const Csr& A, dev::DMat<double>& D, DevBuffers& B, hipStream_t st);
+// both precisions' sliced values from their CSR values
+inline void slice_pair(hipStream_t st, const dev::DMat<double>& D, const dev::DMat<float>& F) {
+    dev::slice_values<double>(st, D);
+    dev::slice_values<float>(st, F);
+}
 void build_blocks(const Csr& A, int begin, int end, int max_nnz, std::vector<int>& starts,
                   int max_rows = dev::BLOCK_ROWS);
 std::vector<int2> block_pairs(const Csr& A, const std::vector<int>& starts_with_end);
@@ -130,7 +137,7 @@ class DevMatrix {
     int launch(const double* x, const double* b, double* y, int mode, double* part, const double* w);
     int launch_on(hipStream_t st, const double* x, const double* b, double* y, int mode, double* part,
                   const double* w);
-    int nblocks() const { return A_.nblk; }
+    int nblocks() const { return dev::row_blocks(A_); }
     void spmv_dev(const double* x, double* y);
     void spmv_host(int precision, const double* x, double* y);
     double time_spmv(int precision, int reps);
@@ -189,6 +196,13 @@ class Solver {
     const HostHierarchy& host() const { return H_; }
     // the host hierarchy with the values of a device recompute copied back
     const HostHierarchy& host_synced();
+    // The aggressive first coarsening is a weak preconditioner: under an FP32
+    // hierarchy CG takes hundreds of iterations, and the iterate it stops at
+    // moves with the rounding of every sum (129^2 plane strain to 1e-12: 324 to
+    // 403 iterations and 1e-10 to 1e-8 of the solution over orders of one dot
+    // product).  Those hierarchies keep one order of every FP32 row sum and of
+    // the outer product's partials, whatever form the matrices have.
+    bool fixed_order() const { return prm_.coarsening == LINA_COARSEN_AGGRESSIVE; }
     const std::vector<int>& colours(int l) const { return colours_.at(l); }
     bool uploaded() const { return bufs_ != nullptr; }
     int n() const { return n_; }

@@ -252,8 +252,9 @@ int lina_spmv(lina_solver* s, int level, int precision, const double* x, double*
 double lina_time_spmv(lina_solver* s, int level, int precision, int reps);
 /* per-launch algorithmic byte count used for roofline reporting, from the
  * uploaded arrays: (value size + index size) nnz + 4 (n+1) row pointers +
- * 8 (blocks+1) block bounds (+ 4 per block of base columns) + x and y once;
- * the index size is 2 where every row block's columns span < 65536, else 4 */
+ * x and y once, and 32 per slice of a sliced copy (index size 2) or 8
+ * (blocks+1) block bounds + 8 per block of base columns (index size 2 where
+ * every row block's columns span < 65536, else 4) */
 double lina_spmv_bytes(const lina_solver* s, int level, int precision);
 /* on != 0: pcg brackets the outer-loop A*p launch of every fourth iteration
  * with HIP events and reports the mean launch duration in lina_stats.spmv_ms */

@@ -1,0 +1,77 @@
+"""Row sums of the sliced matrix copies (dev::Slices): y = A x against numpy
+over row counts around a slice's 64 rows, row lengths around the limits of one
+and several lanes a row, rows of unequal length, and columns that need a third
+base (read from the CSR's indices).
+
+Short rows (means up to 24 entries) keep the column order of the reference's
+loops: FP64 products equal the sequential sum bit for bit.  Otherwise the sum's
+order is free and |y - A x| <= (m + 1) eps sum |a_ij x_j| with m entries a row
+(any order of m - 1 additions of rounded products)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def rows_of(n, mean, spread, seed):
+    """CSR with about `mean` sorted columns a row (spread: up to twice that in some rows)"""
+    rng = np.random.default_rng(seed)
+    lens = np.full(n, min(mean, n))
+    if spread:
+        lens = np.clip(rng.integers(max(1, mean // 2), 2 * mean, n), 1, n)
+    cols = []
+    for i in range(n):
+        m = int(lens[i])
+        if 4 * m >= n:
+            cols.append(np.sort(rng.permutation(n)[:m]))
+        else:
+            cols.append(np.unique(np.concatenate([[i], rng.integers(0, n, m - 1)])))
+    rp = np.concatenate([[0], np.cumsum([len(c) for c in cols])]).astype(np.int32)
+    return rp, np.concatenate(cols).astype(np.int32)
+
+
+@pytest.mark.parametrize("n", [1, 3, 63, 64, 65, 255, 257, 1000, 70001])
+@pytest.mark.parametrize("mean,spread", [(1, False), (7, False), (14, True), (24, False), (25, False), (60, True),
+                                         (130, False), (300, True)])
+def test_products_with_sliced_rows(gpu, n, mean, spread):
+    if n > 1000 and mean > 60:
+        pytest.skip("the long rows are covered by the smaller matrices")
+    print("slices", n, mean, spread, flush=True)
+    rp, ci = rows_of(n, mean, spread, 1000 * mean + n)
+    rng = np.random.default_rng(7)
+    v, x = rng.standard_normal(len(ci)), rng.standard_normal(n)
+    A = gpu.Matrix(rp, ci, v)
+    y, y32 = A.spmv(x), A.spmv(x, precision="mixed")
+    A.close()
+    prod = v * x[ci]
+    m = np.diff(rp)
+    ref = np.array([np.sum(prod[rp[i]:rp[i + 1]].astype(np.longdouble)) for i in range(n)]).astype(np.float64)
+    bound = np.array([np.sum(np.abs(prod[rp[i]:rp[i + 1]])) for i in range(n)])
+    assert np.all(np.abs(y - ref) <= (m + 1) * 2.0 ** -53 * bound)
+    # FP32: values, x and products rounded once each besides the additions
+    assert np.all(np.abs(y32 - ref) <= (m + 4) * 2.0 ** -24 * bound)
+    if len(ci) / n <= 24:
+        seq = np.zeros(n)
+        for j in range(int(m.max())):
+            has = m > j
+            seq[has] += prod[rp[:-1][has] + j]
+        assert np.array_equal(y, seq)
+
+
+def test_values_follow_an_update(gpu):
+    """a hierarchy's sliced copies follow new values (recompute), FP64 and mixed"""
+    from fem_amd import problems as P
+    s1, s2 = P.damage_system(65), P.damage_system(65, seed_h=99)
+    for prec in ("fp64", "mixed"):
+        prm = gpu.params("vcycle", 1, 4, precision=prec)
+        a, b = gpu.AMG(s1[0].rowptr, s1[0].col, s1[0].val, prm), gpu.AMG(s1[0].rowptr, s1[0].col, s1[0].val, prm)
+        d = gpu.DeviceVector(len(s2[0].val))
+        d.upload(s2[0].val)
+        a.recompute(s2[0].val)
+        b.recompute_device(d.ptr)
+        ra, rb = (h.pcg(s2[0].b, tol=1e-11, max_iter=500, stop="relres") for h in (a, b))
+        r = s2[0].b - s2[0].scipy() @ ra["x"]
+        assert np.linalg.norm(r) <= 1e-10 * np.linalg.norm(s2[0].b)
+        assert ra["iters"] == rb["iters"] and np.array_equal(ra["x"], rb["x"])
+        a.close()
+        b.close()
