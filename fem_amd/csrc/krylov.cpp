@@ -728,7 +728,7 @@ int IluSystem::gmres_core(double* Y, const double* Bv, int m, double tol, int ma
         double* v0 = V;
         apply_p(Y, v0);
         matvec(v0, vW_);
-        dev::axpby(st, n, 0.0, vR_, 1.0, Bv);
+        dev::copy(st, n, Bv, vR_);  // not 0 * vR_ + Bv: vR_ may hold anything, NaN included
         dev::axpby(st, n, 1.0, vR_, -1.0, vW_);
         double beta = std::sqrt(dot(vR_, vR_));
         if (iter == 0) {
@@ -738,7 +738,8 @@ int IluSystem::gmres_core(double* Y, const double* Bv, int m, double tol, int ma
             eta = beta / beta0;
         }
         if (eta > tol) {
-            dev::axpby(st, n, 0.0, v0, 1.0 / beta, vR_);
+            dev::copy(st, n, (const double*)vR_, v0);
+            dev::scale(st, n, v0, 1.0 / beta);
             for (int i = 1; i <= m; i++) {
                 double* vi = V + (size_t)(i - 1) * ld;
                 double* vn = V + (size_t)i * ld;
