@@ -70,7 +70,24 @@ class IluSystem {
         double* ovval = nullptr;
     };
 
+    // a factor's levels padded for dev::tri_level, and their value maps
+    struct TriWide {
+        std::vector<dev::TriLevel> lv;
+        int nval = 0;
+        int *vmap = nullptr, *dmap = nullptr;
+        double *val = nullptr, *diag = nullptr;
+    };
+
   private:
+    void build_wide(const Csr& T, bool upper, const std::vector<int>& off, const std::vector<int>& rows, TriWide& W);
+    // w = U^-1 L^-1 z by levels; part: block partials of z.w, returns their number
+    int apply_wide(const double* z, double* w, double* part);
+    TriWide wl_, wu_;
+    int* udmap_ = nullptr;   // rows whose U row is the diagonal alone: its entry (-1: other rows)
+    double* ud_ = nullptr;   // and its value (0: other rows)
+    // Z = M^-1 R and the block partials of R.Z in rz, returns their number
+    int precon_dot(const double* R, double* Z, double* rz);
+    double dot_at(const double* a, const double* b, double* part);  // partials in part
     void build_p(const Csr& A, bool upload);
     void refactor_p(const Csr& A);
     void apply_p(const double* z, double* w);  // in the factors' (permuted) order
@@ -85,7 +102,6 @@ class IluSystem {
     void numeric();
     double *vXo_ = nullptr, *vBo_ = nullptr, *vPz_ = nullptr, *vPw_ = nullptr;
     bool wide_ = false;             // few, wide levels: a launch per level on the whole GPU
-    std::vector<int> hoff_u_;
     void sync_factors();
     void pack_values();
     bool build_plan();

@@ -1437,27 +1437,129 @@ __global__ __launch_bounds__(TPB) void k_ilu0_planned_level(int t0, int t1, cons
         ilu0_planned_row(t, m1, m2, mask, pu, vA, vL, vU, fail);
 }
 
-// One level [t0, t1) of a triangular sweep on a full grid, a row per
-// thread, each row's arithmetic that of PCG_preconl / PCG_preconr: forward
-// (L, diagonal last) s = z_i, s -= l_ij y_j in column order, y_i = s / l_ii;
-// backward (U, diagonal first) s = y_i, s -= u_ij w_j, w_i = s / u_ii.
-__global__ __launch_bounds__(TPB) void k_tri_level(int t0, int t1, const int* __restrict__ rows,
-                                                   const int* __restrict__ rp, const int* __restrict__ ci,
-                                                   const double* __restrict__ v, const double* __restrict__ in,
-                                                   double* out, int upper) {
-    for (int t = t0 + blockIdx.x * TPB + threadIdx.x; t < t1; t += gridDim.x * TPB) {
-        const int i = rows[t];
-        const int b = rp[i], e = rp[i + 1];
-        double s = in[i];
-        if (!upper) {
-            for (int p = b; p < e - 1; p++) s -= v[p] * out[ci[p]];
-            s /= v[e - 1];
-        } else {
-            for (int p = b + 1; p < e; p++) s -= v[p] * out[ci[p]];
-            s /= v[b];
-        }
-        out[i] = s;
+// One wide level of a triangular sweep, a row per lane.  Latency bounds it (a
+// level of 15k-260k rows is 1-20 MB): a row's entries come from padded
+// slot-major arrays in level order, so a lane waits for two memory round trips
+// (entries, results) instead of the four of the factor's CSR (row, bounds,
+// entries, results) -- 301 x 203 Poisson, a level of 15k rows: 3.5 -> 2.5 us.
+template <int K>
+__device__ __forceinline__ double tri_row(const TriLevel& L, int t, double s, const double* out) {
+    int c[K];
+    double v[K], x[K];
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        const int q = min(k, L.K - 1) * L.cnt + t;
+        c[k] = L.col[q];
+        v[k] = L.val[q];
     }
+#pragma unroll
+    for (int k = 0; k < K; k++) x[k] = out[max(c[k], 0)];
+#pragma unroll
+    for (int k = 0; k < K; k++)
+        if (k < L.K && c[k] >= 0) s -= v[k] * x[k];
+    return s;
+}
+
+__global__ __launch_bounds__(TPB) void k_tri_level(const TriLevel L, const double* in, double* out,
+                                                   const double* __restrict__ ud, double* w,
+                                                   const double* __restrict__ r, double* __restrict__ part) {
+    double mine = 0.0;
+    const int t = blockIdx.x * TPB + threadIdx.x;
+    if (t < L.cnt) {
+        const int i = L.rows ? L.rows[t] : L.row0 + t;
+        const double d = L.diag[t], u = ud ? ud[i] : 0.0, ri = r ? r[i] : 0.0;
+        double s = in[i];
+        if (L.K > 0 && L.K <= 4) {
+            s = tri_row<4>(L, t, s, out);
+        } else if (L.K > 0 && L.K <= 8) {
+            s = tri_row<8>(L, t, s, out);
+        } else {
+            for (int k = 0; k < L.K; k++) {
+                const int c = L.col[(size_t)k * L.cnt + t];
+                if (c >= 0) s -= L.val[(size_t)k * L.cnt + t] * out[c];
+            }
+        }
+        s /= d;
+        out[i] = s;
+        if (!w) {
+            mine = ri * s;
+        } else if (u != 0.0) {
+            const double z = s / u;
+            w[i] = z;
+            mine = ri * z;
+        }
+    }
+    if (part) {
+        const double b = block_sum(mine);
+        if (threadIdx.x == 0) part[blockIdx.x] = b;
+    }
+}
+
+__global__ void k_tri_gather(int n, const int* __restrict__ map, const double* __restrict__ v,
+                             double* __restrict__ val) {
+    for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < n; q += gridDim.x * blockDim.x)
+        val[q] = map[q] >= 0 ? v[map[q]] : 0.0;
+}
+
+// the sum of np partials (np > 0) in one fixed order, in every thread; else have
+__device__ __forceinline__ double parts_sum(const double* __restrict__ part, int np, double have) {
+    if (np <= 0) return have;
+    __shared__ double total;
+    double s = 0.0;
+    for (int i = threadIdx.x; i < np; i += TPB) s += part[i];
+    s = block_sum(s);
+    if (threadIdx.x == 0) total = s;
+    __syncthreads();
+    s = total;
+    __syncthreads();
+    return s;
+}
+
+__global__ __launch_bounds__(TPB) void k_ipcg_p(int n, int k, double* __restrict__ P, const double* __restrict__ Z,
+                                                double* __restrict__ scal, const double* __restrict__ rz, int nrz,
+                                                const double* __restrict__ rr, int nrr, double r0, double tol,
+                                                int relres, int max_iter, double* status) {
+    const double s = parts_sum(rz, nrz, scal[IS_S0 + k % 2]);
+    const double b = k > 0 ? s / scal[IS_S0 + (k + 1) % 2] : 0.0;
+    if (blockIdx.x == 0) {
+        const double r2 = k > 0 ? parts_sum(rr, nrr, scal[IS_RR]) : 0.0;
+        if (threadIdx.x == 0) {
+            scal[IS_S0 + k % 2] = s;
+            if (k > 0) {
+                // the loop condition of PCGS.c:224
+                const double r = sqrt(r2), crit = relres ? r : r / r0;
+                const bool was = scal[IS_STOP] != 0.0;
+                const bool stop = was || !(crit > tol) || k >= max_iter;
+                if (!was) scal[IS_IT] = (double)k;
+                if (stop) scal[IS_STOP] = 1.0;
+                double* h = status + 4 * (k % 4);
+                h[1] = r;
+                h[2] = stop ? 1.0 : 0.0;
+                h[3] = scal[IS_IT];
+                __threadfence_system();
+                __hip_atomic_store(h, (double)k, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+            }
+        }
+    }
+    for (int i = blockIdx.x * TPB + threadIdx.x; i < n; i += gridDim.x * TPB)
+        P[i] = k > 0 ? b * P[i] + Z[i] : Z[i];
+}
+
+__global__ __launch_bounds__(TPB) void k_ipcg_xr(int n, int k, double* __restrict__ X, double* __restrict__ R,
+                                                 const double* __restrict__ P, const double* __restrict__ Q,
+                                                 const double* __restrict__ scal, const double* __restrict__ pq,
+                                                 int npq, double* __restrict__ rr) {
+    if (scal[IS_STOP] != 0.0) return;
+    const double a = scal[IS_S0 + k % 2] / parts_sum(pq, npq, scal[IS_PQ]);
+    double s = 0.0;
+    for (int i = blockIdx.x * TPB + threadIdx.x; i < n; i += gridDim.x * TPB) {
+        X[i] += a * P[i];
+        const double r = R[i] + (-a) * Q[i];
+        R[i] = r;
+        s += r * r;
+    }
+    s = block_sum(s);
+    if (threadIdx.x == 0) rr[blockIdx.x] = s;
 }
 
 // out[r] = in[perm[r]] (inverse == 0) or out[perm[r]] = in[r] (inverse == 1)
@@ -1485,12 +1587,11 @@ __global__ __launch_bounds__(TPB) void k_multidot(int n, int m, const double* __
 // out[l] = sum of the nblk partials of dot l (fixed order)
 __global__ __launch_bounds__(TPB) void k_multidot_final(int m, int nblk, const double* __restrict__ part,
                                                         double* __restrict__ out) {
-    for (int l = 0; l < m; l++) {
-        double s = 0.0;
-        for (int i = threadIdx.x; i < nblk; i += TPB) s += part[(size_t)l * nblk + i];
-        double t = block_sum(s);
-        if (threadIdx.x == 0) out[l] = t;
-    }
+    const int l = blockIdx.x;  // one workgroup a dot
+    double s = 0.0;
+    for (int i = threadIdx.x; i < nblk; i += TPB) s += part[(size_t)l * nblk + i];
+    double t = block_sum(s);
+    if (threadIdx.x == 0) out[l] = t;
 }
 
 // y[j] = base[j] + sign * sum_{l<m} V_l[j] * c[l]   (c on the device)
@@ -2849,14 +2950,29 @@ void ilu0_planned_levels(hipStream_t st, const std::vector<int>& off, const int4
     }
 }
 
-void tri_levels_wide(hipStream_t st, const int* rp, const int* ci, const double* v, const std::vector<int>& off,
-                     const int* rows, const double* in, double* out, int upper) {
-    for (size_t L = 0; L + 1 < off.size(); L++) {
-        const int cnt = off[L + 1] - off[L];
-        if (cnt <= 0) continue;
-        hipLaunchKernelGGL(k_tri_level, dim3(grid_for(cnt)), dim3(TPB), 0, st, off[L], off[L + 1], rows, rp, ci, v,
-                           in, out, upper);
-    }
+int tri_level_blocks(const TriLevel& L) { return (L.cnt + TPB - 1) / TPB; }
+
+void tri_level(hipStream_t st, const TriLevel& L, const double* in, double* out, const double* ud, double* w,
+               const double* r, double* part) {
+    if (L.cnt > 0)
+        hipLaunchKernelGGL(k_tri_level, dim3(tri_level_blocks(L)), dim3(TPB), 0, st, L, in, out, ud, w, r, part);
+}
+
+void tri_values(hipStream_t st, int n, const int* map, const double* v, double* val) {
+    if (n > 0) hipLaunchKernelGGL(k_tri_gather, dim3(grid_for(n)), dim3(TPB), 0, st, n, map, v, val);
+}
+
+void ipcg_p(hipStream_t st, int n, int k, double* P, const double* Z, double* scal, const double* rz, int nrz,
+            const double* rr, int nrr, double r0, double tol, int relres, int max_iter, double* status) {
+    hipLaunchKernelGGL(k_ipcg_p, dim3(grid_for(n, 1024)), dim3(TPB), 0, st, n, k, P, Z, scal, rz, nrz, rr, nrr, r0,
+                       tol, relres, max_iter, status);
+}
+
+int ipcg_xr(hipStream_t st, int n, int k, double* X, double* R, const double* P, const double* Q, const double* scal,
+            const double* pq, int npq, double* rr) {
+    const int g = grid_for(n, 1024);
+    hipLaunchKernelGGL(k_ipcg_xr, dim3(g), dim3(TPB), 0, st, n, k, X, R, P, Q, scal, pq, npq, rr);
+    return g;
 }
 
 void permute_idx(hipStream_t st, int n, const int* idx, const double* in, double* out) {
@@ -2879,7 +2995,7 @@ void ilu0_numeric(hipStream_t st, int nlv, const int* lv_off, const int* lv_rows
 int multidot(hipStream_t st, int n, int m, const double* V, size_t ld, const double* r, double* part, double* out) {
     int g = grid_for(n, 512);
     hipLaunchKernelGGL(k_multidot, dim3(g), dim3(TPB), 0, st, n, m, V, ld, r, part);
-    hipLaunchKernelGGL(k_multidot_final, dim3(1), dim3(TPB), 0, st, m, g, part, out);
+    hipLaunchKernelGGL(k_multidot_final, dim3(m), dim3(TPB), 0, st, m, g, part, out);
     return g;
 }
 

@@ -361,11 +361,43 @@ constexpr int ILU_MAXA = 16, ILU_MAXL = 8;
 // schedules of few, wide levels; off: the host copy of the level offsets)
 void ilu0_planned_levels(hipStream_t st, const std::vector<int>& off, const int4* m1, const int4* m2,
                          const int* mask, const int* pu, const double* vA, double* vL, double* vU, int* fail);
-// a triangular sweep one level per launch (rows: the level-ordered rows of
-// the factor, off: host level offsets); the arithmetic of PCG_preconl
-// (upper = 0, diagonal last) or PCG_preconr (upper = 1, diagonal first)
-void tri_levels_wide(hipStream_t st, const int* rp, const int* ci, const double* v, const std::vector<int>& off,
-                     const int* rows, const double* in, double* out, int upper);
+// One level of a triangular factor for a launch of its own (the multicolour
+// order's few wide levels): row t < cnt is factor row rows[t] (row0 + t when
+// rows is nullptr), its K padded entries val/col[k cnt + t] in row order
+// (col < 0: none), its diagonal diag[t].
+struct TriLevel {
+    int cnt = 0, K = 0, row0 = 0;
+    const int* rows = nullptr;
+    const int* col = nullptr;
+    const double* val = nullptr;
+    const double* diag = nullptr;
+};
+// workgroups of a level's launch (its partials' number)
+int tri_level_blocks(const TriLevel& L);
+// out_i = (in_i - sum val out_col) / diag, PCG_preconl's and PCG_preconr's
+// arithmetic.  ud, w (a forward level): rows whose backward row is its diagonal
+// ud[i] alone (0: they are not) also get w_i = out_i / ud[i].  r, part: block
+// partials of r_i times the rows' final results (w_i, or out_i without w).
+void tri_level(hipStream_t st, const TriLevel& L, const double* in, double* out, const double* ud, double* w,
+               const double* r, double* part);
+// val[q] = v[map[q]] (map < 0: 0) for the padded entries and diagonals of a factor
+void tri_values(hipStream_t st, int n, const int* map, const double* v, double* val);
+
+// ILU-pcg on the device (IluSystem::pcg_core).  The sum of np partials is
+// taken by every workgroup that needs it (np <= IPCG_PARTS) instead of a
+// launch of its own; np = 0: already in scal (k_finalize).
+constexpr int IPCG_PARTS = 2048;
+enum { IS_S0 = 0, IS_S1 = 1, IS_PQ = 2, IS_RR = 3, IS_STOP = 4, IS_IT = 5, IS_COUNT = 8 };
+// iteration k's direction P = Z (k = 0) or b P + Z, b = S_k / S_{k-1}, with
+// S_k = R.Z from its partials; before it, for k > 0, the loop test of
+// iteration k - 1 on |R|^2 from its partials: scal[IS_STOP] and, for the host,
+// status[4 (k % 4) ...] = {k, |R|, stop}
+void ipcg_p(hipStream_t st, int n, int k, double* P, const double* Z, double* scal, const double* rz, int nrz,
+            const double* rr, int nrr, double r0, double tol, int relres, int max_iter, double* status);
+// X += a P, R -= a Q, a = S_k / P.Q, and the partials of |R|^2; nothing once
+// scal[IS_STOP] is set.  Returns the partials' number.
+int ipcg_xr(hipStream_t st, int n, int k, double* X, double* R, const double* P, const double* Q, const double* scal,
+            const double* pq, int npq, double* rr);
 // out[r] = in[perm[r]] (inverse 0), out[perm[r]] = in[r] (inverse 1)
 void permute(hipStream_t st, int n, const int* perm, const double* in, double* out, int inverse);
 // out[k] = in[idx[k]], k < n (a gather of n entries)

@@ -511,7 +511,6 @@ void IluSystem::upload(bool pattern_levels_in) {
     nlv_u_ = (int)offu.size() - 1;
     lvu_off_ = kupload(offu, B, st);
     lvu_rows_ = kupload(rowsu, B, st);
-    hoff_u_ = offu;
     const int n = n_;
     for (double** p : {&vX_, &vB_, &vR_, &vP_, &vQ_, &vZ_, &vW_, &vY_, &vT_}) *p = kalloc<double>(n, B);
     dperm_ = nullptr;
@@ -553,6 +552,18 @@ void IluSystem::upload(bool pattern_levels_in) {
         vYu_ = kalloc<double>(n, B);
         pack_values();
     }
+    wl_ = TriWide();
+    wu_ = TriWide();
+    if (wide_) {
+        build_wide(L_, false, off, rows, wl_);
+        build_wide(U_, true, offu, rowsu, wu_);
+        std::vector<int> um(n);
+        for (int i = 0; i < n; i++) um[i] = U_.rp[i + 1] - U_.rp[i] == 1 ? U_.rp[i] : -1;
+        udmap_ = kupload(um, B, st);
+        ud_ = kalloc<double>(n, B);
+        pack_values();
+        hip_check(hipStreamSynchronize(st), "sync");  // the host maps die here
+    }
     part_ = kalloc<double>(std::max(4096, dev::row_blocks(dA_) + 16) * 40, B);
     scal_ = kalloc<double>(64, B);
     fail_ = kalloc<int>(1, B);
@@ -561,9 +572,82 @@ void IluSystem::upload(bool pattern_levels_in) {
 }
 
 void IluSystem::pack_values() {
+    if (wide_) {
+        dev::tri_values(stream_, wl_.nval, wl_.vmap, dL_.v, wl_.val);
+        dev::tri_values(stream_, n_, wl_.dmap, dL_.v, wl_.diag);
+        dev::tri_values(stream_, wu_.nval, wu_.vmap, dU_.v, wu_.val);
+        dev::tri_values(stream_, n_, wu_.dmap, dU_.v, wu_.diag);
+        dev::tri_values(stream_, n_, udmap_, dU_.v, ud_);
+    }
     if (!packed_) return;
     dev::tri_pack_values(stream_, n_, tf_.p.maxp, tf_.vmap, tf_.dmap, tf_.nov, tf_.ovmap, dL_.v, tf_.rec, tf_.ovval);
     dev::tri_pack_values(stream_, n_, tb_.p.maxp, tb_.vmap, tb_.dmap, tb_.nov, tb_.ovmap, dU_.v, tb_.rec, tb_.ovval);
+}
+
+// a factor's levels (pattern levels: every off-diagonal entry counts) padded
+// to each level's longest row, slot-major
+void IluSystem::build_wide(const Csr& T, bool upper, const std::vector<int>& off, const std::vector<int>& rows,
+                           TriWide& W) {
+    const int nlv = (int)off.size() - 1;
+    std::vector<int> vmap, col, dmap(T.n);
+    std::vector<size_t> base(nlv);
+    W.lv.assign(nlv, dev::TriLevel());
+    for (int L = 0; L < nlv; L++) {
+        dev::TriLevel& v = W.lv[L];
+        v.cnt = off[L + 1] - off[L];
+        v.row0 = v.cnt > 0 ? rows[off[L]] : 0;
+        bool run = true;
+        for (int t = 0; t < v.cnt; t++) {
+            const int i = rows[off[L] + t];
+            run = run && i == v.row0 + t;
+            v.K = std::max(v.K, T.rp[i + 1] - T.rp[i] - 1);
+        }
+        v.rows = run ? nullptr : (upper ? lvu_rows_ : lvl_rows_) + off[L];
+        base[L] = vmap.size();
+        vmap.resize(base[L] + (size_t)v.K * v.cnt, -1);
+        col.resize(vmap.size(), -1);
+        for (int t = 0; t < v.cnt; t++) {
+            const int i = rows[off[L] + t];
+            const int d = upper ? T.rp[i] : T.rp[i + 1] - 1;
+            dmap[off[L] + t] = d;
+            size_t q = base[L] + t;
+            for (int p = T.rp[i]; p < T.rp[i + 1]; p++) {
+                if (p == d) continue;
+                vmap[q] = p;
+                col[q] = T.ci[p];
+                q += v.cnt;
+            }
+        }
+    }
+    DevBuffers& B = *bufs_;
+    W.nval = (int)vmap.size();
+    W.vmap = kupload(vmap, B, stream_);
+    W.dmap = kupload(dmap, B, stream_);
+    const int* dcol = kupload(col, B, stream_);
+    W.val = kalloc<double>(vmap.size(), B);
+    W.diag = kalloc<double>(T.n, B);
+    for (int L = 0; L < nlv; L++) {
+        W.lv[L].col = dcol + base[L];
+        W.lv[L].val = W.val + base[L];
+        W.lv[L].diag = W.diag + off[L];
+    }
+    hip_check(hipStreamSynchronize(stream_), "sync");  // the host arrays die here
+}
+
+// The rows of U's first level, whose U rows are their diagonals alone, get
+// their result from the forward level that solves them.
+int IluSystem::apply_wide(const double* z, double* w, double* part) {
+    int np = 0;
+    for (const dev::TriLevel& L : wl_.lv) {
+        dev::tri_level(stream_, L, z, vT_, ud_, w, part ? z : nullptr, part ? part + np : nullptr);
+        np += dev::tri_level_blocks(L);
+    }
+    for (size_t l = 1; l < wu_.lv.size(); l++) {
+        const dev::TriLevel& L = wu_.lv[l];
+        dev::tri_level(stream_, L, vT_, w, nullptr, nullptr, part ? z : nullptr, part ? part + np : nullptr);
+        np += dev::tri_level_blocks(L);
+    }
+    return np;
 }
 
 void IluSystem::apply(const double* z, double* w) {
@@ -583,18 +667,19 @@ void IluSystem::apply_p(const double* z, double* w) {
         return;
     }
     if (wide_) {
-        dev::tri_levels_wide(stream_, dL_.rp, dL_.ci, dL_.v, hoff_l_, lvl_rows_, z, vT_, 0);
-        dev::tri_levels_wide(stream_, dU_.rp, dU_.ci, dU_.v, hoff_u_, lvu_rows_, vT_, w, 1);
+        apply_wide(z, w, nullptr);
         return;
     }
     dev::trsv(stream_, dL_.rp, dL_.ci, dL_.v, nlv_l_, lvl_off_, lvl_rows_, z, vT_, 0);
     dev::trsv(stream_, dU_.rp, dU_.ci, dU_.v, nlv_u_, lvu_off_, lvu_rows_, vT_, w, 1);
 }
 
-double IluSystem::dot(const double* a, const double* b) {
-    int np = dev::dot_part<double>(stream_, n_, a, b, part_);
-    dev::finalize(stream_, np, part_, scal_, 0, 0);
-    hip_check(hipMemcpyAsync(host_, scal_, sizeof(double), hipMemcpyDeviceToHost, stream_), "d2h");
+double IluSystem::dot(const double* a, const double* b) { return dot_at(a, b, part_); }
+
+double IluSystem::dot_at(const double* a, const double* b, double* part) {
+    int np = dev::dot_part<double>(stream_, n_, a, b, part);
+    dev::finalize(stream_, np, part, scal_, dev::IS_COUNT, 0);
+    hip_check(hipMemcpyAsync(host_, scal_ + dev::IS_COUNT, sizeof(double), hipMemcpyDeviceToHost, stream_), "d2h");
     hip_check(hipStreamSynchronize(stream_), "sync");
     return host_[0];
 }
@@ -615,7 +700,19 @@ int IluSystem::pcg_dev(double* X, double* B, double tol, int max_iter, int stop,
     return it;
 }
 
-// pcg (PCGS.c:163-233) with precon = PCG_preconlr and mat_mult = PCG_mult
+int IluSystem::precon_dot(const double* R, double* Z, double* rz) {
+    if (wide_) return apply_wide(R, Z, rz);
+    apply_p(R, Z);
+    return dev::dot_part<double>(stream_, n_, R, Z, rz);
+}
+
+// pcg (PCGS.c:163-233) with precon = PCG_preconlr and mat_mult = PCG_mult.
+// The scalars stay on the device and the host only watches the loop test's
+// result in pinned memory, two iterations behind what it has queued (an
+// iteration queued after the stop leaves X and R untouched): an iteration of
+// the multicolour order is 7 triangular levels, direction, product and update,
+// where reading three dots back cost 11 more launches and copies and three
+// waits.
 int IluSystem::pcg_core(double* X, double* B, double tol, int max_iter, int stop, double* residuum) {
     if (!ilu_ok_) throw NumericError("ILU(0): zero pivot");
     hipStream_t st = stream_;
@@ -625,32 +722,54 @@ int IluSystem::pcg_core(double* X, double* B, double tol, int max_iter, int stop
     const double inv = (double)1 / h;
     dev::axpby(st, n, inv, B, 0.0, B);
     dev::axpby(st, n, inv, X, 0.0, X);
-    double *R = vR_, *P = vP_, *Q = vQ_, *Z = vZ_, *W = vW_;
+    double *R = vR_, *P = vP_, *Q = vQ_, *Z = vZ_;
     dev::spmv<double, double>(st, dA_, X, B, R, dev::MODE_RES, nullptr, nullptr);
-    apply_p(R, W);
-    double r0 = std::sqrt(dot(W, W));
+    // partials of R.Z, P.Q and R.R: a part each of part_ (40 times a product's workgroups)
+    const int cap = std::max(4096, dev::row_blocks(dA_) + 16);
+    double *rz = part_, *pq = part_ + (size_t)30 * cap, *rr = part_ + (size_t)32 * cap;
+    int nrz = precon_dot(R, Z, rz), nrr = 0;
+    double r0 = std::sqrt(dot_at(Z, Z, part_ + (size_t)34 * cap));
     if (r0 == 0) return 0;
-    double r = r0, s = 0, s_old = 0;
-    int i = 0;
-    do {
-        apply_p(R, Z);
-        s_old = s;
-        s = dot(R, Z);
-        if (i > 0) {
-            double b = s / s_old;
-            dev::axpby(st, n, b, P, 1.0, Z);  // P*b + 1*Z, rounded as scalar_mult then vector_add
-        } else {
-            dev::copy(st, n, (const double*)Z, P);
+    dev::fill<double>(st, dev::IS_COUNT, scal_, 0.0);
+    double* status = host_ + 16;  // four iterations' {number, |R|, stop, iterations done}
+    for (int j = 0; j < 16; j++) status[j] = -1.0;
+    auto folded = [&](int np, const double* part, int slot) {  // few partials are summed where they are used
+        if (np <= dev::IPCG_PARTS) return np;
+        dev::finalize(st, np, part, scal_, slot, 0);
+        return 0;
+    };
+    auto enqueue = [&](int k) {
+        if (k > 0) nrz = precon_dot(R, Z, rz);
+        dev::ipcg_p(st, n, k, P, Z, scal_, rz, folded(nrz, rz, dev::IS_S0 + k % 2), rr, nrr, r0, tol,
+                    stop == LINA_STOP_RELRES, std::max(max_iter, 1), status);
+        const int m = dev::spmv<double, double>(st, dA_, P, nullptr, Q, dev::MODE_OUTER, pq, P);
+        nrr = dev::ipcg_xr(st, n, k, X, R, P, Q, scal_, pq, folded(m, pq, dev::IS_PQ), rr);
+    };
+    auto wait = [&](int k) {  // iteration k - 1's loop test, which iteration k's direction evaluates
+        const double* s = status + 4 * (k % 4);
+        for (long spin = 1;; spin++) {
+            double seen;
+            __atomic_load(s, &seen, __ATOMIC_ACQUIRE);
+            if (seen == (double)k) return s;
+            if (spin % 4096) continue;
+            const hipError_t e = hipStreamQuery(st);
+            if (e == hipErrorNotReady) continue;
+            hip_check(e, "ILU-pcg");
+            __atomic_load(s, &seen, __ATOMIC_ACQUIRE);
+            if (seen != (double)k) throw HipError("ILU-pcg: the loop test was not reported");
         }
-        matvec(P, Q);
-        double a = s / dot(P, Q);
-        dev::axpby(st, n, 1.0, X, a, P);
-        dev::axpby(st, n, 1.0, R, -a, Q);
-        r = std::sqrt(dot(R, R));
-        i++;
-    } while ((stop == LINA_STOP_RELRES ? r : r / r0) > tol && i < max_iter);
-    apply_p(R, W);
-    double rw = std::sqrt(dot(W, W));
+    };
+    enqueue(0);
+    enqueue(1);
+    int i = 0;
+    for (int k = 1;; k++) {
+        const double* s = wait(k);
+        i = (int)s[3];
+        if (s[2] != 0.0) break;
+        enqueue(k + 1);  // its report overwrites iteration k - 3's
+    }
+    // every preconditioner call queued after the stop was on the final R
+    double rw = std::sqrt(dot_at(Z, Z, part_ + (size_t)34 * cap));
     dev::axpby(st, n, h, B, 0.0, B);
     dev::axpby(st, n, h, X, 0.0, X);
     hip_check(hipStreamSynchronize(st), "sync");
