@@ -1036,14 +1036,13 @@ __global__ __launch_bounds__(1024) void k_trsv(const int* __restrict__ rp, const
 
 // The same two sweeps with the factors packed by level (TriPack).  One row
 // per thread; each level's row records are loaded D = 2 levels ahead into
-// registers and stay in flight across the barriers, which fence LDS only: the
-// results a level reads come from the LDS ring, so a level costs an LDS round
-// trip, the row's arithmetic and the barrier, and the record stream (about
-// 72 bytes a row) is bounded by what one compute unit can load -- measured on
-// the 1.05M-row damage factors, 2,049 levels a sweep: 1.35 us a level, one
-// preconditioner application 5.5 ms (11.3 ms a sweep with k_trsv).  Deeper
-// prefetch (4 levels) measured no faster.  The arithmetic is k_trsv's:
-// s = in; s -= v_k x_k in the factor's row order; s /= diag.
+// registers across the barriers, which fence LDS only: the results a level
+// reads come from the LDS ring.  This general form takes any row length, level
+// width and source; its optional loads make the compiler wait for every load
+// in flight at each level (1.0 us a level on 513^2 factors, and deeper
+// prefetch is no faster); k_tri_plain below takes the factors without them.
+// The arithmetic is k_trsv's: s = in; s -= v_k x_k in the factor's row order;
+// s /= diag.
 __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     __builtin_amdgcn_s_barrier();
@@ -1109,7 +1108,9 @@ __device__ __forceinline__ void tri_finish(const TriRow<MAXP, SOR>& row, const S
         }
         x = row.a + (so.omega * s) / row.r.diag;
     } else {
-        x = s / row.r.diag;
+        // ILU's U has a unit diagonal: s / 1 = s, and a level is a third shorter without the division
+        x = s;
+        if (__any(row.r.diag != 1.0)) x = s / row.r.diag;
     }
     ring[t & (TRI_RING - 1)] = x;
     out[row.r.orow] = x;
@@ -1239,6 +1240,99 @@ __global__ __launch_bounds__(TRI_NT) void k_tri_pair(TriPack fw, TriPack bw, con
     tri_phase<MAXP, D, false>(fw, none, zp, y, ring, loff);
     __syncthreads();
     tri_phase<MAXP, D, false>(bw, none, y, w, ring, loff);
+}
+
+// The same for factors whose rows all fit their records, whose sources all lie
+// in the ring and whose levels are at most NT RPT rows wide: one straight line
+// a level.  The general form's optional loads (overflow entries, results through
+// global memory, rows past the first NT) leave the compiler unable to count
+// what is in flight, so that it waits for every load at each level and the
+// prefetch hides nothing.  A level then costs its own chain: the ring reads,
+// the products, the division (L), the ring write and the barrier.
+template <int MAXP, int D, int NT, int RPT>
+__device__ __forceinline__ void tri_phase_plain(const TriPack& a, const double* in, double* out, double* ring,
+                                                int* loff) {
+    constexpr int CH = ((TRI_OFFCAP - 2 * D) / D) * D;  // levels per staged window
+    constexpr int Q = sizeof(TriRec<MAXP>) / 16;
+    const int tid = threadIdx.x;
+    // offsets past the last level repeat its end: empty levels
+    auto stage = [&](int c0) {
+        const int m = min(CH, a.nlv - c0) + 2 * D;
+        for (int q = tid; q < m; q += NT) loff[q] = a.off[min(c0 + q, a.nlv)];
+    };
+    stage(0);
+    __syncthreads();
+    const int4* rec = static_cast<const int4*>(a.rec);
+    int4 raw[D][RPT][Q];
+    double rin[D][RPT];
+    int at[D], end[D];
+    auto load = [&](int d, int b, int e) {
+        at[d] = b + tid;
+        end[d] = e;
+#pragma unroll
+        for (int p = 0; p < RPT; p++) {
+            const int t = at[d] + p * NT < e ? at[d] + p * NT : 0;
+            if (p > 0 && b + p * NT >= e) continue;  // no second rows in this level
+#pragma unroll
+            for (int q = 0; q < Q; q++) raw[d][p][q] = rec[(size_t)t * Q + q];
+            rin[d][p] = in[t];
+        }
+    };
+#pragma unroll
+    for (int d = 0; d < D; d++) {
+        __builtin_amdgcn_sched_barrier(0);
+        load(d, loff[d], loff[d + 1]);
+    }
+    int c0 = 0;
+    for (int L0 = 0; L0 < a.nlv; L0 += D) {
+        if (L0 - c0 >= CH) {
+            // the previous level's barrier ended every read of the old window
+            c0 = L0;
+            stage(c0);
+            lds_barrier();
+        }
+#pragma unroll
+        for (int d = 0; d < D; d++) {
+            __builtin_amdgcn_sched_barrier(0);
+            const int nb = loff[L0 + d + D - c0], ne = loff[L0 + d + D + 1 - c0];
+#pragma unroll
+            for (int p = 0; p < RPT; p++) {
+                if (p > 0 && at[d] - tid + p * NT >= end[d]) continue;
+                // nothing may be computed from the loaded words before their
+                // level: each such hoisted instruction is a wait for its load
+#pragma unroll
+                for (int q = 0; q < Q; q++)
+                    asm volatile("" : "+v"(raw[d][p][q].x), "+v"(raw[d][p][q].y), "+v"(raw[d][p][q].z),
+                                 "+v"(raw[d][p][q].w));
+                asm volatile("" : "+v"(rin[d][p]));
+                TriRec<MAXP> r;
+                __builtin_memcpy(&r, raw[d][p], sizeof(r));
+                double s = rin[d][p];
+#pragma unroll
+                for (int k = 0; k < MAXP; k++) s -= r.val[k] * ring[r.src[k]];
+                double x = s;
+                if (__any(r.diag != 1.0)) x = s / r.diag;
+                const int t = at[d] + p * NT;
+                if (t < end[d]) {
+                    ring[t & (TRI_RING - 1)] = x;
+                    out[r.orow] = x;
+                }
+            }
+            load(d, nb, ne);
+            lds_barrier();
+        }
+    }
+}
+
+template <int MAXP, int D, int NT, int RPT>
+__global__ __launch_bounds__(NT) void k_tri_plain(TriPack fw, TriPack bw, const double* __restrict__ zp, double* y,
+                                                  double* w) {
+    __shared__ double ring[TRI_RING + 1];
+    __shared__ int loff[TRI_OFFCAP];
+    if (threadIdx.x == 0) ring[TRI_RING] = 0.0;
+    tri_phase_plain<MAXP, D, NT, RPT>(fw, zp, y, ring, loff);
+    __syncthreads();
+    tri_phase_plain<MAXP, D, NT, RPT>(bw, y, w, ring, loff);
 }
 
 // one exact lexicographic SOR sweep: in = the gathered right-hand side (f,
@@ -2896,7 +2990,28 @@ void tri_solve_pair(hipStream_t st, const TriPack& fw, const TriPack& bw, const 
                     double* zp, double* y, double* w) {
     if (fw.n <= 0) return;
     hipLaunchKernelGGL(k_gather_perm, dim3(std::min(1024, (fw.n + 255) / 256)), dim3(256), 0, st, fw.n, perm, z, zp);
-    const int maxp = std::max(fw.maxp, bw.maxp);
+    const int maxp = std::max(fw.maxp, bw.maxp), width = std::max(fw.maxw, bw.maxw);
+    // straight-line levels where the packs allow them, with as many threads
+    // as the widest level needs and levels prefetched in the registers that
+    // leaves.  Both sweeps, general form -> here (damage factors): 65^2 229 ->
+    // 69 us, 161^2 559 -> 147, 401^2 1,608 -> 603, 513^2 2,095 -> 1,306, 900^2
+    // 3,955 -> 2,906, 1025^2 4,804 -> 3,973: 0.23 us a level of up to 256 rows,
+    // where the chain bounds it, 0.8 us of up to 1,024, where the records do
+    // (4 levels of 56 KB in flight on one compute unit)
+    if (fw.plain && bw.plain && maxp <= 4 && width <= 2 * TRI_NT) {
+#define LINA_TRI_PLAIN(D, NT, RPT)                                                                          \
+    if (maxp == 4)                                                                                          \
+        hipLaunchKernelGGL((k_tri_plain<4, D, NT, RPT>), dim3(1), dim3(NT), 0, st, fw, bw, zp, y, w);        \
+    else                                                                                                    \
+        hipLaunchKernelGGL((k_tri_plain<3, D, NT, RPT>), dim3(1), dim3(NT), 0, st, fw, bw, zp, y, w)
+        if (width <= 64) { LINA_TRI_PLAIN(8, 64, 1); }
+        else if (width <= 256) { LINA_TRI_PLAIN(8, 256, 1); }
+        else if (width <= 512) { LINA_TRI_PLAIN(6, 512, 1); }
+        else if (width <= 1024) { LINA_TRI_PLAIN(4, 1024, 1); }
+        else { LINA_TRI_PLAIN(3, 1024, 2); }
+#undef LINA_TRI_PLAIN
+        return;
+    }
     if (maxp > 4)
         hipLaunchKernelGGL((k_tri_pair<8, 2>), dim3(1), dim3(TRI_NT), 0, st, fw, bw, zp, y, w);
     else if (maxp == 4)

@@ -312,6 +312,8 @@ struct alignas(16) TriRec<3> {
 static_assert(sizeof(TriRec<3>) == 48 && sizeof(TriRec<4>) == 64 && sizeof(TriRec<8>) == 112, "record layout");
 struct TriPack {
     int n = 0, nlv = 0, maxp = 0;
+    int maxw = 0;                 // rows of the widest level
+    bool plain = false;           // no row past maxp entries, no source outside the ring
     const int* off = nullptr;     // nlv + 1 level offsets, bit 31: full[L]
     const void* rec = nullptr;    // n records TriRec<maxp>
     const int* ovp = nullptr;     // n: first overflow entry of rows with cnt > maxp

@@ -156,6 +156,12 @@ static bool tri_pack(const Csr& T, bool upper, bool pattern_only, const std::vec
     P.n = n;
     P.nlv = nlv;
     P.maxp = MAXP;
+    P.maxw = 0;
+    P.plain = ovmap.empty();
+    for (int L = 0; L < nlv; L++) {
+        P.maxw = std::max(P.maxw, off[L + 1] - off[L]);
+        P.plain = P.plain && !full[L];
+    }
     P.off = kupload(offf, B, st);
     D.rec = kupload(rec, B, st);
     P.rec = D.rec;
