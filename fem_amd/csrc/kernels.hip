@@ -590,7 +590,6 @@ __global__ __launch_bounds__(FTPB) void k_finalize_stop(int np, const double* __
     if (threadIdx.x == 0) {
         const double r = sqrt(t);
         scal[S_R] = r;
-        scal[S_AMG0] = t;  // the next zero-guess preconditioner's r0 test when pcg_xr prepared its entry
         const double it = scal[S_IT] + 1.0;
         scal[S_IT] = it;
         const double crit = relres ? r : r / scal[S_R0];
@@ -724,19 +723,10 @@ __global__ void k_pcg_p(int n, double* __restrict__ P, const double* __restrict_
     }
 }
 
-// pcg: a = s/(P.Q); X += a P; R += (-a) Q; partial |R|^2.  Also the next
-// zero-guess preconditioner entry on the new R where asked (precon_in's
-// outputs, with the signed right-hand side ft = 0 + sg_i r_i when sg is
-// given): ff = (XT) ft when ff is given, xf = the initial guess (0; ft / isa_i
-// on the rows marked in isb) when xf is given.  Sum of squares of ft = that
-// of r.
-template <typename XT>
+// pcg: a = s/(P.Q); X += a P; R += (-a) Q; partial |R|^2
 __global__ __launch_bounds__(TPB) void k_pcg_xr(int n, double* __restrict__ X, double* __restrict__ R,
                                                 const double* __restrict__ P, const double* __restrict__ Q,
-                                                const double* __restrict__ scal, double* __restrict__ part,
-                                                XT* __restrict__ ff, XT* __restrict__ xf,
-                                                const double* __restrict__ sg, const uint32_t* __restrict__ isb,
-                                                const double* __restrict__ isa) {
+                                                const double* __restrict__ scal, double* __restrict__ part) {
     if (scal[S_STOP] != 0.0) return;
     double a = scal[S_S] / scal[S_PQ];
     double na = -a;
@@ -746,18 +736,140 @@ __global__ __launch_bounds__(TPB) void k_pcg_xr(int n, double* __restrict__ X, d
         double r = R[i] + na * Q[i];
         R[i] = r;
         s += r * r;
-        if (ff || xf) {
-            const double ft = sg ? 0.0 + sg[i] * r : r;
-            if (ff) ff[i] = (XT)ft;
-            if (xf) {
-                double x0 = 0.0;
-                if (isolated(isb, i)) x0 = ft / isa[i];
-                xf[i] = (XT)x0;
-            }
-        }
     }
     double t = block_sum(s);
     if (threadIdx.x == 0) part[blockIdx.x] = t;
+}
+
+// The pcg iteration whose sums need no launch (see kernels.hpp).  A dependent
+// launch costs about 3 us however little it does, and small systems' solves
+// are nothing else: three sums, the copy and the event of the loop test were
+// 10 us of an iteration of 70-130 us below 70k rows.
+
+// partial_sum of np > 0 partials (its FTPB threads' order) by a workgroup of
+// TPB, the result in every thread; np = 0: have
+__device__ __forceinline__ double folded_sum(const double* __restrict__ part, int np, double have) {
+    if (np <= 0) return have;
+    constexpr int V = FTPB / TPB;
+    __shared__ double ws[FTPB / WAVE];
+    __shared__ double total;
+#pragma unroll
+    for (int q = 0; q < V; q++) {
+        double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+        int i = threadIdx.x + q * TPB;
+        for (; i + 3 * FTPB < np; i += 4 * FTPB) {
+            s0 += part[i];
+            s1 += part[i + FTPB];
+            s2 += part[i + 2 * FTPB];
+            s3 += part[i + 3 * FTPB];
+        }
+        for (; i < np; i += FTPB) s0 += part[i];
+        const double v = wave_sum((s0 + s1) + (s2 + s3));
+        if (threadIdx.x % WAVE == 0) ws[(threadIdx.x + q * TPB) / WAVE] = v;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double t = 0.0;
+        for (int w = 0; w < FTPB / WAVE; w++) t += ws[w];
+        total = t;
+    }
+    __syncthreads();
+    return total;
+}
+
+// the loop test of iteration k - 1 (PCGS.c:224) on its |R|^2, reported to the host
+__device__ __forceinline__ void loop_test(double* scal, int k, double r2, double r0, double tol, int relres,
+                                          int max_iter, int slot_r, int slot_it, int slot_stop, double* status) {
+    const double r = sqrt(r2), crit = relres ? r : r / r0;
+    const bool was = scal[slot_stop] != 0.0;
+    const bool stop = was || !(crit > tol) || k >= max_iter;
+    scal[slot_r] = r;
+    if (!was) scal[slot_it] = (double)k;
+    if (stop) scal[slot_stop] = 1.0;
+    double* h = status + 4 * (k % 4);
+    h[1] = r;
+    h[2] = stop ? 1.0 : 0.0;
+    h[3] = scal[slot_it];
+    __threadfence_system();
+    __hip_atomic_store(h, (double)k, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+template <typename XT>
+__global__ __launch_bounds__(TPB) void k_precon_out_stop(int n, int k, const XT* __restrict__ xs,
+                                                         double* __restrict__ Z, const double* __restrict__ R,
+                                                         const uint32_t* __restrict__ isb,
+                                                         const double* __restrict__ isa, double* __restrict__ scal,
+                                                         const double* __restrict__ rr, int nrr, double tol,
+                                                         int relres, int max_iter, double* status,
+                                                         double* __restrict__ rz, double* __restrict__ zz) {
+    const double r2 = folded_sum(rr, nrr, scal[S_AMG0]);
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+        loop_test(scal, k, r2, scal[S_R0], tol, relres, max_iter, S_R, S_IT, S_STOP, status);
+    const bool restore = r2 == 0.0;
+    double s = 0.0, q = 0.0;
+    for (int i = blockIdx.x * TPB + threadIdx.x; i < n; i += gridDim.x * TPB) {
+        double z;
+        if (restore) {
+            z = 0.0;
+            if (isolated(isb, i)) z = R[i] / isa[i];
+            Z[i] = z;
+        } else if (xs) {
+            z = (double)xs[i];
+            Z[i] = z;
+        } else {
+            z = Z[i];
+        }
+        s += R[i] * z;
+        q += z * z;
+    }
+    const double t = block_sum(s), u = block_sum(q);
+    if (threadIdx.x == 0) {
+        rz[blockIdx.x] = t;
+        zz[blockIdx.x] = u;
+    }
+}
+
+__global__ __launch_bounds__(TPB) void k_pcg_direction(int n, int k, double* __restrict__ P,
+                                                       const double* __restrict__ Z, double* __restrict__ scal,
+                                                       const double* __restrict__ rz, int nrz) {
+    const double s = folded_sum(rz, nrz, scal[S_S + k % 2]);
+    if (blockIdx.x == 0 && threadIdx.x == 0) scal[S_S + k % 2] = s;
+    if (k == 0) {
+        for (int i = blockIdx.x * TPB + threadIdx.x; i < n; i += gridDim.x * TPB) P[i] = Z[i];
+    } else {
+        const double b = s / scal[S_S + (k + 1) % 2];
+        for (int i = blockIdx.x * TPB + threadIdx.x; i < n; i += gridDim.x * TPB) {
+            const double p = P[i] * b;
+            P[i] = p + 1 * Z[i];
+        }
+    }
+}
+
+template <typename XT>
+__global__ __launch_bounds__(TPB) void k_pcg_update(int n, int k, double* __restrict__ X, double* __restrict__ R,
+                                                    const double* __restrict__ P, const double* __restrict__ Q,
+                                                    const double* __restrict__ scal, const double* __restrict__ pq,
+                                                    int npq, double* __restrict__ rr, XT* __restrict__ ff,
+                                                    XT* __restrict__ xf, const uint32_t* __restrict__ isb,
+                                                    const double* __restrict__ isa) {
+    if (scal[S_STOP] != 0.0) return;
+    const double a = scal[S_S + k % 2] / folded_sum(pq, npq, scal[S_PQ]);
+    const double na = -a;
+    double s = 0.0;
+    for (int i = blockIdx.x * TPB + threadIdx.x; i < n; i += gridDim.x * TPB) {
+        X[i] += a * P[i];
+        const double r = R[i] + na * Q[i];
+        R[i] = r;
+        s += r * r;
+        if (ff) ff[i] = (XT)r;
+        if (xf) {
+            double x0 = 0.0;
+            if (isolated(isb, i)) x0 = r / isa[i];
+            xf[i] = (XT)x0;
+        }
+    }
+    const double t = block_sum(s);
+    if (threadIdx.x == 0) rr[blockIdx.x] = t;
 }
 
 // generic x += f*y with f = sign * scal[slot_a] / scal[slot_b] (slot_b < 0: 1)
@@ -1595,44 +1707,17 @@ __global__ void k_tri_gather(int n, const int* __restrict__ map, const double* _
         val[q] = map[q] >= 0 ? v[map[q]] : 0.0;
 }
 
-// the sum of np partials (np > 0) in one fixed order, in every thread; else have
-__device__ __forceinline__ double parts_sum(const double* __restrict__ part, int np, double have) {
-    if (np <= 0) return have;
-    __shared__ double total;
-    double s = 0.0;
-    for (int i = threadIdx.x; i < np; i += TPB) s += part[i];
-    s = block_sum(s);
-    if (threadIdx.x == 0) total = s;
-    __syncthreads();
-    s = total;
-    __syncthreads();
-    return s;
-}
-
 __global__ __launch_bounds__(TPB) void k_ipcg_p(int n, int k, double* __restrict__ P, const double* __restrict__ Z,
                                                 double* __restrict__ scal, const double* __restrict__ rz, int nrz,
                                                 const double* __restrict__ rr, int nrr, double r0, double tol,
                                                 int relres, int max_iter, double* status) {
-    const double s = parts_sum(rz, nrz, scal[IS_S0 + k % 2]);
+    const double s = folded_sum(rz, nrz, scal[IS_S0 + k % 2]);
     const double b = k > 0 ? s / scal[IS_S0 + (k + 1) % 2] : 0.0;
     if (blockIdx.x == 0) {
-        const double r2 = k > 0 ? parts_sum(rr, nrr, scal[IS_RR]) : 0.0;
+        const double r2 = k > 0 ? folded_sum(rr, nrr, scal[IS_RR]) : 0.0;
         if (threadIdx.x == 0) {
             scal[IS_S0 + k % 2] = s;
-            if (k > 0) {
-                // the loop condition of PCGS.c:224
-                const double r = sqrt(r2), crit = relres ? r : r / r0;
-                const bool was = scal[IS_STOP] != 0.0;
-                const bool stop = was || !(crit > tol) || k >= max_iter;
-                if (!was) scal[IS_IT] = (double)k;
-                if (stop) scal[IS_STOP] = 1.0;
-                double* h = status + 4 * (k % 4);
-                h[1] = r;
-                h[2] = stop ? 1.0 : 0.0;
-                h[3] = scal[IS_IT];
-                __threadfence_system();
-                __hip_atomic_store(h, (double)k, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-            }
+            if (k > 0) loop_test(scal, k, r2, r0, tol, relres, max_iter, IS_R, IS_IT, IS_STOP, status);
         }
     }
     for (int i = blockIdx.x * TPB + threadIdx.x; i < n; i += gridDim.x * TPB)
@@ -1644,7 +1729,7 @@ __global__ __launch_bounds__(TPB) void k_ipcg_xr(int n, int k, double* __restric
                                                  const double* __restrict__ scal, const double* __restrict__ pq,
                                                  int npq, double* __restrict__ rr) {
     if (scal[IS_STOP] != 0.0) return;
-    const double a = scal[IS_S0 + k % 2] / parts_sum(pq, npq, scal[IS_PQ]);
+    const double a = scal[IS_S0 + k % 2] / folded_sum(pq, npq, scal[IS_PQ]);
     double s = 0.0;
     for (int i = blockIdx.x * TPB + threadIdx.x; i < n; i += gridDim.x * TPB) {
         X[i] += a * P[i];
@@ -2811,17 +2896,46 @@ void pcg_p(hipStream_t st, int n, double* P, const double* Z, const double* scal
     hipLaunchKernelGGL(k_pcg_p, dim3(grid_for(n)), dim3(TPB), 0, st, n, P, Z, scal, first);
 }
 
-template <typename XT>
 int pcg_xr(hipStream_t st, int n, double* X, double* R, const double* P, const double* Q, const double* scal,
-           double* part, XT* ff, XT* xf, const double* sg, const uint32_t* isb, const double* isa) {
+           double* part) {
     int g = grid_for(n, 1024);
-    hipLaunchKernelGGL((k_pcg_xr<XT>), dim3(g), dim3(TPB), 0, st, n, X, R, P, Q, scal, part, ff, xf, sg, isb, isa);
+    hipLaunchKernelGGL(k_pcg_xr, dim3(g), dim3(TPB), 0, st, n, X, R, P, Q, scal, part);
     return g;
 }
-template int pcg_xr<double>(hipStream_t, int, double*, double*, const double*, const double*, const double*, double*,
-                            double*, double*, const double*, const uint32_t*, const double*);
-template int pcg_xr<float>(hipStream_t, int, double*, double*, const double*, const double*, const double*, double*,
-                           float*, float*, const double*, const uint32_t*, const double*);
+
+template <typename XT>
+int precon_out_stop(hipStream_t st, int n, int k, const XT* xs, double* Z, const double* R, const uint32_t* isb,
+                    const double* isa, double* scal, const double* rr, int nrr, double tol, int relres, int max_iter,
+                    double* status, double* rz, double* zz) {
+    const int g = grid_for(n, 1024);
+    hipLaunchKernelGGL((k_precon_out_stop<XT>), dim3(g), dim3(TPB), 0, st, n, k, xs, Z, R, isb, isa, scal, rr, nrr,
+                       tol, relres, max_iter, status, rz, zz);
+    return g;
+}
+template int precon_out_stop<double>(hipStream_t, int, int, const double*, double*, const double*, const uint32_t*,
+                                     const double*, double*, const double*, int, double, int, int, double*, double*,
+                                     double*);
+template int precon_out_stop<float>(hipStream_t, int, int, const float*, double*, const double*, const uint32_t*,
+                                    const double*, double*, const double*, int, double, int, int, double*, double*,
+                                     double*);
+
+void pcg_direction(hipStream_t st, int n, int k, double* P, const double* Z, double* scal, const double* rz, int nrz) {
+    hipLaunchKernelGGL(k_pcg_direction, dim3(grid_for(n, 2048)), dim3(TPB), 0, st, n, k, P, Z, scal, rz, nrz);
+}
+
+template <typename XT>
+int pcg_update(hipStream_t st, int n, int k, double* X, double* R, const double* P, const double* Q,
+               const double* scal, const double* pq, int npq, double* rr, XT* ff, XT* xf, const uint32_t* isb,
+               const double* isa) {
+    const int g = grid_for(n, 1024);
+    hipLaunchKernelGGL((k_pcg_update<XT>), dim3(g), dim3(TPB), 0, st, n, k, X, R, P, Q, scal, pq, npq, rr, ff, xf, isb,
+                       isa);
+    return g;
+}
+template int pcg_update<double>(hipStream_t, int, int, double*, double*, const double*, const double*, const double*,
+                                const double*, int, double*, double*, double*, const uint32_t*, const double*);
+template int pcg_update<float>(hipStream_t, int, int, double*, double*, const double*, const double*, const double*,
+                               const double*, int, double*, float*, float*, const uint32_t*, const double*);
 
 void axpy_s(hipStream_t st, int n, double* x, const double* y, const double* scal, int slot_a, int slot_b,
             double sign) {

@@ -168,7 +168,7 @@ int dot_part(hipStream_t st, int n, const XT* a, const XT* b, double* part);
 // scal[slot] = sum(part); op 0 plain, 1 sqrt, 2 shift (scal[slot+1] = scal[slot]) then plain
 void finalize(hipStream_t st, int np, const double* part, double* scal, int slot, int op);
 // pcg's residual norm and stop test: unless scal[S_STOP] is already set,
-// scal[S_R] = sqrt(sum(part)), scal[S_AMG0] = sum(part), scal[S_IT] += 1 and
+// scal[S_R] = sqrt(sum(part)), scal[S_IT] += 1 and
 // scal[S_STOP] = 1 when
 // !((relres ? r : r / scal[S_R0]) > tol), r is NaN or S_IT reached max_iter
 void finalize_stop(hipStream_t st, int np, const double* part, double* scal, double tol, int relres, int max_iter);
@@ -234,12 +234,30 @@ void scale(hipStream_t st, int n, double* x, double a);       // x_i *= a
 void restore_if_zero(hipStream_t st, int n, double* x, const double* scal, int slot, int m, const int* rows,
                      const double* a, const double* f);
 void pcg_p(hipStream_t st, int n, double* P, const double* Z, const double* scal, int first);
-// (skips every update once scal[S_STOP] is set).  ff, xf: also the next
-// zero-guess preconditioner entry on the new R, see k_pcg_xr
-template <typename XT = double>
+// The same iteration without launches for its sums (Solver::pcg_dev with a
+// preconditioner of one V-cycle): np partials (at most PCG_PARTS) are added by
+// every workgroup that needs them, in finalize's order (the same bits); np =
+// 0: already in scal.  S_k is scal[S_S + k % 2].
+constexpr int PCG_PARTS = 2048;
+// precon_out of iteration k >= 1, whose zero test and loop test are on |R|^2
+// of iteration k - 1: the test (finalize_stop's) sets scal[S_STOP] and reports
+// {k, |R|, stop, iterations} to the host's status[4 (k % 4) ...]; rz, zz: the
+// partials of R.Z and Z.Z
+template <typename XT>
+int precon_out_stop(hipStream_t st, int n, int k, const XT* xs, double* Z, const double* R, const uint32_t* isb,
+                    const double* isa, double* scal, const double* rr, int nrr, double tol, int relres, int max_iter,
+                    double* status, double* rz, double* zz);
+void pcg_direction(hipStream_t st, int n, int k, double* P, const double* Z, double* scal, const double* rz, int nrz);
+// k_pcg_xr's updates and |R|^2 partials, and the next preconditioner's entry
+// on the new R: ff = (XT) R when given, xf = the initial guess (0; R_i / isa_i
+// on the rows marked in isb) when given
+template <typename XT>
+int pcg_update(hipStream_t st, int n, int k, double* X, double* R, const double* P, const double* Q,
+               const double* scal, const double* pq, int npq, double* rr, XT* ff, XT* xf, const uint32_t* isb,
+               const double* isa);
+// (skips every update once scal[S_STOP] is set)
 int pcg_xr(hipStream_t st, int n, double* X, double* R, const double* P, const double* Q, const double* scal,
-           double* part, XT* ff = nullptr, XT* xf = nullptr, const double* sg = nullptr, const uint32_t* isb = nullptr,
-           const double* isa = nullptr);
+           double* part);
 void axpy_s(hipStream_t st, int n, double* x, const double* y, const double* scal, int slot_a, int slot_b,
             double sign);
 void axpby(hipStream_t st, int n, double a, double* x, double b, const double* y);
@@ -385,11 +403,8 @@ void tri_level(hipStream_t st, const TriLevel& L, const double* in, double* out,
 // val[q] = v[map[q]] (map < 0: 0) for the padded entries and diagonals of a factor
 void tri_values(hipStream_t st, int n, const int* map, const double* v, double* val);
 
-// ILU-pcg on the device (IluSystem::pcg_core).  The sum of np partials is
-// taken by every workgroup that needs it (np <= IPCG_PARTS) instead of a
-// launch of its own; np = 0: already in scal (k_finalize).
-constexpr int IPCG_PARTS = 2048;
-enum { IS_S0 = 0, IS_S1 = 1, IS_PQ = 2, IS_RR = 3, IS_STOP = 4, IS_IT = 5, IS_COUNT = 8 };
+// ILU-pcg on the device (IluSystem::pcg_core), its sums as in pcg_direction
+enum { IS_S0 = 0, IS_S1 = 1, IS_PQ = 2, IS_RR = 3, IS_STOP = 4, IS_IT = 5, IS_R = 6, IS_COUNT = 8 };
 // iteration k's direction P = Z (k = 0) or b P + Z, b = S_k / S_{k-1}, with
 // S_k = R.Z from its partials; before it, for k > 0, the loop test of
 // iteration k - 1 on |R|^2 from its partials: scal[IS_STOP] and, for the host,

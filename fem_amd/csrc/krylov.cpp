@@ -740,7 +740,7 @@ int IluSystem::pcg_core(double* X, double* B, double tol, int max_iter, int stop
     double* status = host_ + 16;  // four iterations' {number, |R|, stop, iterations done}
     for (int j = 0; j < 16; j++) status[j] = -1.0;
     auto folded = [&](int np, const double* part, int slot) {  // few partials are summed where they are used
-        if (np <= dev::IPCG_PARTS) return np;
+        if (np <= dev::PCG_PARTS) return np;
         dev::finalize(st, np, part, scal_, slot, 0);
         return 0;
     };
@@ -751,25 +751,11 @@ int IluSystem::pcg_core(double* X, double* B, double tol, int max_iter, int stop
         const int m = dev::spmv<double, double>(st, dA_, P, nullptr, Q, dev::MODE_OUTER, pq, P);
         nrr = dev::ipcg_xr(st, n, k, X, R, P, Q, scal_, pq, folded(m, pq, dev::IS_PQ), rr);
     };
-    auto wait = [&](int k) {  // iteration k - 1's loop test, which iteration k's direction evaluates
-        const double* s = status + 4 * (k % 4);
-        for (long spin = 1;; spin++) {
-            double seen;
-            __atomic_load(s, &seen, __ATOMIC_ACQUIRE);
-            if (seen == (double)k) return s;
-            if (spin % 4096) continue;
-            const hipError_t e = hipStreamQuery(st);
-            if (e == hipErrorNotReady) continue;
-            hip_check(e, "ILU-pcg");
-            __atomic_load(s, &seen, __ATOMIC_ACQUIRE);
-            if (seen != (double)k) throw HipError("ILU-pcg: the loop test was not reported");
-        }
-    };
     enqueue(0);
     enqueue(1);
     int i = 0;
     for (int k = 1;; k++) {
-        const double* s = wait(k);
+        const double* s = wait_status(status, k, st);  // iteration k - 1's loop test
         i = (int)s[3];
         if (s[2] != 0.0) break;
         enqueue(k + 1);  // its report overwrites iteration k - 3's

@@ -52,6 +52,21 @@ void hip_check(hipError_t e, const char* what) {
     if (e != hipSuccess) throw HipError(std::string(what) + ": " + hipGetErrorString(e));
 }
 
+const double* wait_status(const double* status, int k, hipStream_t st) {
+    const double* s = status + 4 * (k % 4);
+    for (long spin = 1;; spin++) {
+        double seen;
+        __atomic_load(s, &seen, __ATOMIC_ACQUIRE);
+        if (seen == (double)k) return s;
+        if (spin % 4096) continue;
+        const hipError_t e = hipStreamQuery(st);
+        if (e == hipErrorNotReady) continue;
+        hip_check(e, "loop test");
+        __atomic_load(s, &seen, __ATOMIC_ACQUIRE);
+        if (seen != (double)k) throw HipError("the loop test was not reported");
+    }
+}
+
 // ------------------------------------------------------------ memory
 
 DevBuffers::~DevBuffers() {
@@ -799,7 +814,7 @@ void Solver::upload() {
     kB_ = dalloc<double>(n, B);
     // block partials: one per SpMV block (any matrix) or per reduction block
     int np = std::max(4096, maxblk + 16);
-    part_ = dalloc<double>(np, B);
+    part_ = dalloc<double>(np + 4 * dev::DOT_PART_MAX, B);  // and four dots' partials beside a product's
     part_cap_ = np;
     scal_ = dalloc<double>(dev::S_COUNT, B);
     dev::fill(st, dev::S_COUNT, scal_, 0.0);
@@ -1600,17 +1615,14 @@ int Solver::amg_solve_dev(const double* F, double* X, double* relres) {
 // result is replaced by the untouched guess on the device when r0 == 0.
 // w != nullptr: also the block partials of w.X into part_ (their number in
 // *np), the dot k_dot_part(w, X) would give.
-// prepared: pcg_xr already wrote this entry's outputs for F (the signed
-// right-hand side, its FP32 copy, the initial guess, scal[S_AMG0]); see
-// entry_prepared.
-int Solver::vcycle_once(const double* F, double* X, const double* w, int* np, bool prepared) {
+int Solver::vcycle_once(const double* F, double* X, const double* w, int* np) {
     hipStream_t st = stream_;
     DevLevel& top = L_.back();
     const int n = top.n;
     const int lt = (int)L_.size() - 1;
     const double* Ft = F;
     if (has_neg_signs_) {
-        if (!prepared) dev::signs(st, n, signs_, F, ftop_);
+        dev::signs(st, n, signs_, F, ftop_);
         Ft = ftop_;
     }
     // without isolated rows the guess is exactly zero and the pre-smoother
@@ -1619,14 +1631,11 @@ int Solver::vcycle_once(const double* F, double* X, const double* w, int* np, bo
     const bool fp64 = prm_.precision == LINA_PREC_FP64;
     int npd = 0;
     if (isa_ok_) {
-        // entry and exit fused into one elementwise kernel each (the entry
-        // into pcg_xr when prepared)
-        if (!prepared) {
-            int n0;
-            if (fp64) n0 = dev::precon_in<double>(st, n, Ft, part_, xz ? nullptr : X, nullptr, nullptr, isb_, isa_);
-            else n0 = dev::precon_in<float>(st, n, Ft, part_, nullptr, xz ? nullptr : top.xf, top.ff, isb_, isa_);
-            dev::finalize(st, n0, part_, scal_, dev::S_AMG0, 0);
-        }
+        // entry and exit fused into one elementwise kernel each
+        int n0;
+        if (fp64) n0 = dev::precon_in<double>(st, n, Ft, part_, xz ? nullptr : X, nullptr, nullptr, isb_, isa_);
+        else n0 = dev::precon_in<float>(st, n, Ft, part_, nullptr, xz ? nullptr : top.xf, top.ff, isb_, isa_);
+        dev::finalize(st, n0, part_, scal_, dev::S_AMG0, 0);
         if (fp64) {
             vcycle<double>(lt, Ft, X, xz ? X_ZERO : X_GUESS);
             npd = dev::precon_out<double>(st, n, nullptr, X, Ft, isb_, isa_, scal_, dev::S_AMG0, w, part_);
@@ -1635,7 +1644,6 @@ int Solver::vcycle_once(const double* F, double* X, const double* w, int* np, bo
             npd = dev::precon_out<float>(st, n, top.xf, X, Ft, isb_, isa_, scal_, dev::S_AMG0, w, part_);
         }
     } else {
-        if (prepared) throw std::logic_error("vcycle_once: prepared entry without the fused path");
         int n0 = dev::dot_part<double>(st, n, Ft, Ft, part_);
         dev::finalize(st, n0, part_, scal_, dev::S_AMG0, 0);
         if (!xz) {
@@ -1665,14 +1673,13 @@ bool Solver::precon_async() const {
     return prm_.zero_init && prm_.amg_max_iter == 1 && prm_.cycle == LINA_CYCLE_V;
 }
 
-// pcg_xr can write the next preconditioner entry (vcycle_once's fused path;
+// pcg_update can write the next preconditioner entry (vcycle_once's fused path;
 // not with make_positive_diag signs, whose signed right-hand side precon_out
 // would also need)
 bool Solver::entry_prepared_ok() const { return precon_async() && isa_ok_ && !has_neg_signs_; }
 
-int Solver::precon(const double* R, double* Z, const double* w, int* np, bool prepared) {
-    if (precon_async()) return vcycle_once(R, Z, w, np, prepared);
-    if (prepared) throw std::logic_error("precon: prepared entry without a one-V-cycle preconditioner");
+int Solver::precon(const double* R, double* Z, const double* w, int* np) {
+    if (precon_async()) return vcycle_once(R, Z, w, np);
     if (prm_.zero_init) dev::fill<double>(stream_, n_, Z, 0.0);
     int it = amg_solve_dev(R, Z);
     if (w) *np = dev::dot_part<double>(stream_, n_, w, Z, part_);
@@ -1680,10 +1687,16 @@ int Solver::precon(const double* R, double* Z, const double* w, int* np, bool pr
 }
 
 // pcg (PCGS.c:163-233) on device vectors X, B (length n).  The loop test is
-// evaluated on the device (k_finalize_stop); with a preconditioner that needs
-// no host round trip, iteration k+1 is queued before the host waits for
-// iteration k's test, and an iteration queued after the stop leaves X, R and
-// the scalars untouched.
+// evaluated on the device; with a preconditioner that needs no host round
+// trip, iteration k+1 is queued before the host sees iteration k's test, and
+// an iteration queued after the stop leaves X, R and the scalars untouched.
+//
+// A one-V-cycle preconditioner without row signs (fused) has three launches
+// an iteration around its V-cycle and the product: the exit kernel with the
+// loop test of the previous iteration, the direction and the update, each
+// adding up the partial sums it needs; the first preconditioned residual is
+// iteration 0's, and the last one that of the iteration queued at the stop.
+// Other preconditioners keep a launch per sum.
 int Solver::pcg_dev(double* X, double* B, double tol, int max_iter, int stop, lina_stats* stats) {
     hipStream_t st = stream_;
     const int n = n_;
@@ -1701,9 +1714,13 @@ int Solver::pcg_dev(double* X, double* B, double tol, int max_iter, int stop, li
     double* P = kP_;
     double* Q = kQ_;
     double* Z = kZ_;
-    double* W = kW_;
-    dev::fill<double>(st, n, W, 0.0);
-    dev::fill<double>(st, n, Z, 0.0);
+    const bool fused = entry_prepared_ok();
+    const bool fp64 = prm_.precision == LINA_PREC_FP64;
+    double* W = fused ? Z : kW_;
+    if (!fused) {  // the preconditioner's starting vectors
+        dev::fill<double>(st, n, W, 0.0);
+        dev::fill<double>(st, n, Z, 0.0);
+    }
     // R = B + (-1)*(A X) with the caller's matrix (rows of the stored finest
     // matrix carry the make_positive_diag signs)
     if (op_) {
@@ -1728,78 +1745,122 @@ int Solver::pcg_dev(double* X, double* B, double tol, int max_iter, int stop, li
     }
     const int relres = stop == LINA_STOP_RELRES;
     const int cap = std::max(max_iter, 1);  // the loop body runs at least once
-    // one iteration: Z = M^-1 R with R.Z, P, Q = A P with P.Q, X and R with
-    // |R| and the stop test; its state (S_R..S_IT) copied to ring slot k % 2
     // kernel timing samples every fourth iteration's outer SpMV (the events
     // themselves cost a few microseconds)
     auto sampled = [&](int k) { return ktime_ && k % 4 == 0; };
-    // from the second iteration on, pcg_xr writes the preconditioner's entry
-    // on the new R (its FP32 copy, initial guess and r0 test)
-    const bool prep = entry_prepared_ok();
-    const bool fixed = prm_.precision == LINA_PREC_MIXED && fixed_order();
-    auto enqueue = [&](int k) {
-        int m = 0;
-        precon(R, Z, R, &m, prep && k > 0);
-        dev::finalize(st, m, part_, scal_, dev::S_S, 2);  // s_old = s; s = R.Z
-        dev::pcg_p(st, n, P, Z, scal_, k == 0);
-        if (op_) {
-            m = op_->launch_on(st, P, nullptr, Q, dev::MODE_OUTER, part_, P);
-        } else if (has_neg_signs_) {
-            apply_A(P, Q);
-            m = dev::dot_part<double>(st, n, P, Q, part_);
-        } else {
-            if (sampled(k))  // the events bracket the kernel itself
-                m = dev::spmv_outer_timed(st, top.A, P, Q, part_, P, evk_[k % 2][0], evk_[k % 2][1], fixed);
-            else
-                m = dev::spmv<double, double>(st, top.A, P, nullptr, Q, dev::MODE_OUTER, part_, P, nullptr,
-                                              fixed);  // Q = A P, P.Q
-        }
-        dev::finalize(st, m, part_, scal_, dev::S_PQ, 0);
-        if (!prep) {
-            m = dev::pcg_xr(st, n, X, R, P, Q, scal_, part_);
-        } else if (prm_.precision == LINA_PREC_FP64) {
-            m = dev::pcg_xr<double>(st, n, X, R, P, Q, scal_, part_, nullptr, niso_ == 0 ? nullptr : Z, nullptr,
-                                    isb_, isa_);
-        } else {
-            m = dev::pcg_xr<float>(st, n, X, R, P, Q, scal_, part_, top.ff, niso_ == 0 ? nullptr : top.xf, nullptr,
-                                   isb_, isa_);
-        }
-        dev::finalize_stop(st, m, part_, scal_, tol, relres, cap);
-        double* h = host_ring_ + (k % 2) * dev::S_COUNT;
-        hip_check(hipMemcpyAsync(h + dev::S_R, scal_ + dev::S_R, (dev::S_IT - dev::S_R + 1) * sizeof(double),
-                                 hipMemcpyDeviceToHost, st),
-                  "d2h");
-        hip_check(hipEventRecord(evr_[k % 2], st), "event");
-    };
     const bool timed = ktime_ && !has_neg_signs_ && !op_;
-    const int ahead = precon_async() ? 2 : 1;
+    const bool fixed = !fp64 && fixed_order();
+    // Q = A P and the partials of P.Q in part
+    auto product = [&](int k, double* part) {
+        if (op_) return op_->launch_on(st, P, nullptr, Q, dev::MODE_OUTER, part, P);
+        if (has_neg_signs_) {
+            apply_A(P, Q);
+            return dev::dot_part<double>(st, n, P, Q, part);
+        }
+        if (sampled(k))  // the events bracket the kernel itself
+            return dev::spmv_outer_timed(st, top.A, P, Q, part, P, evk_[k % 2][0], evk_[k % 2][1], fixed);
+        return dev::spmv<double, double>(st, top.A, P, nullptr, Q, dev::MODE_OUTER, part, P, nullptr, fixed);
+    };
     double ksum = 0.0;
     int kcount = 0;
-    int enq = 0, done = 0;
+    auto sample = [&](int k) {
+        float kms = 0;
+        hip_check(hipEventSynchronize(evk_[k % 2][1]), "event sync");
+        hip_check(hipEventElapsedTime(&kms, evk_[k % 2][0], evk_[k % 2][1]), "elapsed");
+        ksum += kms;
+        kcount++;
+    };
     double r = 0.0;
     int i = 0;
-    for (;;) {
-        while (enq < cap && enq - done < ahead) enqueue(enq++);
-        hip_check(hipEventSynchronize(evr_[done % 2]), "event sync");
-        const double* h = host_ring_ + (done % 2) * dev::S_COUNT;
-        const int it_dev = (int)h[dev::S_IT];
-        if (timed && sampled(done) && it_dev == done + 1) {
-            float kms = 0;
-            hip_check(hipEventElapsedTime(&kms, evk_[done % 2][0], evk_[done % 2][1]), "elapsed");
-            ksum += kms;
-            kcount++;
+    if (fused) {
+        double *pq = part_, *rz = part_ + part_cap_, *rr = rz + dev::DOT_PART_MAX;
+        double* zz[2] = {rr + dev::DOT_PART_MAX, rr + 2 * dev::DOT_PART_MAX};
+        double* status = host_ring_;
+        for (int j = 0; j < 16; j++) status[j] = -1.0;
+        auto folded = [&](int m, const double* part, int slot) {  // many partials keep their launch
+            if (m <= dev::PCG_PARTS) return m;
+            dev::finalize(st, m, part, scal_, slot, 0);
+            return 0;
+        };
+        int nrr = 0, nzz = 0;
+        auto enqueue = [&](int k) {
+            int nrz;
+            if (k == 0) {
+                nrz = dev::dot_part<double>(st, n, R, Z, rz);
+            } else if (fp64) {
+                vcycle<double>((int)L_.size() - 1, R, Z, niso_ == 0 ? X_ZERO : X_GUESS);
+                nrz = dev::precon_out_stop<double>(st, n, k, nullptr, Z, R, isb_, isa_, scal_, rr, nrr, tol, relres,
+                                                   cap, status, rz, zz[k % 2]);
+            } else {
+                vcycle<float>((int)L_.size() - 1, top.ff, top.xf, niso_ == 0 ? X_ZERO : X_GUESS);
+                nrz = dev::precon_out_stop<float>(st, n, k, top.xf, Z, R, isb_, isa_, scal_, rr, nrr, tol, relres,
+                                                  cap, status, rz, zz[k % 2]);
+            }
+            nzz = nrz;
+            dev::pcg_direction(st, n, k, P, Z, scal_, rz, nrz);
+            const int m = product(k, pq);
+            const int mf = folded(m, pq, dev::S_PQ);
+            if (fp64)
+                nrr = dev::pcg_update<double>(st, n, k, X, R, P, Q, scal_, pq, mf, rr, nullptr,
+                                              niso_ == 0 ? nullptr : Z, isb_, isa_);
+            else
+                nrr = dev::pcg_update<float>(st, n, k, X, R, P, Q, scal_, pq, mf, rr, top.ff,
+                                             niso_ == 0 ? nullptr : top.xf, isb_, isa_);
+        };
+        enqueue(0);
+        enqueue(1);
+        int k = 1;
+        for (;; k++) {
+            const double* s = wait_status(status, k, st);  // iteration k - 1's loop test
+            if (timed && sampled(k - 1) && (int)s[3] == k) sample(k - 1);
+            r = s[1];
+            i = (int)s[3];
+            if (s[2] != 0.0) break;
+            enqueue(k + 1);
         }
-        r = h[dev::S_R];
-        i = it_dev;
-        done++;
-        if (h[dev::S_STOP] != 0.0 || (done == enq && enq >= cap)) break;
+        // iteration k preconditioned the final R (one queued after it started
+        // from another guess); the reference's calls: one before the loop,
+        // one an iteration, one after it
+        precon_calls_ = vcycles_ = i + 2;
+        dev::finalize(st, nzz, zz[k % 2], scal_, dev::S_T1, 1);
+    } else {
+        // one iteration: Z = M^-1 R with R.Z, P, Q = A P with P.Q, X and R
+        // with |R| and the stop test; its state (S_R..S_IT) copied to ring slot k % 2
+        auto enqueue = [&](int k) {
+            int m = 0;
+            precon(R, Z, R, &m);
+            dev::finalize(st, m, part_, scal_, dev::S_S, 2);  // s_old = s; s = R.Z
+            dev::pcg_p(st, n, P, Z, scal_, k == 0);
+            m = product(k, part_);
+            dev::finalize(st, m, part_, scal_, dev::S_PQ, 0);
+            m = dev::pcg_xr(st, n, X, R, P, Q, scal_, part_);
+            dev::finalize_stop(st, m, part_, scal_, tol, relres, cap);
+            double* h = host_ring_ + (k % 2) * dev::S_COUNT;
+            hip_check(hipMemcpyAsync(h + dev::S_R, scal_ + dev::S_R, (dev::S_IT - dev::S_R + 1) * sizeof(double),
+                                     hipMemcpyDeviceToHost, st),
+                      "d2h");
+            hip_check(hipEventRecord(evr_[k % 2], st), "event");
+        };
+        const int ahead = precon_async() ? 2 : 1;
+        int enq = 0, done = 0;
+        for (;;) {
+            while (enq < cap && enq - done < ahead) enqueue(enq++);
+            hip_check(hipEventSynchronize(evr_[done % 2]), "event sync");
+            const double* h = host_ring_ + (done % 2) * dev::S_COUNT;
+            const int it_dev = (int)h[dev::S_IT];
+            if (timed && sampled(done) && it_dev == done + 1) sample(done);
+            r = h[dev::S_R];
+            i = it_dev;
+            done++;
+            if (h[dev::S_STOP] != 0.0 || (done == enq && enq >= cap)) break;
+        }
+        // an iteration queued after the stop ran its V-cycle and nothing else
+        vcycles_ -= enq - i;
+        precon_calls_ -= enq - i;
+        precon(R, W, W, &np);
+        dev::finalize(st, np, part_, scal_, dev::S_T1, 1);
     }
-    // an iteration queued after the stop ran its V-cycle and nothing else
-    vcycles_ -= enq - i;
-    precon_calls_ -= enq - i;
-    double relres_out = r;
-    precon(R, W, W, &np);
-    dev::finalize(st, np, part_, scal_, dev::S_T1, 1);
+    const double relres_out = r;
     double rw = read_scalar(dev::S_T1);
     dev::scale_by(st, n, B, scal_, dev::S_H, 0);
     dev::scale_by(st, n, X, scal_, dev::S_H, 0);

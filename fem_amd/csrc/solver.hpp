@@ -28,6 +28,11 @@ struct NumericError : std::runtime_error {
 void hip_check(hipError_t e, const char* what);
 const char* last_error();
 
+// The report of iteration number k of a device-side loop: waits until
+// status[4 (k % 4)] (pinned, written by a kernel on st) reads k; returns that
+// slot.  Throws when st fails or runs out of work without the report.
+const double* wait_status(const double* status, int k, hipStream_t st);
+
 struct DevBuffers {
     std::vector<void*> ptrs;
     ~DevBuffers();
@@ -215,8 +220,8 @@ class Solver {
     int amg_solve_dev(const double* F, double* X, double* relres = nullptr);
     int amg_solve_host(const double* f, double* x, double* relres = nullptr);
     // Z = M^-1 R; w != nullptr: block partials of w.Z in part(), their number in *np
-    int precon(const double* R, double* Z, const double* w = nullptr, int* np = nullptr, bool prepared = false);
-    int vcycle_once(const double* F, double* X, const double* w = nullptr, int* np = nullptr, bool prepared = false);
+    int precon(const double* R, double* Z, const double* w = nullptr, int* np = nullptr);
+    int vcycle_once(const double* F, double* X, const double* w = nullptr, int* np = nullptr);
     bool precon_async() const;
     bool entry_prepared_ok() const;
     int spmv_host(int level, int precision, const double* x, double* y);
