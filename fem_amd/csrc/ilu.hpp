@@ -85,6 +85,8 @@ class IluSystem {
     TriWide wl_, wu_;
     int* udmap_ = nullptr;   // rows whose U row is the diagonal alone: its entry (-1: other rows)
     double* ud_ = nullptr;   // and its value (0: other rows)
+    Captured iteration_;     // some pcg iterations on this upload's buffers (X in vXg_)
+    double* vXg_ = nullptr;
     // Z = M^-1 R and the block partials of R.Z in rz, returns their number
     int precon_dot(const double* R, double* Z, double* rz);
     double dot_at(const double* a, const double* b, double* part);  // partials in part

@@ -777,34 +777,44 @@ __device__ __forceinline__ double folded_sum(const double* __restrict__ part, in
     return total;
 }
 
-// the loop test of iteration k - 1 (PCGS.c:224) on its |R|^2, reported to the host
-__device__ __forceinline__ void loop_test(double* scal, int k, double r2, double r0, double tol, int relres,
-                                          int max_iter, int slot_r, int slot_it, int slot_stop, double* status) {
+// pcg's loop test (PCGS.c:224) on an iteration's |R|^2, reported to the host
+// (one thread); nothing once it has stopped
+__device__ __forceinline__ void loop_test(double* scal, double r2, double r0, double tol, bool relres, double max_iter,
+                                          int slot_r, int slot_it, int slot_stop, double* status) {
+    if (scal[slot_stop] != 0.0) return;
     const double r = sqrt(r2), crit = relres ? r : r / r0;
-    const bool was = scal[slot_stop] != 0.0;
-    const bool stop = was || !(crit > tol) || k >= max_iter;
+    const double k = scal[slot_it] + 1.0;
+    const bool stop = !(crit > tol) || k >= max_iter;
     scal[slot_r] = r;
-    if (!was) scal[slot_it] = (double)k;
+    scal[slot_it] = k;
     if (stop) scal[slot_stop] = 1.0;
-    double* h = status + 4 * (k % 4);
+    double* h = status + 4 * ((int)k % 4);
     h[1] = r;
     h[2] = stop ? 1.0 : 0.0;
-    h[3] = scal[slot_it];
+    h[3] = k;
     __threadfence_system();
-    __hip_atomic_store(h, (double)k, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(h, k, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+__global__ void k_loop_start(double* scal, double a, int ia, double b, int ib, double c, int ic, double d, int id,
+                             int z0, int z1, int z2) {
+    scal[ia] = a;
+    scal[ib] = b;
+    scal[ic] = c;
+    scal[id] = d;
+    scal[z0] = scal[z1] = scal[z2] = 0.0;
 }
 
 template <typename XT>
-__global__ __launch_bounds__(TPB) void k_precon_out_stop(int n, int k, const XT* __restrict__ xs,
+__global__ __launch_bounds__(TPB) void k_precon_out_stop(int n, const XT* __restrict__ xs,
                                                          double* __restrict__ Z, const double* __restrict__ R,
                                                          const uint32_t* __restrict__ isb,
                                                          const double* __restrict__ isa, double* __restrict__ scal,
-                                                         const double* __restrict__ rr, int nrr, double tol,
-                                                         int relres, int max_iter, double* status,
+                                                         const double* __restrict__ rr, int nrr, double* status,
                                                          double* __restrict__ rz, double* __restrict__ zz) {
     const double r2 = folded_sum(rr, nrr, scal[S_AMG0]);
     if (blockIdx.x == 0 && threadIdx.x == 0)
-        loop_test(scal, k, r2, scal[S_R0], tol, relres, max_iter, S_R, S_IT, S_STOP, status);
+        loop_test(scal, r2, scal[S_R0], scal[S_TOL], scal[S_RELRES] != 0.0, scal[S_MAXIT], S_R, S_IT, S_STOP, status);
     const bool restore = r2 == 0.0;
     double s = 0.0, q = 0.0;
     for (int i = blockIdx.x * TPB + threadIdx.x; i < n; i += gridDim.x * TPB) {
@@ -825,19 +835,19 @@ __global__ __launch_bounds__(TPB) void k_precon_out_stop(int n, int k, const XT*
     const double t = block_sum(s), u = block_sum(q);
     if (threadIdx.x == 0) {
         rz[blockIdx.x] = t;
-        zz[blockIdx.x] = u;
+        if (scal[S_DONE] == 0.0) zz[blockIdx.x] = u;
     }
 }
 
-__global__ __launch_bounds__(TPB) void k_pcg_direction(int n, int k, double* __restrict__ P,
+__global__ __launch_bounds__(TPB) void k_pcg_direction(int n, int first, double* __restrict__ P,
                                                        const double* __restrict__ Z, double* __restrict__ scal,
                                                        const double* __restrict__ rz, int nrz) {
-    const double s = folded_sum(rz, nrz, scal[S_S + k % 2]);
-    if (blockIdx.x == 0 && threadIdx.x == 0) scal[S_S + k % 2] = s;
-    if (k == 0) {
+    const double s = folded_sum(rz, nrz, 0.0);
+    if (blockIdx.x == 0 && threadIdx.x == 0) scal[S_RZ] = s;  // for the update
+    if (first) {
         for (int i = blockIdx.x * TPB + threadIdx.x; i < n; i += gridDim.x * TPB) P[i] = Z[i];
     } else {
-        const double b = s / scal[S_S + (k + 1) % 2];
+        const double b = s / scal[S_S];
         for (int i = blockIdx.x * TPB + threadIdx.x; i < n; i += gridDim.x * TPB) {
             const double p = P[i] * b;
             P[i] = p + 1 * Z[i];
@@ -846,14 +856,19 @@ __global__ __launch_bounds__(TPB) void k_pcg_direction(int n, int k, double* __r
 }
 
 template <typename XT>
-__global__ __launch_bounds__(TPB) void k_pcg_update(int n, int k, double* __restrict__ X, double* __restrict__ R,
+__global__ __launch_bounds__(TPB) void k_pcg_update(int n, double* __restrict__ X, double* __restrict__ R,
                                                     const double* __restrict__ P, const double* __restrict__ Q,
-                                                    const double* __restrict__ scal, const double* __restrict__ pq,
-                                                    int npq, double* __restrict__ rr, XT* __restrict__ ff,
+                                                    double* __restrict__ scal, const double* __restrict__ pq, int npq,
+                                                    double* __restrict__ rr, XT* __restrict__ ff,
                                                     XT* __restrict__ xf, const uint32_t* __restrict__ isb,
                                                     const double* __restrict__ isa) {
-    if (scal[S_STOP] != 0.0) return;
-    const double a = scal[S_S + k % 2] / folded_sum(pq, npq, scal[S_PQ]);
+    if (scal[S_STOP] != 0.0) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) scal[S_DONE] = 1.0;
+        return;
+    }
+    const double rzs = scal[S_RZ];
+    const double a = rzs / folded_sum(pq, npq, scal[S_PQ]);
+    if (blockIdx.x == 0 && threadIdx.x == 0) scal[S_S] = rzs;  // for the next direction
     const double na = -a;
     double s = 0.0;
     for (int i = blockIdx.x * TPB + threadIdx.x; i < n; i += gridDim.x * TPB) {
@@ -1707,29 +1722,33 @@ __global__ void k_tri_gather(int n, const int* __restrict__ map, const double* _
         val[q] = map[q] >= 0 ? v[map[q]] : 0.0;
 }
 
-__global__ __launch_bounds__(TPB) void k_ipcg_p(int n, int k, double* __restrict__ P, const double* __restrict__ Z,
+__global__ __launch_bounds__(TPB) void k_ipcg_p(int n, int first, double* __restrict__ P, const double* __restrict__ Z,
                                                 double* __restrict__ scal, const double* __restrict__ rz, int nrz,
-                                                const double* __restrict__ rr, int nrr, double r0, double tol,
-                                                int relres, int max_iter, double* status) {
-    const double s = folded_sum(rz, nrz, scal[IS_S0 + k % 2]);
-    const double b = k > 0 ? s / scal[IS_S0 + (k + 1) % 2] : 0.0;
-    if (blockIdx.x == 0) {
-        const double r2 = k > 0 ? folded_sum(rr, nrr, scal[IS_RR]) : 0.0;
-        if (threadIdx.x == 0) {
-            scal[IS_S0 + k % 2] = s;
-            if (k > 0) loop_test(scal, k, r2, r0, tol, relres, max_iter, IS_R, IS_IT, IS_STOP, status);
-        }
+                                                const double* __restrict__ rr, int nrr, double* status) {
+    const double s = folded_sum(rz, nrz, scal[IS_RZ]);
+    if (nrz > 0 && blockIdx.x == 0 && threadIdx.x == 0) scal[IS_RZ] = s;  // for the update
+    if (first) {
+        for (int i = blockIdx.x * TPB + threadIdx.x; i < n; i += gridDim.x * TPB) P[i] = Z[i];
+        return;
     }
-    for (int i = blockIdx.x * TPB + threadIdx.x; i < n; i += gridDim.x * TPB)
-        P[i] = k > 0 ? b * P[i] + Z[i] : Z[i];
+    const double b = s / scal[IS_S];
+    if (blockIdx.x == 0) {
+        const double r2 = folded_sum(rr, nrr, scal[IS_RR]);
+        if (threadIdx.x == 0)
+            loop_test(scal, r2, scal[IS_R0], scal[IS_TOL], scal[IS_RELRES] != 0.0, scal[IS_MAXIT], IS_R, IS_IT,
+                      IS_STOP, status);
+    }
+    for (int i = blockIdx.x * TPB + threadIdx.x; i < n; i += gridDim.x * TPB) P[i] = b * P[i] + Z[i];
 }
 
-__global__ __launch_bounds__(TPB) void k_ipcg_xr(int n, int k, double* __restrict__ X, double* __restrict__ R,
+__global__ __launch_bounds__(TPB) void k_ipcg_xr(int n, double* __restrict__ X, double* __restrict__ R,
                                                  const double* __restrict__ P, const double* __restrict__ Q,
-                                                 const double* __restrict__ scal, const double* __restrict__ pq,
-                                                 int npq, double* __restrict__ rr) {
+                                                 double* __restrict__ scal, const double* __restrict__ pq, int npq,
+                                                 double* __restrict__ rr) {
     if (scal[IS_STOP] != 0.0) return;
-    const double a = scal[IS_S0 + k % 2] / folded_sum(pq, npq, scal[IS_PQ]);
+    const double rzs = scal[IS_RZ];
+    const double a = rzs / folded_sum(pq, npq, scal[IS_PQ]);
+    if (blockIdx.x == 0 && threadIdx.x == 0) scal[IS_S] = rzs;  // for the next direction
     double s = 0.0;
     for (int i = blockIdx.x * TPB + threadIdx.x; i < n; i += gridDim.x * TPB) {
         X[i] += a * P[i];
@@ -2903,38 +2922,46 @@ int pcg_xr(hipStream_t st, int n, double* X, double* R, const double* P, const d
     return g;
 }
 
+void pcg_start(hipStream_t st, double* scal, double tol, int relres, int max_iter) {
+    hipLaunchKernelGGL(k_loop_start, dim3(1), dim3(1), 0, st, scal, tol, (int)S_TOL, (double)relres, (int)S_RELRES,
+                       (double)max_iter, (int)S_MAXIT, 0.0, (int)S_STOP, (int)S_STOP, (int)S_IT, (int)S_DONE);
+}
+
+void ipcg_start(hipStream_t st, double* scal, double r0, double tol, int relres, int max_iter) {
+    hipLaunchKernelGGL(k_loop_start, dim3(1), dim3(1), 0, st, scal, tol, (int)IS_TOL, (double)relres, (int)IS_RELRES,
+                       (double)max_iter, (int)IS_MAXIT, r0, (int)IS_R0, (int)IS_STOP, (int)IS_IT, (int)IS_IT);
+}
+
 template <typename XT>
-int precon_out_stop(hipStream_t st, int n, int k, const XT* xs, double* Z, const double* R, const uint32_t* isb,
-                    const double* isa, double* scal, const double* rr, int nrr, double tol, int relres, int max_iter,
-                    double* status, double* rz, double* zz) {
+int precon_out_stop(hipStream_t st, int n, const XT* xs, double* Z, const double* R, const uint32_t* isb,
+                    const double* isa, double* scal, const double* rr, int nrr, double* status, double* rz,
+                    double* zz) {
     const int g = grid_for(n, 1024);
-    hipLaunchKernelGGL((k_precon_out_stop<XT>), dim3(g), dim3(TPB), 0, st, n, k, xs, Z, R, isb, isa, scal, rr, nrr,
-                       tol, relres, max_iter, status, rz, zz);
+    hipLaunchKernelGGL((k_precon_out_stop<XT>), dim3(g), dim3(TPB), 0, st, n, xs, Z, R, isb, isa, scal, rr, nrr, status,
+                       rz, zz);
     return g;
 }
-template int precon_out_stop<double>(hipStream_t, int, int, const double*, double*, const double*, const uint32_t*,
-                                     const double*, double*, const double*, int, double, int, int, double*, double*,
-                                     double*);
-template int precon_out_stop<float>(hipStream_t, int, int, const float*, double*, const double*, const uint32_t*,
-                                    const double*, double*, const double*, int, double, int, int, double*, double*,
-                                     double*);
+template int precon_out_stop<double>(hipStream_t, int, const double*, double*, const double*, const uint32_t*,
+                                     const double*, double*, const double*, int, double*, double*, double*);
+template int precon_out_stop<float>(hipStream_t, int, const float*, double*, const double*, const uint32_t*,
+                                    const double*, double*, const double*, int, double*, double*, double*);
 
-void pcg_direction(hipStream_t st, int n, int k, double* P, const double* Z, double* scal, const double* rz, int nrz) {
-    hipLaunchKernelGGL(k_pcg_direction, dim3(grid_for(n, 2048)), dim3(TPB), 0, st, n, k, P, Z, scal, rz, nrz);
+void pcg_direction(hipStream_t st, int n, int first, double* P, const double* Z, double* scal, const double* rz,
+                   int nrz) {
+    hipLaunchKernelGGL(k_pcg_direction, dim3(grid_for(n, 2048)), dim3(TPB), 0, st, n, first, P, Z, scal, rz, nrz);
 }
 
 template <typename XT>
-int pcg_update(hipStream_t st, int n, int k, double* X, double* R, const double* P, const double* Q,
-               const double* scal, const double* pq, int npq, double* rr, XT* ff, XT* xf, const uint32_t* isb,
-               const double* isa) {
+int pcg_update(hipStream_t st, int n, double* X, double* R, const double* P, const double* Q, double* scal,
+               const double* pq, int npq, double* rr, XT* ff, XT* xf, const uint32_t* isb, const double* isa) {
     const int g = grid_for(n, 1024);
-    hipLaunchKernelGGL((k_pcg_update<XT>), dim3(g), dim3(TPB), 0, st, n, k, X, R, P, Q, scal, pq, npq, rr, ff, xf, isb,
+    hipLaunchKernelGGL((k_pcg_update<XT>), dim3(g), dim3(TPB), 0, st, n, X, R, P, Q, scal, pq, npq, rr, ff, xf, isb,
                        isa);
     return g;
 }
-template int pcg_update<double>(hipStream_t, int, int, double*, double*, const double*, const double*, const double*,
+template int pcg_update<double>(hipStream_t, int, double*, double*, const double*, const double*, double*,
                                 const double*, int, double*, double*, double*, const uint32_t*, const double*);
-template int pcg_update<float>(hipStream_t, int, int, double*, double*, const double*, const double*, const double*,
+template int pcg_update<float>(hipStream_t, int, double*, double*, const double*, const double*, double*,
                                const double*, int, double*, float*, float*, const uint32_t*, const double*);
 
 void axpy_s(hipStream_t st, int n, double* x, const double* y, const double* scal, int slot_a, int slot_b,
@@ -3191,16 +3218,16 @@ void tri_values(hipStream_t st, int n, const int* map, const double* v, double* 
     if (n > 0) hipLaunchKernelGGL(k_tri_gather, dim3(grid_for(n)), dim3(TPB), 0, st, n, map, v, val);
 }
 
-void ipcg_p(hipStream_t st, int n, int k, double* P, const double* Z, double* scal, const double* rz, int nrz,
-            const double* rr, int nrr, double r0, double tol, int relres, int max_iter, double* status) {
-    hipLaunchKernelGGL(k_ipcg_p, dim3(grid_for(n, 1024)), dim3(TPB), 0, st, n, k, P, Z, scal, rz, nrz, rr, nrr, r0,
-                       tol, relres, max_iter, status);
+void ipcg_p(hipStream_t st, int n, int first, double* P, const double* Z, double* scal, const double* rz, int nrz,
+            const double* rr, int nrr, double* status) {
+    hipLaunchKernelGGL(k_ipcg_p, dim3(grid_for(n, 1024)), dim3(TPB), 0, st, n, first, P, Z, scal, rz, nrz, rr, nrr,
+                       status);
 }
 
-int ipcg_xr(hipStream_t st, int n, int k, double* X, double* R, const double* P, const double* Q, const double* scal,
+int ipcg_xr(hipStream_t st, int n, double* X, double* R, const double* P, const double* Q, double* scal,
             const double* pq, int npq, double* rr) {
     const int g = grid_for(n, 1024);
-    hipLaunchKernelGGL(k_ipcg_xr, dim3(g), dim3(TPB), 0, st, n, k, X, R, P, Q, scal, pq, npq, rr);
+    hipLaunchKernelGGL(k_ipcg_xr, dim3(g), dim3(TPB), 0, st, n, X, R, P, Q, scal, pq, npq, rr);
     return g;
 }
 

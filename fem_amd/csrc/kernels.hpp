@@ -54,7 +54,12 @@ enum {
     S_AMG0 = 12,  // sum of squares of the preconditioner's right-hand side
     S_STOP = 13,  // pcg's device-side stop flag (nonzero: converged, NaN or out of iterations)
     S_IT = 14,    // pcg iterations completed on the device
-    S_COUNT = 16
+    S_TOL = 15,   // the loop test's tolerance, kind (S_RELRES) and iteration limit
+    S_RELRES = 16,
+    S_MAXIT = 17,
+    S_DONE = 18,  // an iteration after the one that stopped has begun
+    S_RZ = 19,    // R.Z of the iteration in progress (S_S: of the last one)
+    S_COUNT = 20
 };
 
 // Sliced copy of a matrix, the form the row kernels stream where its padding
@@ -237,24 +242,30 @@ void pcg_p(hipStream_t st, int n, double* P, const double* Z, const double* scal
 // The same iteration without launches for its sums (Solver::pcg_dev with a
 // preconditioner of one V-cycle): np partials (at most PCG_PARTS) are added by
 // every workgroup that needs them, in finalize's order (the same bits); np =
-// 0: already in scal.  S_k is scal[S_S + k % 2].
+// 0: already in scal.  Nothing depends on the iteration's number, so that one
+// captured iteration serves all.
 constexpr int PCG_PARTS = 2048;
-// precon_out of iteration k >= 1, whose zero test and loop test are on |R|^2
-// of iteration k - 1: the test (finalize_stop's) sets scal[S_STOP] and reports
-// {k, |R|, stop, iterations} to the host's status[4 (k % 4) ...]; rz, zz: the
-// partials of R.Z and Z.Z
+// precon_out of an iteration after the first, whose zero test and loop test
+// are on the previous iteration's |R|^2: the test (finalize_stop's, with
+// scal[S_TOL], S_RELRES, S_MAXIT) counts it in scal[S_IT] = k, sets
+// scal[S_STOP] and reports {k, |R|, stop, iterations} to the host's
+// status[4 (k % 4) ...]; rz, zz: the partials of R.Z and Z.Z (zz: kept from
+// the iteration that found the stop)
+// scal's S_STOP, S_IT and S_DONE cleared, the loop test's values set
+void pcg_start(hipStream_t st, double* scal, double tol, int relres, int max_iter);
 template <typename XT>
-int precon_out_stop(hipStream_t st, int n, int k, const XT* xs, double* Z, const double* R, const uint32_t* isb,
-                    const double* isa, double* scal, const double* rr, int nrr, double tol, int relres, int max_iter,
-                    double* status, double* rz, double* zz);
-void pcg_direction(hipStream_t st, int n, int k, double* P, const double* Z, double* scal, const double* rz, int nrz);
-// k_pcg_xr's updates and |R|^2 partials, and the next preconditioner's entry
-// on the new R: ff = (XT) R when given, xf = the initial guess (0; R_i / isa_i
-// on the rows marked in isb) when given
+int precon_out_stop(hipStream_t st, int n, const XT* xs, double* Z, const double* R, const uint32_t* isb,
+                    const double* isa, double* scal, const double* rr, int nrr, double* status, double* rz, double* zz);
+// scal[S_RZ] = R.Z, P = Z (first) or b P + Z, b = R.Z / scal[S_S]
+void pcg_direction(hipStream_t st, int n, int first, double* P, const double* Z, double* scal, const double* rz,
+                   int nrz);
+// k_pcg_xr's updates and |R|^2 partials, scal[S_S] = scal[S_RZ], and the next
+// preconditioner's entry on the new R: ff = (XT) R when given, xf = the initial
+// guess (0; R_i / isa_i on the rows marked in isb) when given; nothing once
+// scal[S_STOP] is set
 template <typename XT>
-int pcg_update(hipStream_t st, int n, int k, double* X, double* R, const double* P, const double* Q,
-               const double* scal, const double* pq, int npq, double* rr, XT* ff, XT* xf, const uint32_t* isb,
-               const double* isa);
+int pcg_update(hipStream_t st, int n, double* X, double* R, const double* P, const double* Q, double* scal,
+               const double* pq, int npq, double* rr, XT* ff, XT* xf, const uint32_t* isb, const double* isa);
 // (skips every update once scal[S_STOP] is set)
 int pcg_xr(hipStream_t st, int n, double* X, double* R, const double* P, const double* Q, const double* scal,
            double* part);
@@ -404,16 +415,17 @@ void tri_level(hipStream_t st, const TriLevel& L, const double* in, double* out,
 void tri_values(hipStream_t st, int n, const int* map, const double* v, double* val);
 
 // ILU-pcg on the device (IluSystem::pcg_core), its sums as in pcg_direction
-enum { IS_S0 = 0, IS_S1 = 1, IS_PQ = 2, IS_RR = 3, IS_STOP = 4, IS_IT = 5, IS_R = 6, IS_COUNT = 8 };
-// iteration k's direction P = Z (k = 0) or b P + Z, b = S_k / S_{k-1}, with
-// S_k = R.Z from its partials; before it, for k > 0, the loop test of
-// iteration k - 1 on |R|^2 from its partials: scal[IS_STOP] and, for the host,
-// status[4 (k % 4) ...] = {k, |R|, stop}
-void ipcg_p(hipStream_t st, int n, int k, double* P, const double* Z, double* scal, const double* rz, int nrz,
-            const double* rr, int nrr, double r0, double tol, int relres, int max_iter, double* status);
-// X += a P, R -= a Q, a = S_k / P.Q, and the partials of |R|^2; nothing once
-// scal[IS_STOP] is set.  Returns the partials' number.
-int ipcg_xr(hipStream_t st, int n, int k, double* X, double* R, const double* P, const double* Q, const double* scal,
+enum { IS_S = 0, IS_RZ = 1, IS_PQ = 2, IS_RR = 3, IS_STOP = 4, IS_IT = 5, IS_R = 6, IS_R0 = 7, IS_TOL = 8,
+       IS_RELRES = 9, IS_MAXIT = 10, IS_COUNT = 12 };
+// scal's IS_STOP and IS_IT cleared, the loop test's values set
+void ipcg_start(hipStream_t st, double* scal, double r0, double tol, int relres, int max_iter);
+// an iteration's direction P = Z (first) or b P + Z; before it, but for the
+// first, the loop test on the previous iteration's |R|^2 as in precon_out_stop
+void ipcg_p(hipStream_t st, int n, int first, double* P, const double* Z, double* scal, const double* rz, int nrz,
+            const double* rr, int nrr, double* status);
+// X += a P, R -= a Q, a = R.Z / P.Q (scal[IS_RZ], set by ipcg_p), scal[IS_S] =
+// R.Z and the partials of |R|^2; nothing once scal[IS_STOP] is set.  Returns the partials' number.
+int ipcg_xr(hipStream_t st, int n, double* X, double* R, const double* P, const double* Q, double* scal,
             const double* pq, int npq, double* rr);
 // out[r] = in[perm[r]] (inverse 0), out[perm[r]] = in[r] (inverse 1)
 void permute(hipStream_t st, int n, const int* perm, const double* in, double* out, int inverse);

@@ -204,6 +204,7 @@ IluSystem::IluSystem() {}
 
 IluSystem::~IluSystem() {
     if (stream_) (void)hipStreamSynchronize(stream_);
+    iteration_.reset();
     if (host_) (void)hipHostFree(host_);
     bufs_.reset();
     if (stream_) (void)hipStreamDestroy(stream_);
@@ -495,6 +496,8 @@ void IluSystem::upload(bool pattern_levels_in) {
     // first use included: nothing may still run on them, and no pointer to
     // them may survive
     hip_check(hipStreamSynchronize(stream_), "sync");
+    iteration_.reset();
+    vXg_ = nullptr;
     bufs_.reset(new DevBuffers());
     vbasis_ = nullptr;
     hcols_ = nullptr;
@@ -685,9 +688,10 @@ double IluSystem::dot(const double* a, const double* b) { return dot_at(a, b, pa
 double IluSystem::dot_at(const double* a, const double* b, double* part) {
     int np = dev::dot_part<double>(stream_, n_, a, b, part);
     dev::finalize(stream_, np, part, scal_, dev::IS_COUNT, 0);
-    hip_check(hipMemcpyAsync(host_, scal_ + dev::IS_COUNT, sizeof(double), hipMemcpyDeviceToHost, stream_), "d2h");
+    hip_check(hipMemcpyAsync(host_, scal_, (dev::IS_COUNT + 1) * sizeof(double), hipMemcpyDeviceToHost, stream_),
+              "d2h");
     hip_check(hipStreamSynchronize(stream_), "sync");
-    return host_[0];
+    return host_[dev::IS_COUNT];
 }
 
 void IluSystem::matvec(const double* x, double* y) {
@@ -736,32 +740,50 @@ int IluSystem::pcg_core(double* X, double* B, double tol, int max_iter, int stop
     int nrz = precon_dot(R, Z, rz), nrr = 0;
     double r0 = std::sqrt(dot_at(Z, Z, part_ + (size_t)34 * cap));
     if (r0 == 0) return 0;
-    dev::fill<double>(st, dev::IS_COUNT, scal_, 0.0);
     double* status = host_ + 16;  // four iterations' {number, |R|, stop, iterations done}
     for (int j = 0; j < 16; j++) status[j] = -1.0;
+    dev::ipcg_start(st, scal_, r0, tol, stop == LINA_STOP_RELRES, std::max(max_iter, 1));
+    double* Y = X;
     auto folded = [&](int np, const double* part, int slot) {  // few partials are summed where they are used
         if (np <= dev::PCG_PARTS) return np;
         dev::finalize(st, np, part, scal_, slot, 0);
         return 0;
     };
-    auto enqueue = [&](int k) {
-        if (k > 0) nrz = precon_dot(R, Z, rz);
-        dev::ipcg_p(st, n, k, P, Z, scal_, rz, folded(nrz, rz, dev::IS_S0 + k % 2), rr, nrr, r0, tol,
-                    stop == LINA_STOP_RELRES, std::max(max_iter, 1), status);
+    auto finish = [&](int mrz, int mrr, bool first) {
+        dev::ipcg_p(st, n, first, P, Z, scal_, rz, mrz, rr, mrr, status);
         const int m = dev::spmv<double, double>(st, dA_, P, nullptr, Q, dev::MODE_OUTER, pq, P);
-        nrr = dev::ipcg_xr(st, n, k, X, R, P, Q, scal_, pq, folded(m, pq, dev::IS_PQ), rr);
+        return dev::ipcg_xr(st, n, Y, R, P, Q, scal_, pq, folded(m, pq, dev::IS_PQ), rr);
     };
-    enqueue(0);
-    enqueue(1);
-    int i = 0;
+    auto later = [&]() { (void)finish(folded(precon_dot(R, Z, rz), rz, dev::IS_RZ), nrr, false); };
+    // long solves go on with replays of captured iterations (see Solver::pcg_dev)
+    constexpr int EAGER = 48, REPLAY = 8;
+    nrr = finish(folded(nrz, rz, dev::IS_RZ), 0, true);
+    int queued = 0;
     for (int k = 1;; k++) {
-        const double* s = wait_status(status, k, st);  // iteration k - 1's loop test
-        i = (int)s[3];
-        if (s[2] != 0.0) break;
-        enqueue(k + 1);  // its report overwrites iteration k - 3's
+        while (queued < k + (queued >= EAGER ? 2 : 0)) {
+            if (queued < EAGER) {
+                later();
+                queued++;
+                continue;
+            }
+            if (Y != vXg_ || !vXg_) {  // captured iterations work on the system's own iterate
+                if (!vXg_) vXg_ = kalloc<double>(n, *bufs_);
+                dev::copy(st, n, (const double*)X, vXg_);
+                Y = vXg_;
+            }
+            if (!iteration_.ready())
+                iteration_.capture(st, [&]() {
+                    for (int q = 0; q < REPLAY; q++) later();
+                });
+            iteration_.launch(st);
+            queued += REPLAY;
+        }
+        if (wait_status(status, k, st)) break;  // iteration k - 1's loop test
     }
+    if (Y != X) dev::copy(st, n, (const double*)Y, X);
     // every preconditioner call queued after the stop was on the final R
     double rw = std::sqrt(dot_at(Z, Z, part_ + (size_t)34 * cap));
+    const int i = (int)host_[dev::IS_IT];  // read with it
     dev::axpby(st, n, h, B, 0.0, B);
     dev::axpby(st, n, h, X, 0.0, X);
     hip_check(hipStreamSynchronize(st), "sync");

@@ -23,6 +23,7 @@
 #include <memory>
 #include <stdexcept>
 #include <string>
+#include <tuple>
 #include <type_traits>
 #include <vector>
 
@@ -52,18 +53,44 @@ void hip_check(hipError_t e, const char* what) {
     if (e != hipSuccess) throw HipError(std::string(what) + ": " + hipGetErrorString(e));
 }
 
-const double* wait_status(const double* status, int k, hipStream_t st) {
+void Captured::reset() {
+    if (exec_) (void)hipGraphExecDestroy(exec_);
+    if (graph_) (void)hipGraphDestroy(graph_);
+    exec_ = nullptr;
+    graph_ = nullptr;
+}
+
+void Captured::capture(hipStream_t st, const std::function<void()>& record) {
+    reset();
+    hip_check(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal), "begin capture");
+    try {
+        record();
+    } catch (...) {
+        hipGraph_t g = nullptr;  // the stream leaves capture whatever happened
+        (void)hipStreamEndCapture(st, &g);
+        if (g) (void)hipGraphDestroy(g);
+        throw;
+    }
+    hip_check(hipStreamEndCapture(st, &graph_), "end capture");
+    hip_check(hipGraphInstantiate(&exec_, graph_, nullptr, nullptr, 0), "instantiate");
+}
+
+void Captured::launch(hipStream_t st) const { hip_check(hipGraphLaunch(exec_, st), "graph launch"); }
+
+bool wait_status(const double* status, int k, hipStream_t st) {
     const double* s = status + 4 * (k % 4);
+    bool idle = false;
     for (long spin = 1;; spin++) {
         double seen;
         __atomic_load(s, &seen, __ATOMIC_ACQUIRE);
-        if (seen == (double)k) return s;
+        // a later iteration in the slot: k did not stop the loop
+        if (seen >= (double)k) return seen == (double)k && s[2] != 0.0;
+        if (idle) throw HipError("the loop test was not reported");
         if (spin % 4096) continue;
         const hipError_t e = hipStreamQuery(st);
         if (e == hipErrorNotReady) continue;
         hip_check(e, "loop test");
-        __atomic_load(s, &seen, __ATOMIC_ACQUIRE);
-        if (seen != (double)k) throw HipError("the loop test was not reported");
+        idle = true;  // everything queued is done: one more look
     }
 }
 
@@ -469,6 +496,7 @@ Solver::Solver() {}
 
 Solver::~Solver() {
     if (stream_) (void)hipStreamSynchronize(stream_);
+    iteration_.reset();
     if (ev0_) (void)hipEventDestroy(ev0_);
     if (ev1_) (void)hipEventDestroy(ev1_);
     for (auto& pr : evk_)
@@ -604,6 +632,7 @@ void Solver::upload() {
     // a re-upload (recompute) frees every earlier buffer, including the
     // BiCGStab work vectors allocated on first use
     hip_check(hipStreamSynchronize(stream_), "sync");
+    iteration_.reset();
     if (bufs_ && (host_stale_ || host_top_stale_)) sync_host_levels();  // values of a device recompute
     rap_.reset();  // the device products' plans belong to the patterns uploaded before
     host_stale_ = false;
@@ -814,7 +843,7 @@ void Solver::upload() {
     kB_ = dalloc<double>(n, B);
     // block partials: one per SpMV block (any matrix) or per reduction block
     int np = std::max(4096, maxblk + 16);
-    part_ = dalloc<double>(np + 4 * dev::DOT_PART_MAX, B);  // and four dots' partials beside a product's
+    part_ = dalloc<double>(np + 3 * dev::DOT_PART_MAX, B);  // and three dots' partials beside a product's
     part_cap_ = np;
     scal_ = dalloc<double>(dev::S_COUNT, B);
     dev::fill(st, dev::S_COUNT, scal_, 0.0);
@@ -1686,6 +1715,16 @@ int Solver::precon(const double* R, double* Z, const double* w, int* np) {
     return it;
 }
 
+// whether two parameter blocks make the same V-cycle of one hierarchy
+static bool same_cycle(const lina_amg_params& a, const lina_amg_params& b) {
+    auto key = [](const lina_amg_params& p) {
+        return std::make_tuple(p.dof, p.depth, p.smoothing_iterations, p.aggr_smoothing_iterations, p.coarsening,
+                               p.smoother, p.omega, p.amg_eps, p.amg_max_iter, p.zero_init, p.precision,
+                               p.coarse_smoother, p.coarse_sweeps, p.cycle, p.skip_levels);
+    };
+    return key(a) == key(b);
+}
+
 // pcg (PCGS.c:163-233) on device vectors X, B (length n).  The loop test is
 // evaluated on the device; with a preconditioner that needs no host round
 // trip, iteration k+1 is queued before the host sees iteration k's test, and
@@ -1695,8 +1734,7 @@ int Solver::precon(const double* R, double* Z, const double* w, int* np) {
 // an iteration around its V-cycle and the product: the exit kernel with the
 // loop test of the previous iteration, the direction and the update, each
 // adding up the partial sums it needs; the first preconditioned residual is
-// iteration 0's, and the last one that of the iteration queued at the stop.
-// Other preconditioners keep a launch per sum.
+// iteration 0's.  Other preconditioners keep a launch per sum.
 int Solver::pcg_dev(double* X, double* B, double tol, int max_iter, int stop, lina_stats* stats) {
     hipStream_t st = stream_;
     const int n = n_;
@@ -1704,7 +1742,7 @@ int Solver::pcg_dev(double* X, double* B, double tol, int max_iter, int stop, li
     vcycles_ = 0;
     precon_calls_ = 0;
     hip_check(hipEventRecord(ev0_, st), "event");
-    dev::fill<double>(st, 2, scal_ + dev::S_STOP, 0.0);  // S_STOP, S_IT
+    dev::pcg_start(st, scal_, tol, stop == LINA_STOP_RELRES, std::max(max_iter, 1));
     // h = |B| (h==0 -> 1), B and X scaled by 1/h
     int np = dev::dot_part<double>(st, n, B, B, part_);
     dev::finalize(st, np, part_, scal_, dev::S_H, 1);
@@ -1770,59 +1808,88 @@ int Solver::pcg_dev(double* X, double* B, double tol, int max_iter, int stop, li
         ksum += kms;
         kcount++;
     };
-    double r = 0.0;
+    double r = 0.0, rw = 0.0;
     int i = 0;
     if (fused) {
-        double *pq = part_, *rz = part_ + part_cap_, *rr = rz + dev::DOT_PART_MAX;
-        double* zz[2] = {rr + dev::DOT_PART_MAX, rr + 2 * dev::DOT_PART_MAX};
+        double *pq = part_, *rz = part_ + part_cap_, *rr = rz + dev::DOT_PART_MAX, *zz = rr + dev::DOT_PART_MAX;
         double* status = host_ring_;
         for (int j = 0; j < 16; j++) status[j] = -1.0;
-        auto folded = [&](int m, const double* part, int slot) {  // many partials keep their launch
-            if (m <= dev::PCG_PARTS) return m;
-            dev::finalize(st, m, part, scal_, slot, 0);
-            return 0;
-        };
-        int nrr = 0, nzz = 0;
-        auto enqueue = [&](int k) {
-            int nrz;
-            if (k == 0) {
-                nrz = dev::dot_part<double>(st, n, R, Z, rz);
-            } else if (fp64) {
-                vcycle<double>((int)L_.size() - 1, R, Z, niso_ == 0 ? X_ZERO : X_GUESS);
-                nrz = dev::precon_out_stop<double>(st, n, k, nullptr, Z, R, isb_, isa_, scal_, rr, nrr, tol, relres,
-                                                   cap, status, rz, zz[k % 2]);
-            } else {
-                vcycle<float>((int)L_.size() - 1, top.ff, top.xf, niso_ == 0 ? X_ZERO : X_GUESS);
-                nrz = dev::precon_out_stop<float>(st, n, k, top.xf, Z, R, isb_, isa_, scal_, rr, nrr, tol, relres,
-                                                  cap, status, rz, zz[k % 2]);
+        double* Y = X;
+        const int lt = (int)L_.size() - 1, xinit = niso_ == 0 ? X_ZERO : X_GUESS;
+        const int ndot = std::min(std::max((n + 255) / 256, 1), dev::DOT_PART_MAX);  // an elementwise kernel's partials
+        auto finish = [&](int k, int nrz, bool first) {
+            dev::pcg_direction(st, n, first, P, Z, scal_, rz, nrz);
+            int m = product(k, pq);
+            if (m > dev::PCG_PARTS) {  // many partials keep their launch
+                dev::finalize(st, m, pq, scal_, dev::S_PQ, 0);
+                m = 0;
             }
-            nzz = nrz;
-            dev::pcg_direction(st, n, k, P, Z, scal_, rz, nrz);
-            const int m = product(k, pq);
-            const int mf = folded(m, pq, dev::S_PQ);
-            if (fp64)
-                nrr = dev::pcg_update<double>(st, n, k, X, R, P, Q, scal_, pq, mf, rr, nullptr,
-                                              niso_ == 0 ? nullptr : Z, isb_, isa_);
-            else
-                nrr = dev::pcg_update<float>(st, n, k, X, R, P, Q, scal_, pq, mf, rr, top.ff,
-                                             niso_ == 0 ? nullptr : top.xf, isb_, isa_);
+            const int nrr = fp64 ? dev::pcg_update<double>(st, n, Y, R, P, Q, scal_, pq, m, rr, nullptr,
+                                                           niso_ == 0 ? nullptr : Z, isb_, isa_)
+                                 : dev::pcg_update<float>(st, n, Y, R, P, Q, scal_, pq, m, rr, top.ff,
+                                                          niso_ == 0 ? nullptr : top.xf, isb_, isa_);
+            if (nrr != ndot) throw std::logic_error("pcg: unexpected partials");
         };
-        enqueue(0);
-        enqueue(1);
-        int k = 1;
-        for (;; k++) {
-            const double* s = wait_status(status, k, st);  // iteration k - 1's loop test
-            if (timed && sampled(k - 1) && (int)s[3] == k) sample(k - 1);
-            r = s[1];
-            i = (int)s[3];
-            if (s[2] != 0.0) break;
-            enqueue(k + 1);
+        auto later = [&](int k) {
+            int nrz;
+            if (fp64) {
+                vcycle<double>(lt, R, Z, xinit);
+                nrz = dev::precon_out_stop<double>(st, n, nullptr, Z, R, isb_, isa_, scal_, rr, ndot, status, rz, zz);
+            } else {
+                vcycle<float>(lt, top.ff, top.xf, xinit);
+                nrz = dev::precon_out_stop<float>(st, n, top.xf, Z, R, isb_, isa_, scal_, rr, ndot, status, rz, zz);
+            }
+            finish(k, nrz, false);
+        };
+        // Long solves go on with replays of REPLAY captured iterations: the
+        // host takes 2.7 us a launch (3.9 with the sliced kernels' arguments),
+        // the GPU 1.8 a node and about 20 us a graph, so that replays of one
+        // iteration lose (257^2 Poisson, 37 iterations: 3.58 -> 3.88 ms) and
+        // those of several pay once a solve is long enough for the capture and
+        // for the iterations replayed past its end.  Not under kernel timing,
+        // whose events are the launch's own, nor for another operator's matrix.
+        constexpr int EAGER = 48, REPLAY = 4;
+        const bool replay = !op_ && !ktime_;
+        finish(0, dev::dot_part<double>(st, n, R, Z, rz), true);
+        int queued = 0;
+        for (int k = 1;; k++) {
+            // the test of iteration k - 1 comes in the middle of iteration k:
+            // what follows can be queued then, but for a graph's latency
+            while (queued < k + (replay && queued >= EAGER ? 2 : 0)) {
+                if (!replay || queued < EAGER) {
+                    later(++queued);
+                    continue;
+                }
+                if (Y != kX_) {  // captured iterations work on the solver's own iterate
+                    dev::copy(st, n, (const double*)Y, kX_);
+                    Y = kX_;
+                }
+                if (!(iteration_.ready() && same_cycle(iteration_prm_, prm_))) {
+                    iteration_.capture(st, [&]() {
+                        for (int q = 0; q < REPLAY; q++) later(0);
+                    });
+                    iteration_prm_ = prm_;
+                }
+                iteration_.launch(st);
+                queued += REPLAY;
+            }
+            const bool stopped = wait_status(status, k, st);  // iteration k - 1's loop test
+            if (timed && sampled(k - 1)) sample(k - 1);
+            if (stopped) break;
         }
-        // iteration k preconditioned the final R (one queued after it started
-        // from another guess); the reference's calls: one before the loop,
-        // one an iteration, one after it
+        // M^-1 of the final R and its norm come from the iteration that found
+        // the stop; the reference's calls: one before the loop, one an
+        // iteration, one after it
+        dev::finalize(st, ndot, zz, scal_, dev::S_T1, 1);
+        if (X != Y) dev::copy(st, n, (const double*)Y, X);
+        double* last = host_ring_ + 20;  // S_R ... S_IT
+        hip_check(hipMemcpyAsync(last, scal_ + dev::S_R, (dev::S_IT - dev::S_R + 1) * sizeof(double),
+                                 hipMemcpyDeviceToHost, st), "d2h");
+        hip_check(hipStreamSynchronize(st), "sync");
+        r = last[0];
+        rw = last[dev::S_T1 - dev::S_R];
+        i = (int)last[dev::S_IT - dev::S_R];
         precon_calls_ = vcycles_ = i + 2;
-        dev::finalize(st, nzz, zz[k % 2], scal_, dev::S_T1, 1);
     } else {
         // one iteration: Z = M^-1 R with R.Z, P, Q = A P with P.Q, X and R
         // with |R| and the stop test; its state (S_R..S_IT) copied to ring slot k % 2
@@ -1859,9 +1926,9 @@ int Solver::pcg_dev(double* X, double* B, double tol, int max_iter, int stop, li
         precon_calls_ -= enq - i;
         precon(R, W, W, &np);
         dev::finalize(st, np, part_, scal_, dev::S_T1, 1);
+        rw = read_scalar(dev::S_T1);
     }
     const double relres_out = r;
-    double rw = read_scalar(dev::S_T1);
     dev::scale_by(st, n, B, scal_, dev::S_H, 0);
     dev::scale_by(st, n, X, scal_, dev::S_H, 0);
     hip_check(hipEventRecord(ev1_, st), "event");

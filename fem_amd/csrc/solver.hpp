@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <functional>
 #include <memory>
 #include <stdexcept>
 #include <string>
@@ -28,10 +29,30 @@ struct NumericError : std::runtime_error {
 void hip_check(hipError_t e, const char* what);
 const char* last_error();
 
-// The report of iteration number k of a device-side loop: waits until
-// status[4 (k % 4)] (pinned, written by a kernel on st) reads k; returns that
-// slot.  Throws when st fails or runs out of work without the report.
-const double* wait_status(const double* status, int k, hipStream_t st);
+// Waits for the report of iteration number k of a device-side loop (its kernels
+// on st write status[4 (k % 4) ...] in pinned memory, see dev::loop_test):
+// whether it stopped the loop.  Throws when st fails or runs out of work
+// without the report.
+bool wait_status(const double* status, int k, hipStream_t st);
+
+// A captured piece of a stream's work that is replayed while nothing it was
+// captured from changes (the owner resets it then).
+class Captured {
+  public:
+    Captured() = default;
+    Captured(const Captured&) = delete;
+    Captured& operator=(const Captured&) = delete;
+    ~Captured() { reset(); }
+    void reset();
+    bool ready() const { return exec_ != nullptr; }
+    // record(): enqueues the work on st, without a synchronisation
+    void capture(hipStream_t st, const std::function<void()>& record);
+    void launch(hipStream_t st) const;
+
+  private:
+    hipGraph_t graph_ = nullptr;
+    hipGraphExec_t exec_ = nullptr;
+};
 
 struct DevBuffers {
     std::vector<void*> ptrs;
@@ -349,6 +370,8 @@ class Solver {
     int part_cap_ = 0;
     hipEvent_t evk_[2][2] = {{nullptr, nullptr}, {nullptr, nullptr}};  // outer SpMV timing, per ring slot
     hipEvent_t evr_[2] = {nullptr, nullptr};                            // pcg iteration done, per ring slot
+    Captured iteration_;          // some pcg iterations with iteration_prm_, on this upload's buffers
+    lina_amg_params iteration_prm_{};
     double* host_ring_ = nullptr;                                       // pinned: 2 x S_COUNT scalars
     double *bS_ = nullptr, *bPS_ = nullptr, *bPP_ = nullptr, *bAPP_ = nullptr, *bAPS_ = nullptr, *bR_ = nullptr,
            *bR0_ = nullptr, *bP_ = nullptr;
