@@ -56,17 +56,36 @@ class Captured {
 
 struct DevBuffers {
     std::vector<void*> ptrs;
+    char* chunk = nullptr;  // the rest of the last shared allocation of small arrays
+    size_t left = 0;
     ~DevBuffers();
 };
 
-// device arrays owned by a DevBuffers (freed with it)
+// device arrays owned by a DevBuffers (freed with it).  Arrays up to 64 KB
+// share allocations of 1 MB, at multiples of 256 bytes: a small hierarchy has a
+// few hundred, and a hipMalloc costs more than their upload.
 template <typename T>
 T* dalloc(size_t n, DevBuffers& owner) {
     if (n == 0) n = 1;
-    void* p = nullptr;
-    hip_check(hipMalloc(&p, n * sizeof(T)), "hipMalloc");
-    owner.ptrs.push_back(p);
-    return (T*)p;
+    const size_t bytes = n * sizeof(T), shared = 1 << 20;
+    if (bytes > (64u << 10)) {
+        void* p = nullptr;
+        hip_check(hipMalloc(&p, bytes), "hipMalloc");
+        owner.ptrs.push_back(p);
+        return (T*)p;
+    }
+    const size_t take = (bytes + 255) / 256 * 256;
+    if (owner.left < take) {
+        void* p = nullptr;
+        hip_check(hipMalloc(&p, shared), "hipMalloc");
+        owner.ptrs.push_back(p);
+        owner.chunk = (char*)p;
+        owner.left = shared;
+    }
+    T* p = (T*)owner.chunk;
+    owner.chunk += take;
+    owner.left -= take;
+    return p;
 }
 
 template <typename T>
