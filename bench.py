@@ -759,7 +759,7 @@ def main():
         "iteration_roofline": {"mixed": res["mixed"]["iteration"]["frac"], "fp64": res["fp64"]["iteration"]["frac"],
                                "bytes": "outer SpMV + 2 dots + fused updates + per level (sweeps, residual, R, P) "
                                         "+ coarse inverse, from the actual level sizes"},
-        "spmv_fp32": {"achieved": spmv32_gbs, "avg_ms": spmv32_ms, "kernel": "k_spmv<float, float, 3, 1>"},
+        "spmv_fp32": {"achieved": spmv32_gbs, "avg_ms": spmv32_ms, "kernel": "k_sell_spmv<float, float, 3> (sliced copy)"},
         "cpu_baseline": cpu,
     }
     print(json.dumps(out))
