@@ -300,6 +300,33 @@ SlicePlan plan_slices(const Csr& A, const std::vector<int>& groups, bool free_or
     return p;
 }
 
+static bool same_rows(const SlicePlan& a, const SlicePlan& b) {
+    auto eq = [](const dev::SliceHead& x, const dev::SliceHead& y) {
+        return x.row0 == y.row0 && x.row1 == y.row1 && x.step0 == y.step0 && x.steps == y.steps;
+    };
+    return a.lt == b.lt && a.steps == b.steps && a.head.size() == b.head.size() &&
+           std::equal(a.head.begin(), a.head.end(), b.head.begin(), eq);
+}
+
+// every row in one slice whose steps hold its entries, every slice's steps in
+// the plan's
+static void validate(const Csr& A, const SlicePlan& p) {
+    if (p.head.empty()) return;
+    const int T = 1 << p.lt;
+    int row = 0;
+    size_t step = 0;
+    for (const dev::SliceHead& h : p.head) {
+        if (h.row0 != row || h.row1 < h.row0 || h.row1 > A.n || h.row1 - h.row0 > 64 / T)
+            throw std::logic_error("upload: bad slice rows");
+        if ((size_t)h.step0 != step || h.steps < 0) throw std::logic_error("upload: bad slice steps");
+        for (int i = h.row0; i < h.row1; i++)
+            if (A.rp[i + 1] - A.rp[i] > (long)h.steps * T) throw std::logic_error("upload: row longer than its slice");
+        row = h.row1;
+        step += h.steps;
+    }
+    if (row != A.n || step != p.steps) throw std::logic_error("upload: slices do not cover the matrix");
+}
+
 // steps in flight per lane: all of a short row, else the count that wastes
 // least of its last round (7 for the 7 and 14 entries of the P1 stencils:
 // 2.1M rows x 14 in FP64, 69 us with 8, 65 us with 7)
@@ -309,8 +336,8 @@ static int slice_unroll(double mean_steps) {
     return (w + 6) / 7 * 7 < (w + 7) / 8 * 8 ? 7 : 8;
 }
 
-// D.sl from the plan (D's CSR uploaded); share: the other precision's copy,
-// whose layout and codes are reused.  Large streams are loaded nontemporally:
+// D.sl from the plan (D's CSR uploaded); share: the other precision's copy of
+// the same plan (same_rows), whose heads and codes are reused.  Large streams are loaded nontemporally:
 // FP64 from 64 MB (read once per Krylov iteration; 2.1M rows x 14, 79 -> 69
 // us, 1.05M x 7, 22.0 -> 20.4 us), FP32 from 128 MB (2.1M x 14, 40 -> 37 us;
 // smaller ones stay in the last-level cache between sweeps and lose: 403k x
@@ -326,6 +353,8 @@ static void make_slices(const SlicePlan& p, dev::DMat<VT>& D, DevBuffers& B, hip
     S.steps = p.steps;
     S.unroll = slice_unroll((double)S.steps / S.ns);
     S.nt = S.steps * 64 * (sizeof(VT) + 2) >= (sizeof(VT) == 8 ? 64u << 20 : 128u << 20);
+    if (share && (share->sl.ns != S.ns || share->sl.lt != S.lt || share->sl.steps != S.steps))
+        throw std::logic_error("slices shared between different plans");
     S.v = dalloc<VT>(S.steps * 64, B);
     if (share) {
         S.head = share->sl.head;
@@ -349,15 +378,16 @@ bool slice_matrix(const Csr& A, dev::DMat<double>& D, DevBuffers& B, hipStream_t
 
 // plan: the slices (none: empty), starts_with_end: the row blocks (none:
 // empty); share: a copy of A with other values uploaded before; its row
-// pointers and column indices are reused, its slice layout when its plan
-// (share_plan) has the same rows, its 16-bit offsets when its block schedule
+// pointers and column indices are reused, its slices' heads and codes with
+// share_slices (the same plan), its 16-bit offsets when its block schedule
 // (share_starts) is the same
 template <typename VT, typename OT = double>
 static void upload_mat(const Csr& A, const SlicePlan& plan, const std::vector<int>& starts_with_end,
                        dev::DMat<VT>& D, DevBuffers& B, hipStream_t st, const dev::DMat<OT>* share = nullptr,
-                       const SlicePlan* share_plan = nullptr, const std::vector<int>* share_starts = nullptr,
+                       bool share_slices = false, const std::vector<int>* share_starts = nullptr,
                        const int* row_ids = nullptr, const std::vector<int>* seg = nullptr) {
     validate(A, starts_with_end, dev::block_nnz<VT>());
+    validate(A, plan);
     D.active = nullptr;
     D.n = A.n;
     D.ncols = A.ncols;
@@ -390,11 +420,7 @@ static void upload_mat(const Csr& A, const SlicePlan& plan, const std::vector<in
         }
         D.lpr = dev::lanes_per_row(A.n > 0 ? (double)A.nnz() / A.n : 0.0);
     }
-    if (!plan.head.empty()) {
-        const bool same = share && share_plan && share_plan->lt == plan.lt &&
-                          share_plan->head.size() == plan.head.size();
-        make_slices<VT, OT>(plan, D, B, st, same ? share : nullptr);
-    }
+    if (!plan.head.empty()) make_slices<VT, OT>(plan, D, B, st, share_slices ? share : nullptr);
     if (seg) {  // the systems of each slice, or of each block where there are no slices
         std::vector<int> first;
         for (const dev::SliceHead& k : plan.head) first.push_back(k.row0);
@@ -436,33 +462,59 @@ static std::vector<int> schedule(const Csr& A) {
     return starts;
 }
 
-// upload A as FP64 + FP32 copies sharing the index arrays; free32: the FP32
-// rows may be summed in any order (see Solver::fixed_order); partials: the
-// FP64 product's block partials are summed by a Krylov method (its row order is
-// kept then, and its partials' too without free32); returns the larger
-// workgroup count of a row kernel
-int upload_pair(const Csr& A0, dev::DMat<double>& D, dev::DMat<float>& F, DevBuffers& B, hipStream_t st,
-                const std::vector<int>* seg, bool free32, bool partials) {
-    Csr A = drop_outside_zeros(A0);
-    // the FP64 finest matrix (partials) keeps a row's column order
-    SlicePlan p64 = plan_slices(A, {}, !partials), p32 = plan_slices(A, {}, free32);
+// the slices and row blocks of a matrix's FP64 and FP32 copies
+struct PairPlan {
+    SlicePlan p64, p32;
     std::vector<int> s64, s32;
-    if (partials && !free32 && !seg && !p64.head.empty() && p64.lt == 0) {
+    bool shared = false;  // one plan: the FP32 copy takes the FP64 copy's heads and codes
+};
+
+// free32: the FP32 rows may be summed in any order (see Solver::fixed_order);
+// partials: the FP64 product's block partials are summed by a Krylov method
+// (its row order is kept then, and its partials' too without free32)
+static PairPlan plan_pair(const Csr& A, bool batch, bool free32, bool partials) {
+    PairPlan q;
+    // the FP64 finest matrix (partials) keeps a row's column order
+    q.p64 = plan_slices(A, {}, !partials);
+    q.p32 = plan_slices(A, {}, free32);
+    if (partials && !free32 && !batch && !q.p64.head.empty() && q.p64.lt == 0) {
         // slices by row block where they fill their wavefronts (1.05M rows x
         // 7: 256-row blocks), else the block form beside them (2.1M x 14, 146
         // rows a block: 76 us, 87 us as slices of 64, 64 and 18 rows)
-        s64 = schedule<double>(A);
-        SlicePlan q = plan_slices(A, {}, false, &s64);
-        if (!q.head.empty() && A.n >= 0.9 * 64 * q.head.size()) {
-            p64 = std::move(q);
-            s64.clear();
+        q.s64 = schedule<double>(A);
+        SlicePlan b = plan_slices(A, {}, false, &q.s64);
+        if (!b.head.empty() && A.n >= 0.9 * 64 * b.head.size()) {
+            q.p64 = std::move(b);
+            q.s64.clear();
         }
     }
-    if (p64.head.empty()) s64 = schedule<double>(A);
-    if (p32.head.empty()) s32 = schedule<float>(A);
-    upload_mat<double, double>(A, p64, s64, D, B, st, nullptr, nullptr, nullptr, nullptr, seg);
-    upload_mat(A, p32, s32, F, B, st, &D, &p64, &s64, nullptr, seg);
+    if (q.p64.head.empty()) q.s64 = schedule<double>(A);
+    if (q.p32.head.empty()) q.s32 = schedule<float>(A);
+    // the FP32 plan is cut every 64 rows, the FP64 plan now and then by row
+    // block: as many slices need not be the same rows
+    q.shared = same_rows(q.p64, q.p32);
+    return q;
+}
+
+// upload A as FP64 + FP32 copies sharing the index arrays (options: see
+// plan_pair); returns the larger workgroup count of a row kernel
+int upload_pair(const Csr& A0, dev::DMat<double>& D, dev::DMat<float>& F, DevBuffers& B, hipStream_t st,
+                const std::vector<int>* seg, bool free32, bool partials) {
+    Csr A = drop_outside_zeros(A0);
+    const PairPlan q = plan_pair(A, seg != nullptr, free32, partials);
+    upload_mat<double, double>(A, q.p64, q.s64, D, B, st, nullptr, false, nullptr, nullptr, seg);
+    upload_mat(A, q.p32, q.s32, F, B, st, &D, q.shared, &q.s64, nullptr, seg);
     return std::max(dev::row_blocks(D), dev::row_blocks(F));
+}
+
+std::vector<dev::SliceHead> slice_layout(const Csr& A, bool free32, bool partials, int precision, int* lt,
+                                         size_t* steps) {
+    const PairPlan q = plan_pair(A, false, free32, partials);
+    const bool fp64 = precision == LINA_PREC_FP64;
+    const SlicePlan& own = fp64 ? q.p64 : q.p32;
+    *lt = own.lt;
+    *steps = own.steps;
+    return !fp64 && q.shared ? q.p64.head : own.head;
 }
 
 // level schedule of the lexicographic sweep: forward, level(i) = 1 + max over
@@ -718,8 +770,8 @@ void Solver::upload() {
         else d.colour_blk = q64.group;
         if (q32.head.empty()) c32 = colour_schedule(dev::block_nnz<float>(), d.colour_blk32);
         else d.colour_blk32 = q32.group;
-        upload_mat<double, double>(Ac, q64, c64, d.Ac, B, st, nullptr, nullptr, nullptr, perm.data(), segl);
-        upload_mat(Ac, q32, c32, d.Acf, B, st, &d.Ac, &q64, &c64, perm.data(), segl);
+        upload_mat<double, double>(Ac, q64, c64, d.Ac, B, st, nullptr, false, nullptr, perm.data(), segl);
+        upload_mat(Ac, q32, c32, d.Acf, B, st, &d.Ac, same_rows(q64, q32), &c64, perm.data(), segl);
         d.perm = dupload(perm, B, st);
         d.ncolours = nc;
         if (track_) {

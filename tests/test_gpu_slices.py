@@ -75,3 +75,37 @@ def test_values_follow_an_update(gpu):
         assert ra["iters"] == rb["iters"] and np.array_equal(ra["x"], rb["x"])
         a.close()
         b.close()
+
+
+@pytest.mark.parametrize("hub", [3, 300])
+def test_finest_copies_with_unequal_row_blocks(gpu, hub):
+    """an aggressive hierarchy's finest matrix whose FP64 copy is cut by row
+    block and whose FP32 copy is cut every 64 rows: as many slices, other rows"""
+    import scipy.sparse as sp
+    from fem_amd import problems as P
+    s = P.damage_system(783)[0]
+    A, n = s.scipy().tocsr(), s.n
+    for c in (20_000, 333_333):  # rows coupled to `hub` far ones
+        j = 1000 + (c + 2039 * np.arange(hub)) % (n - 2000)
+        j = j[j != c]
+        i = np.full(len(j), c)
+        w = sp.coo_matrix((np.full(len(j), 1e-3), (i, j)), shape=(n, n)).tocsr()
+        w = w + w.T
+        A = A + sp.diags(np.asarray(w.sum(axis=1)).ravel()) - w
+    A = A.tocsr()
+    A.sort_indices()
+    rp, ci = A.indptr, A.indices
+    rows = [gpu.slice_layout(rp, ci, False, True, p)[0] for p in ("fp64", "mixed")]
+    unequal = len(rows[0]) == len(rows[1]) and not np.array_equal(rows[0], rows[1])
+    assert unequal == (hub == 300)
+    print("finest copies", hub, len(rows[0]), flush=True)
+    amg = gpu.AMG(rp, ci, A.data, gpu.params("vcycle", 1, 6, precision="mixed"))
+    x = np.random.default_rng(5).standard_normal(n)
+    ref, bound = A @ x, abs(A) @ np.abs(x)
+    m = np.diff(rp)
+    assert np.all(np.abs(amg.spmv(x) - ref) <= 2 * (m + 1) * 2.0 ** -53 * bound)
+    assert np.all(np.abs(amg.spmv(x, precision="mixed") - ref) <= (m + 4) * 2.0 ** -24 * bound)
+    b = np.random.default_rng(6).standard_normal(n)
+    got = amg.pcg(b, tol=1e-9, max_iter=400, stop="relres")
+    amg.close()
+    assert np.linalg.norm(A @ got["x"] - b) <= 1e-8 * np.linalg.norm(b)
