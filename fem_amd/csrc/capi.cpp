@@ -364,8 +364,8 @@ double lina_spmv_bytes(const lina_solver* s, int level, int precision) {
     return s->s.spmv_bytes(level, precision);
 }
 
-int lina_slice_layout(int n, const int* rowptr, const int* col, int free32, int partials, int precision, int cap,
-                      int* heads, int* lanes, long* steps) {
+int lina_slice_layout(int n, const int* rowptr, const int* col, const int* colours, int free32, int partials,
+                      int precision, int cap, int* heads, int* lanes, long* steps) {
     return guard([&]() {
         if (!rowptr || !col || !lanes || !steps || (cap > 0 && !heads)) throw std::invalid_argument("null argument");
         if (precision != LINA_PREC_FP64 && precision != LINA_PREC_MIXED) throw std::invalid_argument("precision");
@@ -373,7 +373,7 @@ int lina_slice_layout(int n, const int* rowptr, const int* col, int free32, int 
         const Csr A = make_csr(n, rowptr, col, ones.data());
         int lt = 0;
         size_t st = 0;
-        const auto h = lina::slice_layout(A, free32 != 0, partials != 0, precision, &lt, &st);
+        const auto h = lina::slice_layout(A, colours, free32 != 0, partials != 0, precision, &lt, &st);
         for (int s = 0; s < std::min(cap, (int)h.size()); s++) {
             heads[4 * s] = h[s].row0;
             heads[4 * s + 1] = h[s].row1;

@@ -239,7 +239,10 @@ static std::vector<int2> block_systems(const std::vector<int>& starts_with_end, 
 //
 // No slices where more than twice the entries would be read: those are the
 // coarsest levels with a few rows many times the mean, which the block form
-// splits evenly.
+// splits evenly.  Nor where more than four times the entries and 1M (10 MB in
+// FP64) would be stored: a step takes 64 entries however few rows its slice has,
+// so many small groups of long rows (a clique's colours) cost up to 64 / T
+// times what they read.
 struct SlicePlan {
     std::vector<dev::SliceHead> head;
     std::vector<int> group;  // first slice of each group, then the slice count
@@ -293,9 +296,10 @@ SlicePlan plan_slices(const Csr& A, const std::vector<int>& groups, bool free_or
     // entries read: lanes past a slice's rows load nothing
     size_t read = 0;
     for (const dev::SliceHead& h : p.head) read += (size_t)h.steps * T * (h.row1 - h.row0);
-    if (read > 2 * (size_t)nnz) {  // 64 steps < 2^32: step0 fits an int
+    if (read > 2 * (size_t)nnz || 64 * steps > 4 * (size_t)nnz + (1 << 20)) {  // nnz < 2^31: step0 fits an int
         p.head.clear();
         p.group.clear();
+        p.steps = 0;
     }
     return p;
 }
@@ -507,9 +511,52 @@ int upload_pair(const Csr& A0, dev::DMat<double>& D, dev::DMat<float>& F, DevBuf
     return std::max(dev::row_blocks(D), dev::row_blocks(F));
 }
 
-std::vector<dev::SliceHead> slice_layout(const Csr& A, bool free32, bool partials, int precision, int* lt,
-                                         size_t* steps) {
-    const PairPlan q = plan_pair(A, false, free32, partials);
+// the rows of A colour by colour (natural order within one): perm the row of A
+// in each place, rows the colours' offsets
+static Csr colour_permuted(const Csr& A, const std::vector<int>& col, int nc, std::vector<int>& perm,
+                           std::vector<int>& rows) {
+    rows.assign(nc + 1, 0);
+    for (int i = 0; i < A.n; i++) rows[col[i] + 1]++;
+    for (int c = 0; c < nc; c++) rows[c + 1] += rows[c];
+    perm.assign(A.n, 0);
+    std::vector<int> fill(rows.begin(), rows.end() - 1);
+    for (int i = 0; i < A.n; i++) perm[fill[col[i]]++] = i;
+    Csr Ac;
+    Ac.n = A.n;
+    Ac.ncols = A.n;
+    Ac.rp.assign(A.n + 1, 0);
+    Ac.ci.reserve(A.nnz());
+    Ac.v.reserve(A.nnz());
+    for (int r = 0; r < A.n; r++) {
+        const int i = perm[r];
+        Ac.ci.insert(Ac.ci.end(), A.ci.begin() + A.rp[i], A.ci.begin() + A.rp[i + 1]);
+        Ac.v.insert(Ac.v.end(), A.v.begin() + A.rp[i], A.v.begin() + A.rp[i + 1]);
+        Ac.rp[r + 1] = (int)Ac.ci.size();
+    }
+    return Ac;
+}
+
+// the slices of a colour-permuted copy's two precisions
+static PairPlan plan_colours(const Csr& Ac, const std::vector<int>& rows, bool free32) {
+    PairPlan q;
+    q.p64 = plan_slices(Ac, rows, true);
+    q.p32 = plan_slices(Ac, rows, free32);
+    q.shared = same_rows(q.p64, q.p32);
+    return q;
+}
+
+std::vector<dev::SliceHead> slice_layout(const Csr& A, const int* colours, bool free32, bool partials, int precision,
+                                         int* lt, size_t* steps) {
+    PairPlan q;
+    if (colours) {
+        std::vector<int> col(colours, colours + A.n), perm, rows;
+        const int nc = A.n > 0 ? *std::max_element(col.begin(), col.end()) + 1 : 0;
+        for (int c : col)
+            if (c < 0) throw std::invalid_argument("negative colour");
+        q = plan_colours(colour_permuted(A, col, nc, perm, rows), rows, free32);
+    } else {
+        q = plan_pair(A, false, free32, partials);
+    }
     const bool fp64 = precision == LINA_PREC_FP64;
     const SlicePlan& own = fp64 ? q.p64 : q.p32;
     *lt = own.lt;
@@ -729,29 +776,8 @@ void Solver::upload() {
         // colour-permuted copy for the multicolour sweeps
         const std::vector<int>& col = colours_[l];
         int nc = ncolours_[l];
-        std::vector<int> perm(d.n);
-        {
-            std::vector<int> cnt(nc + 1, 0);
-            for (int i = 0; i < d.n; i++) cnt[col[i] + 1]++;
-            for (int c = 0; c < nc; c++) cnt[c + 1] += cnt[c];
-            std::vector<int> fill(cnt.begin(), cnt.end() - 1);
-            for (int i = 0; i < d.n; i++) perm[fill[col[i]]++] = i;
-            d.colour_rows = cnt;
-        }
-        Csr Ac;
-        Ac.n = d.n;
-        Ac.ncols = d.n;
-        Ac.rp.assign(d.n + 1, 0);
-        Ac.ci.reserve(h.A.nnz());
-        Ac.v.reserve(h.A.nnz());
-        for (int r = 0; r < d.n; r++) {
-            int i = perm[r];
-            for (int p = h.A.rp[i]; p < h.A.rp[i + 1]; p++) {
-                Ac.ci.push_back(h.A.ci[p]);
-                Ac.v.push_back(h.A.v[p]);
-            }
-            Ac.rp[r + 1] = (int)Ac.ci.size();
-        }
+        std::vector<int> perm;
+        const Csr Ac = colour_permuted(h.A, col, nc, perm, d.colour_rows);
         // colour c's rows form the slices or blocks [colour_blk[c], colour_blk[c+1])
         auto colour_schedule = [&](int max_nnz, std::vector<int>& cb) {
             std::vector<int> starts;
@@ -764,14 +790,13 @@ void Solver::upload() {
             starts.push_back(d.n);
             return starts;
         };
-        const SlicePlan q64 = plan_slices(Ac, d.colour_rows, true), q32 = plan_slices(Ac, d.colour_rows, !fixed_order());
-        std::vector<int> c64, c32;
-        if (q64.head.empty()) c64 = colour_schedule(dev::block_nnz<double>(), d.colour_blk);
-        else d.colour_blk = q64.group;
-        if (q32.head.empty()) c32 = colour_schedule(dev::block_nnz<float>(), d.colour_blk32);
-        else d.colour_blk32 = q32.group;
-        upload_mat<double, double>(Ac, q64, c64, d.Ac, B, st, nullptr, false, nullptr, perm.data(), segl);
-        upload_mat(Ac, q32, c32, d.Acf, B, st, &d.Ac, same_rows(q64, q32), &c64, perm.data(), segl);
+        PairPlan q = plan_colours(Ac, d.colour_rows, !fixed_order());
+        if (q.p64.head.empty()) q.s64 = colour_schedule(dev::block_nnz<double>(), d.colour_blk);
+        else d.colour_blk = q.p64.group;
+        if (q.p32.head.empty()) q.s32 = colour_schedule(dev::block_nnz<float>(), d.colour_blk32);
+        else d.colour_blk32 = q.p32.group;
+        upload_mat<double, double>(Ac, q.p64, q.s64, d.Ac, B, st, nullptr, false, nullptr, perm.data(), segl);
+        upload_mat(Ac, q.p32, q.s32, d.Acf, B, st, &d.Ac, q.shared, &q.s64, perm.data(), segl);
         d.perm = dupload(perm, B, st);
         d.ncolours = nc;
         if (track_) {

@@ -146,10 +146,11 @@ struct DevLevel {
 
 int upload_pair(const Csr& A0, dev::DMat<double>& D, dev::DMat<float>& F, DevBuffers& B, hipStream_t st,
                 const std::vector<int>* seg, bool free32, bool partials);
-// the slices that upload_pair's FP64 or FP32 copy of A reads (none: row blocks),
-// log2 of the lanes a row and the steps its values are stored for; no device needed
-std::vector<dev::SliceHead> slice_layout(const Csr& A, bool free32, bool partials, int precision, int* lt,
-                                         size_t* steps);
+// the slices that upload_pair's FP64 or FP32 copy of A (colours: of A with its
+// rows colour by colour) reads (none: row blocks), log2 of the lanes a row and
+// the steps its values are stored for; no device needed
+std::vector<dev::SliceHead> slice_layout(const Csr& A, const int* colours, bool free32, bool partials, int precision,
+                                         int* lt, size_t* steps);
 // a sliced copy of D (CSR of A uploaded) where worthwhile; false: none
 bool slice_matrix(const Csr& A, dev::DMat<double>& D, DevBuffers& B, hipStream_t st);
 // both precisions' sliced values from their CSR values

@@ -108,7 +108,7 @@ def lib():
     L.lina_spmv_bytes.argtypes = [C.c_void_p, C.c_int, C.c_int]
     L.lina_spmv_bytes.restype = C.c_double
     L.lina_amg_kernel_timing.argtypes = [C.c_void_p, C.c_int]
-    L.lina_slice_layout.argtypes = [C.c_int, _ip, _ip, C.c_int, C.c_int, C.c_int, C.c_int, _ip, _ip,
+    L.lina_slice_layout.argtypes = [C.c_int, _ip, _ip, _ip, C.c_int, C.c_int, C.c_int, C.c_int, _ip, _ip,
                                     C.POINTER(C.c_long)]
     L.lina_amg_tuned.argtypes = [C.c_void_p, _ip, C.c_char_p, _ip, _ip, C.c_int]
     L.lina_dev_alloc.argtypes = [C.c_long]
@@ -368,13 +368,15 @@ class AMG:
         return lib().lina_spmv_bytes(self.h, l, PREC[precision])
 
 
-def slice_layout(rowptr, col, free32=True, partials=False, precision="fp64"):
-    """(heads, lanes, steps) of the sliced copy of a matrix: a row (row0, row1,
-    step0, steps) per slice, lanes a row, steps stored (lina_slice_layout; no
-    slices: the row-block form)"""
+def slice_layout(rowptr, col, free32=True, partials=False, precision="fp64", colours=None):
+    """(heads, lanes, steps) of the sliced copy of a matrix (colours: with its
+    rows colour by colour): a row (row0, row1, step0, steps) per slice, lanes a
+    row, steps stored (lina_slice_layout; no slices: the row-block form)"""
     rp, ci = np.ascontiguousarray(rowptr, np.int32), np.ascontiguousarray(col, np.int32)
     lanes, steps = np.zeros(1, np.int32), C.c_long()
-    args = (len(rp) - 1, _i(rp), _i(ci), int(free32), int(partials), PREC[precision])
+    colours = None if colours is None else np.ascontiguousarray(colours, np.int32)
+    args = (len(rp) - 1, _i(rp), _i(ci), None if colours is None else _i(colours), int(free32), int(partials),
+            PREC[precision])
     none = np.zeros((1, 4), np.int32)
     m = _check(lib().lina_slice_layout(*args, 0, _i(none), _i(lanes), C.byref(steps)))
     heads = np.zeros((max(m, 1), 4), np.int32)

@@ -262,11 +262,12 @@ int lina_amg_kernel_timing(lina_solver* s, int on);
 /* the sliced layout that a matrix's FP64 (precision LINA_PREC_FP64) or FP32
  * copy is stored and read in, worked out on the host: slice s holds the rows
  * [heads[4s], heads[4s+1]) and the steps [heads[4s+2], + heads[4s+3]) of the
- * copy's *steps, 64 entries each, *lanes lanes a row.  free32: FP32 row sums in
- * any order; partials: the FP64 product feeds a Krylov method's dot (the finest
+ * copy's *steps, 64 entries each, *lanes lanes a row.  colours (NULL: none): of
+ * the copy with its rows colour by colour instead.  free32: FP32 row sums in any
+ * order; partials: the FP64 product feeds a Krylov method's dot (the finest
  * matrix).  Writes up to cap slices, returns their number (0: row blocks) */
-int lina_slice_layout(int n, const int* rowptr, const int* col, int free32, int partials, int precision, int cap,
-                      int* heads, int* lanes, long* steps);
+int lina_slice_layout(int n, const int* rowptr, const int* col, const int* colours, int free32, int partials,
+                      int precision, int cap, int* heads, int* lanes, long* steps);
 /* the autotuner's choices (params.autotune): per tuned matrix its level, kind
  * (A, P, R, C = colour-permuted A) and lanes per row for the FP64 / FP32
  * copies; returns the number of entries (arrays of size cap) */

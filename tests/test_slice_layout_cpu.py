@@ -1,7 +1,8 @@
 """The sliced layouts of a matrix's FP64 and FP32 copies, worked out on the
 host: every copy is stored with the steps its slices read, whichever way the
 two plans are cut (the finest FP64 matrix of an aggressive hierarchy by row
-block, the FP32 copy every 64 rows).  No device call is made here."""
+block, the FP32 copy every 64 rows), and no copy stores more than its bound.
+No device call is made here."""
 import numpy as np
 import pytest
 
@@ -78,3 +79,21 @@ def test_layouts_over_row_counts_and_lengths(n, mean, free32, partials):
     rp, ci = rows_with(m, n)
     for precision in ("fp64", "mixed"):
         check_layout(rp, *lina.slice_layout(rp, ci, free32, partials, precision))
+
+
+@pytest.mark.parametrize("free32", [True, False])
+@pytest.mark.parametrize("clique,sliced", [(40, True), (700, False)])
+def test_small_colours_of_long_rows_do_not_fill_memory(clique, sliced, free32):
+    """a clique's rows have a colour each: a slice of one row stores 64 / lanes
+    times the row"""
+    n = 200_000
+    m = np.full(n, 7)
+    m[:clique] = clique
+    rp, ci = rows_with(m, clique)
+    colours = np.arange(n) % 4
+    colours[:clique] = np.arange(clique)
+    for precision in ("fp64", "mixed"):
+        heads, lanes, steps = lina.slice_layout(rp, ci, free32, precision=precision, colours=colours)
+        assert (len(heads) > 0) == sliced
+        assert 64 * steps <= 4 * len(ci) + 2 ** 20
+        check_layout(np.append(0, np.cumsum(m[np.argsort(colours, kind="stable")])), heads, lanes, steps)
