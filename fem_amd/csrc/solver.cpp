@@ -501,14 +501,16 @@ static PairPlan plan_pair(const Csr& A, bool batch, bool free32, bool partials) 
 }
 
 // upload A as FP64 + FP32 copies sharing the index arrays (options: see
-// plan_pair); returns the larger workgroup count of a row kernel
+// plan_pair); returns the largest workgroup count of a row kernel over either
+// copy in either form
 int upload_pair(const Csr& A0, dev::DMat<double>& D, dev::DMat<float>& F, DevBuffers& B, hipStream_t st,
                 const std::vector<int>* seg, bool free32, bool partials) {
     Csr A = drop_outside_zeros(A0);
     const PairPlan q = plan_pair(A, seg != nullptr, free32, partials);
     upload_mat<double, double>(A, q.p64, q.s64, D, B, st, nullptr, false, nullptr, nullptr, seg);
     upload_mat(A, q.p32, q.s32, F, B, st, &D, q.shared, &q.s64, nullptr, seg);
-    return std::max(dev::row_blocks(D), dev::row_blocks(F));
+    const int blocks = std::max((int)schedule<double>(A).size(), (int)schedule<float>(A).size()) - 1;
+    return std::max({dev::row_blocks(D), dev::row_blocks(F), blocks});
 }
 
 // the rows of A colour by colour (natural order within one): perm the row of A
@@ -918,8 +920,10 @@ void Solver::upload() {
     kW_ = dalloc<double>(n, B);
     kX_ = dalloc<double>(n, B);
     kB_ = dalloc<double>(n, B);
-    // block partials: one per SpMV block (any matrix) or per reduction block
-    int np = std::max(4096, maxblk + 16);
+    // block partials: one per SpMV workgroup (any matrix, and any sliced operator
+    // of this size: at least 2 rows a slice, 4 slices a workgroup) or per
+    // reduction block
+    int np = std::max({4096, maxblk + 16, n / (2 * dev::SLICES_PER_BLOCK) + 32});
     part_ = dalloc<double>(np + 3 * dev::DOT_PART_MAX, B);  // and three dots' partials beside a product's
     part_cap_ = np;
     scal_ = dalloc<double>(dev::S_COUNT, B);

@@ -109,3 +109,29 @@ def test_finest_copies_with_unequal_row_blocks(gpu, hub):
     got = amg.pcg(b, tol=1e-9, max_iter=400, stop="relres")
     amg.close()
     assert np.linalg.norm(A @ got["x"] - b) <= 1e-8 * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("irregular", [False, True])
+def test_operator_with_longer_rows_than_the_hierarchy(gpu, irregular):
+    """pcg on an operator of about 100 entries a row (more sliced workgroups than
+    the hierarchy's matrices have; irregular: in row blocks) under a P1 hierarchy"""
+    import scipy.sparse as sp
+    from fem_amd import problems as P
+    s = P.poisson(257)
+    n = s.n
+    i = np.arange(n)
+    if irregular:
+        i = i[i % 50 == 0]
+    j = (i[:, None] + 37 * np.arange(1, 48 if not irregular else 400)) % n
+    w = sp.coo_matrix((np.full(j.size, 1e-4), (np.repeat(i, j.shape[1]), j.ravel())), shape=(n, n)).tocsr()
+    w = w + w.T
+    A = (s.scipy() + sp.diags(np.asarray(w.sum(axis=1)).ravel()) - w).tocsr()
+    A.sort_indices()
+    amg = gpu.AMG(s.rowptr, s.col, s.val, gpu.params("vcycle", 1, 5))
+    op = gpu.Matrix(A.indptr, A.indices, A.data)
+    assert (len(gpu.slice_layout(A.indptr, A.indices, True, True)[0]) == 0) == irregular
+    b = np.random.default_rng(8).standard_normal(n)
+    got = amg.pcg_operator(op, b, tol=1e-9, max_iter=500)
+    op.close()
+    amg.close()
+    assert np.linalg.norm(A @ got["x"] - b) <= 1e-8 * np.linalg.norm(b)
