@@ -696,6 +696,16 @@ int lina_ilu_factor_nnz(const lina_ilu* h, char which) {
     return which == 'L' ? s.L().nnz() : s.U().nnz();
 }
 
+long lina_ilu_level_entries(const lina_ilu* h, char which) {
+    long out = -1;
+    const int rc = guard([&]() {
+        if (!h || (which != 'L' && which != 'U')) throw std::invalid_argument("bad argument");
+        out = (long)const_cast<lina_ilu*>(h)->s.wide_entries(which);
+        return 0;
+    });
+    return rc < 0 ? -1 : out;
+}
+
 int lina_ilu_factor_copy(const lina_ilu* h, char which, int* rowptr, int* col, double* val) {
     lina::IluSystem& s = const_cast<lina_ilu*>(h)->s;
     const Csr& M = which == 'L' ? s.L() : s.U();

@@ -70,16 +70,21 @@ class IluSystem {
         double* ovval = nullptr;
     };
 
+    // entries that the padded levels of factor 'L' or 'U' store (0: the sweeps
+    // take another form); needs no device
+    size_t wide_entries(char which);
+
     // a factor's levels padded for dev::tri_level, and their value maps
     struct TriWide {
         std::vector<dev::TriLevel> lv;
-        int nval = 0;
+        size_t nval = 0;
         int *vmap = nullptr, *dmap = nullptr;
         double *val = nullptr, *diag = nullptr;
     };
 
   private:
-    void build_wide(const Csr& T, bool upper, const std::vector<int>& off, const std::vector<int>& rows, TriWide& W);
+    void build_wide(const Csr& T, const dev::DMat<double>& D, bool upper, const std::vector<int>& off,
+                    const std::vector<int>& rows, TriWide& W);
     // w = U^-1 L^-1 z by levels; part: block partials of z.w, returns their number
     int apply_wide(const double* z, double* w, double* part);
     TriWide wl_, wu_;

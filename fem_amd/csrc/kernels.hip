@@ -1663,13 +1663,15 @@ __global__ __launch_bounds__(TPB) void k_ilu0_planned_level(int t0, int t1, cons
 // slot-major arrays in level order, so a lane waits for two memory round trips
 // (entries, results) instead of the four of the factor's CSR (row, bounds,
 // entries, results) -- 301 x 203 Poisson, a level of 15k rows: 3.5 -> 2.5 us.
+// Entries past a level's slots (tri_level_slots) come from the CSR, after them
+// and in row order: the same sums.
 template <int K>
 __device__ __forceinline__ double tri_row(const TriLevel& L, int t, double s, const double* out) {
     int c[K];
     double v[K], x[K];
 #pragma unroll
     for (int k = 0; k < K; k++) {
-        const int q = min(k, L.K - 1) * L.cnt + t;
+        const size_t q = (size_t)min(k, L.K - 1) * L.cnt + t;
         c[k] = L.col[q];
         v[k] = L.val[q];
     }
@@ -1700,6 +1702,9 @@ __global__ __launch_bounds__(TPB) void k_tri_level(const TriLevel L, const doubl
                 if (c >= 0) s -= L.val[(size_t)k * L.cnt + t] * out[c];
             }
         }
+        if (L.rp)
+            for (int p = L.rp[i] + L.first + L.K, e = L.rp[i + 1] - 1 + L.first; p < e; p++)
+                s -= L.v[p] * out[L.ci[p]];
         s /= d;
         out[i] = s;
         if (!w) {
@@ -1716,9 +1721,9 @@ __global__ __launch_bounds__(TPB) void k_tri_level(const TriLevel L, const doubl
     }
 }
 
-__global__ void k_tri_gather(int n, const int* __restrict__ map, const double* __restrict__ v,
+__global__ void k_tri_gather(long n, const int* __restrict__ map, const double* __restrict__ v,
                              double* __restrict__ val) {
-    for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < n; q += gridDim.x * blockDim.x)
+    for (long q = blockIdx.x * blockDim.x + threadIdx.x; q < n; q += gridDim.x * blockDim.x)
         val[q] = map[q] >= 0 ? v[map[q]] : 0.0;
 }
 
@@ -3214,8 +3219,10 @@ void tri_level(hipStream_t st, const TriLevel& L, const double* in, double* out,
         hipLaunchKernelGGL(k_tri_level, dim3(tri_level_blocks(L)), dim3(TPB), 0, st, L, in, out, ud, w, r, part);
 }
 
-void tri_values(hipStream_t st, int n, const int* map, const double* v, double* val) {
-    if (n > 0) hipLaunchKernelGGL(k_tri_gather, dim3(grid_for(n)), dim3(TPB), 0, st, n, map, v, val);
+void tri_values(hipStream_t st, long n, const int* map, const double* v, double* val) {
+    if (n <= 0) return;
+    const int g = grid_for((int)std::min(n, 1L << 30));
+    hipLaunchKernelGGL(k_tri_gather, dim3(g), dim3(TPB), 0, st, n, map, v, val);
 }
 
 void ipcg_p(hipStream_t st, int n, int first, double* P, const double* Z, double* scal, const double* rz, int nrz,

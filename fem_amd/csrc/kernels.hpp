@@ -394,15 +394,27 @@ void ilu0_planned_levels(hipStream_t st, const std::vector<int>& off, const int4
                          const int* mask, const int* pu, const double* vA, double* vL, double* vU, int* fail);
 // One level of a triangular factor for a launch of its own (the multicolour
 // order's few wide levels): row t < cnt is factor row rows[t] (row0 + t when
-// rows is nullptr), its K padded entries val/col[k cnt + t] in row order
-// (col < 0: none), its diagonal diag[t].
+// rows is nullptr), its first K entries val/col[k cnt + t] in row order, padded
+// (col < 0: none), its diagonal diag[t].  Levels with longer rows (rp given):
+// row i's other entries are ci/v[rp[i] + first + K, rp[i + 1] - 1 + first) of
+// the factor's CSR (first: 1 for U, whose rows begin with the diagonal, 0 for
+// L, whose rows end with it).
 struct TriLevel {
-    int cnt = 0, K = 0, row0 = 0;
+    int cnt = 0, K = 0, row0 = 0, first = 0;
     const int* rows = nullptr;
     const int* col = nullptr;
     const double* val = nullptr;
     const double* diag = nullptr;
+    const int *rp = nullptr, *ci = nullptr;
+    const double* v = nullptr;
 };
+// padded entries a row of a wide level of cnt rows with ent off-diagonal
+// entries in all and at most longest in one: those of its longest row, unless
+// that pads beyond three times the entries (a few long rows)
+inline int tri_level_slots(long cnt, long ent, int longest) {
+    if (cnt <= 0 || longest * cnt <= 3 * ent) return longest;
+    return (int)((3 * ent + cnt - 1) / cnt);
+}
 // workgroups of a level's launch (its partials' number)
 int tri_level_blocks(const TriLevel& L);
 // out_i = (in_i - sum val out_col) / diag, PCG_preconl's and PCG_preconr's
@@ -412,7 +424,7 @@ int tri_level_blocks(const TriLevel& L);
 void tri_level(hipStream_t st, const TriLevel& L, const double* in, double* out, const double* ud, double* w,
                const double* r, double* part);
 // val[q] = v[map[q]] (map < 0: 0) for the padded entries and diagonals of a factor
-void tri_values(hipStream_t st, int n, const int* map, const double* v, double* val);
+void tri_values(hipStream_t st, long n, const int* map, const double* v, double* val);
 
 // ILU-pcg on the device (IluSystem::pcg_core), its sums as in pcg_direction
 enum { IS_S = 0, IS_RZ = 1, IS_PQ = 2, IS_RR = 3, IS_STOP = 4, IS_IT = 5, IS_R = 6, IS_R0 = 7, IS_TOL = 8,

@@ -480,6 +480,43 @@ void IluSystem::set_factors(const Csr& L, const Csr& U, bool up) {
     if (up) upload();
 }
 
+// slots a row of each level (dev::tri_level_slots) of a triangular factor and,
+// in longest, its longest row
+static std::vector<int> wide_slots(const Csr& T, const std::vector<int>& off, const std::vector<int>& rows,
+                                   std::vector<int>& longest) {
+    const int nlv = (int)off.size() - 1;
+    std::vector<int> K(nlv);
+    longest.assign(nlv, 0);
+    for (int L = 0; L < nlv; L++) {
+        long ent = 0;
+        for (int t = off[L]; t < off[L + 1]; t++) {
+            const int m = T.rp[rows[t] + 1] - T.rp[rows[t]] - 1;
+            longest[L] = std::max(longest[L], m);
+            ent += m;
+        }
+        K[L] = dev::tri_level_slots(off[L + 1] - off[L], ent, longest[L]);
+    }
+    return K;
+}
+
+// a few wide levels (the multicolour order's): one launch per level on the
+// whole GPU instead of the one-workgroup level packs
+static bool wide_levels(int n, int nlv_l, int nlv_u) { return n >= 4096 && nlv_l <= 64 && nlv_u <= 64; }
+
+size_t IluSystem::wide_entries(char which) {
+    if (ordering_ == 0) return 0;
+    const Csr& T = which == 'L' ? L() : U();
+    std::vector<int> off, rows, offu, rowsu, longest;
+    tri_levels(L(), false, off, rows, true);
+    tri_levels(U(), true, offu, rowsu, true);
+    if (!wide_levels(n_, (int)off.size() - 1, (int)offu.size() - 1)) return 0;
+    const std::vector<int>& o = which == 'L' ? off : offu;
+    const std::vector<int> K = wide_slots(T, o, which == 'L' ? rows : rowsu, longest);
+    size_t sum = 0;
+    for (size_t l = 0; l < K.size(); l++) sum += (size_t)K[l] * (o[l + 1] - o[l]);
+    return sum;
+}
+
 // pattern_levels: level schedules from the factors' patterns (their values
 // are computed on the device afterwards)
 void IluSystem::upload(bool pattern_levels_in) {
@@ -530,9 +567,7 @@ void IluSystem::upload(bool pattern_levels_in) {
         if ((int)vpos_.size() == A_.nnz() && A_.nnz() > 0) dvpos_ = kupload(vpos_, B, st);
         for (double** p : {&vXo_, &vBo_, &vPz_, &vPw_}) *p = kalloc<double>(n, B);
     }
-    // a few wide levels (the multicolour order's): one launch per level on
-    // the whole GPU instead of the one-workgroup level packs
-    wide_ = pattern_levels && n >= 4096 && nlv_l_ <= 64 && nlv_u_ <= 64;
+    wide_ = pattern_levels && wide_levels(n, nlv_l_, nlv_u_);
     // level packs: the forward sweep writes y in the backward sweep's order
     std::vector<int> posu(n), natural(n);
     for (int t = 0; t < n; t++) posu[rowsu[t]] = t;
@@ -564,8 +599,8 @@ void IluSystem::upload(bool pattern_levels_in) {
     wl_ = TriWide();
     wu_ = TriWide();
     if (wide_) {
-        build_wide(L_, false, off, rows, wl_);
-        build_wide(U_, true, offu, rowsu, wu_);
+        build_wide(L_, dL_, false, off, rows, wl_);
+        build_wide(U_, dU_, true, offu, rowsu, wu_);
         std::vector<int> um(n);
         for (int i = 0; i < n; i++) um[i] = U_.rp[i + 1] - U_.rp[i] == 1 ? U_.rp[i] : -1;
         udmap_ = kupload(um, B, st);
@@ -594,22 +629,27 @@ void IluSystem::pack_values() {
 }
 
 // a factor's levels (pattern levels: every off-diagonal entry counts) padded
-// to each level's longest row, slot-major
-void IluSystem::build_wide(const Csr& T, bool upper, const std::vector<int>& off, const std::vector<int>& rows,
-                           TriWide& W) {
+// to dev::tri_level_slots entries a row, slot-major; D: the factor on the device
+void IluSystem::build_wide(const Csr& T, const dev::DMat<double>& D, bool upper, const std::vector<int>& off,
+                           const std::vector<int>& rows, TriWide& W) {
     const int nlv = (int)off.size() - 1;
     std::vector<int> vmap, col, dmap(T.n);
     std::vector<size_t> base(nlv);
+    std::vector<int> longest;
+    const std::vector<int> K = wide_slots(T, off, rows, longest);
     W.lv.assign(nlv, dev::TriLevel());
     for (int L = 0; L < nlv; L++) {
         dev::TriLevel& v = W.lv[L];
         v.cnt = off[L + 1] - off[L];
         v.row0 = v.cnt > 0 ? rows[off[L]] : 0;
         bool run = true;
-        for (int t = 0; t < v.cnt; t++) {
-            const int i = rows[off[L] + t];
-            run = run && i == v.row0 + t;
-            v.K = std::max(v.K, T.rp[i + 1] - T.rp[i] - 1);
+        for (int t = 0; t < v.cnt; t++) run = run && rows[off[L] + t] == v.row0 + t;
+        v.K = K[L];
+        if (v.K < longest[L]) {
+            v.first = upper;
+            v.rp = D.rp;
+            v.ci = D.ci;
+            v.v = D.v;
         }
         v.rows = run ? nullptr : (upper ? lvu_rows_ : lvl_rows_) + off[L];
         base[L] = vmap.size();
@@ -619,9 +659,9 @@ void IluSystem::build_wide(const Csr& T, bool upper, const std::vector<int>& off
             const int i = rows[off[L] + t];
             const int d = upper ? T.rp[i] : T.rp[i + 1] - 1;
             dmap[off[L] + t] = d;
+            const int p0 = T.rp[i] + upper, p1 = std::min(T.rp[i + 1] - !upper, p0 + v.K);
             size_t q = base[L] + t;
-            for (int p = T.rp[i]; p < T.rp[i + 1]; p++) {
-                if (p == d) continue;
+            for (int p = p0; p < p1; p++) {
                 vmap[q] = p;
                 col[q] = T.ci[p];
                 q += v.cnt;
@@ -629,7 +669,7 @@ void IluSystem::build_wide(const Csr& T, bool upper, const std::vector<int>& off
         }
     }
     DevBuffers& B = *bufs_;
-    W.nval = (int)vmap.size();
+    W.nval = vmap.size();
     W.vmap = kupload(vmap, B, stream_);
     W.dmap = kupload(dmap, B, stream_);
     const int* dcol = kupload(col, B, stream_);

@@ -480,6 +480,8 @@ def _bind_krylov(L):
     L.lina_ilu_ok.argtypes = [C.c_void_p]
     L.lina_ilu_refactor.argtypes = [C.c_void_p, C.c_int, _ip, _ip, _dp]
     L.lina_ilu_factor_nnz.argtypes = [C.c_void_p, C.c_char]
+    L.lina_ilu_level_entries.argtypes = [C.c_void_p, C.c_char]
+    L.lina_ilu_level_entries.restype = C.c_long
     L.lina_ilu_factor_copy.argtypes = [C.c_void_p, C.c_char, _ip, _ip, _dp]
     L.lina_ilu_apply.argtypes = [C.c_void_p, _dp, _dp]
     L.lina_ilu_pcg.argtypes = [C.c_void_p, _dp, _dp, C.c_double, C.c_int, C.c_int, _dp]
@@ -541,6 +543,10 @@ class ILU:
         v = np.zeros(max(nnz, 1))
         lib().lina_ilu_factor_copy(self.h, which.encode(), _i(rp), _i(ci), _d(v))
         return rp, ci[:nnz], v[:nnz]
+
+    def level_entries(self, which: str) -> int:
+        """entries, padding included, of the multicolour order's sweep levels (0: another form)"""
+        return _check(lib().lina_ilu_level_entries(self.h, which.encode()))
 
     def apply_device(self, d_z: int, d_w: int):
         """w = U^-1 L^-1 z on device vectors (DeviceVector ptrs)"""

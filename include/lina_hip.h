@@ -197,6 +197,9 @@ int lina_ilu_ok(const lina_ilu* h); /* 0: zero pivot, as the reference's return 
  * steps' use).  lina_ilu_ok reports a zero pivot. */
 int lina_ilu_refactor(lina_ilu* h, int n, const int* rowptr, const int* col, const double* val);
 int lina_ilu_factor_nnz(const lina_ilu* h, char which);
+/* entries, padding included, that the multicolour order's levels of factor
+ * 'L' or 'U' store for the sweeps (0: the sweeps take another form); -1 on error */
+long lina_ilu_level_entries(const lina_ilu* h, char which);
 int lina_ilu_factor_copy(const lina_ilu* h, char which, int* rowptr, int* col, double* val);
 /* PCG_default(A, L, U) (PCGS.c:29-34) with factors given by the caller (L:
  * diagonal last in each row, U: diagonal first); NULL on error */

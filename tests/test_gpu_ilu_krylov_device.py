@@ -82,3 +82,30 @@ def test_gmres_does_not_read_its_work_vectors(gpu):
     got = f.gmres(b, m=20, tol=1e-10, max_iter=400)
     f.close()
     assert np.linalg.norm(A @ got["x"] - b) <= 1e-8 * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("n,hub", [(4099, 300), (30000, 9000)])
+def test_long_rows_in_wide_levels(gpu, n, hub):
+    """rows past a level's slots: their other entries come from the factor's CSR"""
+    print("long rows", n, hub, flush=True)
+    A = spd(n, 4, n)
+    for c in (n // 3, n - 5):
+        j = (c + 1 + 3 * np.arange(hub)) % n
+        w = sp.coo_matrix((np.full(hub, 0.01), (np.full(hub, c), j)), shape=(n, n)).tocsr()
+        w = w + w.T
+        A = A + sp.diags(np.asarray(w.sum(axis=1)).ravel()) - w
+    A = A.tocsr()
+    A.sort_indices()
+    f = gpu.ILU(A.indptr, A.indices, A.data, ordering="multicolour")
+    perm = f.permutation()
+    L, U = (sp.csr_matrix((v, c, r), shape=(n, n)) for r, c, v in (f.factor("L"), f.factor("U")))
+    assert max(f.level_entries(w) for w in "LU") < 3 * (L.nnz + U.nnz)
+    b = np.random.default_rng(9).standard_normal(n)
+    w = f.apply(b)[perm]
+    m = int(max(np.diff(L.indptr).max(), np.diff(U.indptr).max()))
+    # each sweep solves a system perturbed by at most (m + 1) eps, and the check rounds as much again
+    bound = abs(L) @ (abs(U) @ np.abs(w))
+    assert np.all(np.abs(L @ (U @ w) - b[perm]) <= 4 * (m + 1) * 2.0 ** -53 * bound)
+    got = f.pcg(b, tol=1e-10, max_iter=300, stop="relres")
+    f.close()
+    assert np.linalg.norm(A @ got["x"] - b) <= 1e-9 * np.linalg.norm(b)

@@ -136,3 +136,30 @@ def test_ordered_ilu_and_rn_reject_unknown_orderings():
     prm = lina.rn_params("pcg", 1, 3, ilu_ordering=7)
     with pytest.raises(lina.LinaError, match="ordering"):
         lina.ReflectiveNewton(s.rowptr, s.col, s.val, s.b, np.zeros(s.n), np.ones(s.n), prm)
+
+
+def test_wide_level_storage_is_bounded():
+    """multicolour ILU(0): a level's padded entries stay near the factor's own
+    where a few rows are hundreds of times longer than the others"""
+    import scipy.sparse as sp
+    s = P.damage_system(129)[0]
+    A = s.scipy().tocsr()
+    for hub in (0, 40, 2500):
+        B = A
+        for c in (5000, 11111):
+            j = (c + 3 + 5 * np.arange(hub)) % s.n
+            j = j[j != c]
+            w = sp.coo_matrix((np.full(len(j), 1e-3), (np.full(len(j), c), j)), shape=A.shape).tocsr()
+            w = w + w.T
+            B = B + sp.diags(np.asarray(w.sum(axis=1)).ravel()) - w
+        B = B.tocsr()
+        B.sort_indices()
+        f = lina.ILU(B.indptr, B.indices, B.data, upload=False, ordering="multicolour")
+        assert f.ok
+        for which in "LU":
+            entries = len(f.factor(which)[1]) - s.n
+            assert entries <= f.level_entries(which) <= 3 * entries + s.n
+        f.close()
+    f = lina.ILU(s.rowptr, s.col, s.val, upload=False)
+    assert f.level_entries("L") == f.level_entries("U") == 0
+    f.close()
