@@ -81,10 +81,17 @@ bool wait_status(const double* status, int k, hipStream_t st) {
     const double* s = status + 4 * (k % 4);
     bool idle = false;
     for (long spin = 1;; spin++) {
-        double seen;
+        double seen, stop, again;
         __atomic_load(s, &seen, __ATOMIC_ACQUIRE);
-        // a later iteration in the slot: k did not stop the loop
-        if (seen >= (double)k) return seen == (double)k && s[2] != 0.0;
+        if (seen >= (double)k) {
+            // iteration k + 4 may be writing the slot: its flag comes before its
+            // number, so read both until the number has held still
+            __atomic_load(s + 2, &stop, __ATOMIC_ACQUIRE);
+            __atomic_load(s, &again, __ATOMIC_ACQUIRE);
+            if (again != seen) continue;
+            // a later iteration in the slot: k did not stop the loop
+            return seen == (double)k && stop != 0.0;
+        }
         if (idle) throw HipError("the loop test was not reported");
         if (spin % 4096) continue;
         const hipError_t e = hipStreamQuery(st);
