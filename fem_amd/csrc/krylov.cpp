@@ -758,7 +758,7 @@ int IluSystem::precon_dot(const double* R, double* Z, double* rz) {
 
 // pcg (PCGS.c:163-233) with precon = PCG_preconlr and mat_mult = PCG_mult.
 // The scalars stay on the device and the host only watches the loop test's
-// result in pinned memory, two iterations behind what it has queued (an
+// result in pinned memory, an iteration or two replays behind what it has queued (an
 // iteration queued after the stop leaves X and R untouched): an iteration of
 // the multicolour order is 7 triangular levels, direction, product and update,
 // where reading three dots back cost 11 more launches and copies and three
@@ -795,30 +795,42 @@ int IluSystem::pcg_core(double* X, double* B, double tol, int max_iter, int stop
         return dev::ipcg_xr(st, n, Y, R, P, Q, scal_, pq, folded(m, pq, dev::IS_PQ), rr);
     };
     auto later = [&]() { (void)finish(folded(precon_dot(R, Z, rz), rz, dev::IS_RZ), nrr, false); };
-    // long solves go on with replays of captured iterations (see Solver::pcg_dev)
-    constexpr int EAGER = 48, REPLAY = 8;
+    // Long solves go on with replays of captured iterations (see
+    // Solver::pcg_dev).  200 iterations, without -> with: wide levels, 66k rows
+    // 10.2 -> 8.2 ms, 526k 14.1 -> 13.7; one workgroup's sweeps, 4k rows 15.4 ->
+    // 14.7 ms, 9k 24.2 -> 23.5, 66k 139.1 -> 138.6, where one iteration replayed
+    // past the stop takes 0.7 ms (4.8 ms at 1.05M rows).
+    constexpr int EAGER = 48, REPLAY = 8, AHEAD = 16, FIRST = 32;
+    const bool replay = n <= (wide_ ? 1 << 20 : 1 << 14);
+    const int cap_iter = std::max(max_iter, 1);
+    LoopTrend trend(stop == LINA_STOP_RELRES ? tol : tol * r0);
     nrr = finish(folded(nrz, rz, dev::IS_RZ), 0, true);
     int queued = 0;
     for (int k = 1;; k++) {
-        while (queued < k + (queued >= EAGER ? 2 : 0)) {
-            if (queued < EAGER) {
+        for (;;) {
+            const double left = std::min(trend.left(), (double)(cap_iter - k)) - (queued - k);
+            if (replay && queued >= EAGER && queued < k + 2 && left > (iteration_.ready() ? AHEAD : FIRST)) {
+                if (Y != vXg_ || !vXg_) {  // captured iterations work on the system's own iterate
+                    if (!vXg_) vXg_ = kalloc<double>(n, *bufs_);
+                    dev::copy(st, n, (const double*)X, vXg_);
+                    Y = vXg_;
+                }
+                if (!iteration_.ready())
+                    iteration_.capture(st, [&]() {
+                        for (int q = 0; q < REPLAY; q++) later();
+                    });
+                iteration_.launch(st);
+                queued += REPLAY;
+            } else if (queued < k) {
                 later();
                 queued++;
-                continue;
+            } else {
+                break;
             }
-            if (Y != vXg_ || !vXg_) {  // captured iterations work on the system's own iterate
-                if (!vXg_) vXg_ = kalloc<double>(n, *bufs_);
-                dev::copy(st, n, (const double*)X, vXg_);
-                Y = vXg_;
-            }
-            if (!iteration_.ready())
-                iteration_.capture(st, [&]() {
-                    for (int q = 0; q < REPLAY; q++) later();
-                });
-            iteration_.launch(st);
-            queued += REPLAY;
         }
-        if (wait_status(status, k, st)) break;  // iteration k - 1's loop test
+        double norm;
+        if (wait_status(status, k, st, &norm)) break;  // iteration k - 1's loop test
+        trend.add(norm);
     }
     if (Y != X) dev::copy(st, n, (const double*)Y, X);
     // every preconditioner call queued after the stop was on the final R

@@ -77,18 +77,20 @@ void Captured::capture(hipStream_t st, const std::function<void()>& record) {
 
 void Captured::launch(hipStream_t st) const { hip_check(hipGraphLaunch(exec_, st), "graph launch"); }
 
-bool wait_status(const double* status, int k, hipStream_t st) {
+bool wait_status(const double* status, int k, hipStream_t st, double* r) {
     const double* s = status + 4 * (k % 4);
     bool idle = false;
     for (long spin = 1;; spin++) {
-        double seen, stop, again;
+        double seen, norm, stop, again;
         __atomic_load(s, &seen, __ATOMIC_ACQUIRE);
         if (seen >= (double)k) {
-            // iteration k + 4 may be writing the slot: its flag comes before its
-            // number, so read both until the number has held still
+            // iteration k + 4 may be writing the slot: its norm and flag come
+            // before its number, so read them until the number has held still
+            __atomic_load(s + 1, &norm, __ATOMIC_ACQUIRE);
             __atomic_load(s + 2, &stop, __ATOMIC_ACQUIRE);
             __atomic_load(s, &again, __ATOMIC_ACQUIRE);
             if (again != seen) continue;
+            *r = norm;
             // a later iteration in the slot: k did not stop the loop
             return seen == (double)k && stop != 0.0;
         }
@@ -99,6 +101,14 @@ bool wait_status(const double* status, int k, hipStream_t st) {
         hip_check(e, "loop test");
         idle = true;  // everything queued is done: one more look
     }
+}
+
+double LoopTrend::left() const {
+    if (n_ < W) return 0.0;
+    const double now = r_[(n_ - 1) % W], then = r_[n_ % W];
+    if (!(now > target_)) return 0.0;
+    if (!(now < then) || !(target_ > 0.0)) return 1e9;
+    return std::log(now / target_) * (W - 1) / std::log(then / now);
 }
 
 // ------------------------------------------------------------ memory
@@ -1933,37 +1943,49 @@ int Solver::pcg_dev(double* X, double* B, double tol, int max_iter, int stop, li
         // host takes 2.7 us a launch (3.9 with the sliced kernels' arguments),
         // the GPU 1.8 a node and about 20 us a graph, so that replays of one
         // iteration lose (257^2 Poisson, 37 iterations: 3.58 -> 3.88 ms) and
-        // those of several pay once a solve is long enough for the capture and
-        // for the iterations replayed past its end.  Not under kernel timing,
-        // whose events are the launch's own, nor for another operator's matrix.
-        constexpr int EAGER = 48, REPLAY = 4;
-        const bool replay = !op_ && !ktime_;
+        // those of several pay where launches bound an iteration: 200
+        // iterations, without -> with replays, 4k rows 18.4 -> 16.3 ms, 66k 22.6
+        // -> 20.9, 132k 47.4 -> 47.3, where the line is drawn.  An iteration
+        // replayed past the stop is a whole V-cycle (five of them: 5 % of a
+        // solve of 49), and a capture costs 0.5-0.9 ms, what 70-100 replayed
+        // iterations gain: both only when the last norms say that the solve
+        // goes on for longer.  Not under kernel timing, whose events are the
+        // launch's own, nor for another operator's matrix.
+        constexpr int EAGER = 48, REPLAY = 4, AHEAD = 16, FIRST = 96, ROWS = 1 << 17;
+        const bool replay = !op_ && !ktime_ && n <= ROWS;
+        LoopTrend trend(relres ? tol : tol * r0);
         finish(0, dev::dot_part<double>(st, n, R, Z, rz), true);
         int queued = 0;
         for (int k = 1;; k++) {
             // the test of iteration k - 1 comes in the middle of iteration k:
             // what follows can be queued then, but for a graph's latency
-            while (queued < k + (replay && queued >= EAGER ? 2 : 0)) {
-                if (!replay || queued < EAGER) {
+            for (;;) {
+                const bool ready = iteration_.ready() && same_cycle(iteration_prm_, prm_);
+                const double left = std::min(trend.left(), (double)(cap - k)) - (queued - k);
+                if (replay && queued >= EAGER && queued < k + 2 && left > (ready ? AHEAD : FIRST)) {
+                    if (Y != kX_) {  // captured iterations work on the solver's own iterate
+                        dev::copy(st, n, (const double*)Y, kX_);
+                        Y = kX_;
+                    }
+                    if (!ready) {
+                        iteration_.capture(st, [&]() {
+                            for (int q = 0; q < REPLAY; q++) later(0);
+                        });
+                        iteration_prm_ = prm_;
+                    }
+                    iteration_.launch(st);
+                    queued += REPLAY;
+                } else if (queued < k) {
                     later(++queued);
-                    continue;
+                } else {
+                    break;
                 }
-                if (Y != kX_) {  // captured iterations work on the solver's own iterate
-                    dev::copy(st, n, (const double*)Y, kX_);
-                    Y = kX_;
-                }
-                if (!(iteration_.ready() && same_cycle(iteration_prm_, prm_))) {
-                    iteration_.capture(st, [&]() {
-                        for (int q = 0; q < REPLAY; q++) later(0);
-                    });
-                    iteration_prm_ = prm_;
-                }
-                iteration_.launch(st);
-                queued += REPLAY;
             }
-            const bool stopped = wait_status(status, k, st);  // iteration k - 1's loop test
+            double norm;
+            const bool stopped = wait_status(status, k, st, &norm);  // iteration k - 1's loop test
             if (timed && sampled(k - 1)) sample(k - 1);
             if (stopped) break;
+            trend.add(norm);
         }
         // M^-1 of the final R and its norm come from the iteration that found
         // the stop; the reference's calls: one before the loop, one an

@@ -31,9 +31,29 @@ const char* last_error();
 
 // Waits for the report of iteration number k of a device-side loop (its kernels
 // on st write status[4 (k % 4) ...] in pinned memory, see dev::loop_test):
-// whether it stopped the loop.  Throws when st fails or runs out of work
-// without the report.
-bool wait_status(const double* status, int k, hipStream_t st);
+// whether it stopped the loop, and |R| of that iteration (or of a later one that
+// has taken the slot since).  Throws when st fails or runs out of work without
+// the report.
+bool wait_status(const double* status, int k, hipStream_t st, double* r);
+
+// The iterations that a Krylov loop seems to have left, from the norms of its
+// last residuals.  Only how work is queued depends on it, never a result.
+class LoopTrend {
+  public:
+    // target: the norm at which the loop stops
+    explicit LoopTrend(double target) : target_(target) {}
+    void add(double r) {
+        r_[n_ % W] = r;
+        n_++;
+    }
+    // at the mean rate of the last W norms; unlimited while they do not fall
+    double left() const;
+
+  private:
+    static constexpr int W = 16;
+    double target_, r_[W] = {};
+    long n_ = 0;
+};
 
 // A captured piece of a stream's work that is replayed while nothing it was
 // captured from changes (the owner resets it then).

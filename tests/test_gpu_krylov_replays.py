@@ -1,0 +1,163 @@
+"""Long pcg solves that go on with replays of captured iterations.
+
+A replay runs the kernels that the launched iterations run, on the same
+buffers, so whether and when a solve replays never changes a bit.  AMG-pcg is
+compared with a handle whose kernel timing is on (it never replays), ILU-pcg
+with a fresh handle at limits for which only an existing capture is replayed."""
+import time
+
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+from fem_amd import problems as P
+
+pytestmark = pytest.mark.gpu
+
+
+def isolate(s, rows):
+    """the system with `rows` coupled to nothing"""
+    keep = np.ones(s.n)
+    keep[rows] = 0.0
+    A = s.scipy().tocsr()
+    A = (sp.diags(keep) @ A @ sp.diags(keep) + sp.diags(2.0 * (1.0 - keep))).tocsr()
+    A.eliminate_zeros()
+    A.sort_indices()
+    return A
+
+
+def system(kind):
+    if kind == "isolated":
+        s = P.degraded_elasticity(49)
+        return isolate(s, np.arange(5, s.n, 97)), 2, 4
+    s, dof, depth = {"poisson": lambda: (P.poisson(65), 1, 4), "elastic": lambda: (P.degraded_elasticity(65), 2, 4)}[kind]()
+    return s.scipy().tocsr(), dof, depth
+
+
+def handles(gpu, A, prm):
+    """a handle that replays and one that does not"""
+    a, b = gpu.AMG(A.indptr, A.indices, A.data, prm), gpu.AMG(A.indptr, A.indices, A.data, prm)
+    b.kernel_timing(True)
+    return a, b
+
+
+def same(pair, b, **kw):
+    u, v = (h.pcg(b, stop="relres", **kw) for h in pair)
+    assert u["iters"] == v["iters"] and np.array_equal(u["x"], v["x"]) and u["residual"] == v["residual"]
+    assert u["vcycles"] == v["vcycles"] == u["iters"] + 2
+    return u
+
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+@pytest.mark.parametrize("kind", ["poisson", "elastic", "isolated"])
+def test_amg_replays_keep_the_bits(gpu, kind, prec):
+    print("amg replays", kind, prec, flush=True)
+    A, dof, depth = system(kind)
+    n = A.shape[0]
+    prm = gpu.params("vcycle", dof, depth, precision=prec)
+    pair = handles(gpu, A, prm)
+    b = np.random.default_rng(2).standard_normal(n)
+    # ends at limits: without a capture, at the first captures, inside and past replays
+    for limit in (47, 49, 60, 146, 147, 180, 181, 66, 67, 68, 69):
+        assert same(pair, b, tol=1e-300, max_iter=limit)["iters"] == limit
+    # ends at a tolerance, from another start
+    x0 = np.random.default_rng(3).standard_normal(n)
+    got = same(pair, b, x0=x0, tol=1e-8, max_iter=4000)
+    assert np.linalg.norm(A @ got["x"] - b) <= 1e-6 * np.linalg.norm(b)
+    # another right-hand side in the caller's device vectors
+    c = np.random.default_rng(4).standard_normal(n)
+    for limit in (150, 20):
+        want = pair[1].pcg(c, tol=1e-300, max_iter=limit, stop="relres")["x"]
+        x, d = gpu.DeviceVector(n), gpu.DeviceVector(n)
+        x.fill(0.0)
+        d.upload(c)
+        pair[0].pcg_device(x.ptr, d.ptr, tol=1e-300, max_iter=limit, stop="relres")
+        assert np.array_equal(x.download(), want)
+    for h in pair:
+        h.close()
+
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+def test_amg_replays_follow_values_and_parameters(gpu, prec):
+    A, dof, depth = system("elastic")
+    n = A.shape[0]
+    pair = handles(gpu, A, gpu.params("vcycle", dof, depth, precision=prec))
+    b = np.random.default_rng(5).standard_normal(n)
+    same(pair, b, tol=1e-300, max_iter=200)
+    new = A.copy()
+    new.data = 1.3 * A.data + 0.02 * A.data * (A.indices == np.repeat(np.arange(n), np.diff(A.indptr)))
+    for h in pair:
+        h.recompute(new.data)
+    got = same(pair, b, tol=1e-9, max_iter=4000)
+    assert np.linalg.norm(new @ got["x"] - b) <= 1e-7 * np.linalg.norm(b)
+    for kw in ({"precision": "mixed" if prec == "fp64" else "fp64"}, {"coarse_sweeps": 2}, {"smoother": 4}, {}):
+        prm = gpu.params("vcycle", dof, depth, **{"precision": prec, **kw})
+        for h in pair:
+            h.set_params(prm)
+        same(pair, b, tol=1e-300, max_iter=170)
+    d = gpu.DeviceVector(len(A.data))
+    d.upload(A.data)
+    for h in pair:
+        h.recompute_device(d.ptr)
+    same(pair, b, tol=1e-300, max_iter=170)
+    for h in pair:
+        h.close()
+
+
+@pytest.mark.parametrize("m", [33, 97])
+@pytest.mark.parametrize("ordering", ["multicolour", "natural"])
+def test_ilu_replays_keep_the_bits(gpu, m, ordering):
+    print("ilu replays", m, ordering, flush=True)
+    s = P.poisson(m)
+    A = s.scipy().tocsr()
+    b = np.random.default_rng(7).standard_normal(s.n)
+
+    def fresh(val=None):
+        f = gpu.ILU(s.rowptr, s.col, s.val, ordering=ordering)
+        if val is not None:
+            f.refactor(s.rowptr, s.col, val)
+        return f
+
+    f = fresh()
+    f.pcg(b, tol=1e-300, max_iter=400, stop="relres")  # captures
+    val = None
+    for step in range(2):
+        for limit in (49, 65, 66, 72, 79, 80):  # at most 32 iterations left at the first replay: a fresh handle launches
+            g = fresh(val)
+            u, v = (h.pcg(b, tol=1e-300, max_iter=limit, stop="relres") for h in (f, g))
+            g.close()
+            assert u["iters"] == v["iters"] == limit and np.array_equal(u["x"], v["x"])
+        # new values on the same handle
+        val = (1.0 + step) * s.val + 0.1 * (s.col == np.repeat(np.arange(s.n), np.diff(s.rowptr)))
+        f.refactor(s.rowptr, s.col, val)
+    A.data[:] = val
+    got = f.pcg(b, tol=1e-10, max_iter=2000, stop="relres")
+    assert np.linalg.norm(A @ got["x"] - b) <= 1e-8 * np.linalg.norm(b)
+    f.close()
+
+
+@pytest.mark.parametrize("solver", ["amg", "ilu"])
+def test_an_iteration_more_costs_an_iteration(gpu, solver):
+    """no replays past the end where an iteration takes long: 49 iterations
+    against 48 (a solve of 49 took 8 % and 16 % longer when they started there)"""
+    if solver == "amg":
+        s = P.poisson(513)
+        h = gpu.AMG(s.rowptr, s.col, s.val, gpu.params("vcycle", 1, 6, precision="mixed"))
+    else:
+        s = P.poisson(257)
+        h = gpu.ILU(s.rowptr, s.col, s.val)
+    b = np.random.default_rng(1).standard_normal(s.n)
+
+    def run(limit):
+        best = 1e9
+        for _ in range(9):
+            t = time.perf_counter()
+            h.pcg(b, tol=0.0, max_iter=limit, stop="relres")
+            best = min(best, time.perf_counter() - t)
+        return best
+
+    run(48)
+    t48, t49 = run(48), run(49)
+    h.close()
+    print(solver, "48: %.2f ms, 49: %.2f ms" % (t48 * 1e3, t49 * 1e3), flush=True)
+    assert t49 <= 1.05 * t48
