@@ -1174,7 +1174,8 @@ void Solver::refresh_after_recompute() {
     const auto t1 = std::chrono::steady_clock::now();
     bool vals = false;
     if (uploaded()) {
-        vals = refresh_values() && refresh_isolated();
+        vals = refresh_values();
+        vals = refresh_isolated() && vals;  // a full upload takes the isolated rows' divisors too
         if (!vals) {
             track_ = true;  // from now on upload() keeps what a values-only refresh compares
             upload();

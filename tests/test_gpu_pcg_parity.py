@@ -298,6 +298,35 @@ def test_recompute_values_only_upload(gpu, kind, prec):
     b.close()
 
 
+@pytest.mark.parametrize("kind,prec", [("reference", "fp64"), ("vcycle", "mixed")])
+def test_isolated_rows_follow_a_full_reupload(gpu, kind, prec):
+    """rows coupled to nothing start from f_i / a_ii (AMG_fix_isolated): with new
+    values whose coarse patterns change on the way, from the new a_ii.  Values
+    scaled by 2 leave the hierarchy's P and R, so that a fresh hierarchy gives
+    the same bits."""
+    import scipy.sparse as sp
+    s = P.degraded_elasticity(33)
+    keep = np.ones(s.n)
+    keep[5::97] = 0.0
+    A = (sp.diags(keep) @ s.scipy() @ sp.diags(keep) + sp.diags(3.0 * (1.0 - keep))).tocsr()
+    A.eliminate_zeros()
+    A.sort_indices()
+    mid = A.data.copy()
+    mid[np.flatnonzero(A.indices != np.repeat(np.arange(s.n), np.diff(A.indptr)))[::3]] = 0.0
+    prm = gpu.params(kind, 2, 3, precision=prec)
+    a = gpu.AMG(A.indptr, A.indices, A.data, prm)
+    a.recompute(mid)
+    a.recompute(2.0 * A.data)
+    b = gpu.AMG(A.indptr, A.indices, 2.0 * A.data, prm)
+    f = np.random.default_rng(2).standard_normal(s.n)
+    say("isolated rows", kind, prec)
+    ra, rb = (h.pcg(f, tol=1e-300, max_iter=3, stop="relres") for h in (a, b))
+    xa, xb = (h.amg_solve(f, np.zeros(s.n)) for h in (a, b))
+    a.close()
+    b.close()
+    assert np.array_equal(ra["x"], rb["x"]) and xa[0] == xb[0] and np.array_equal(xa[1], xb[1])
+
+
 @pytest.mark.parametrize("case", ["poisson17", "poisson33", "poisson33_std", "pair17"])
 def test_amg_solve_reference_jacobi_matches_golden(gpu, case):
     """The reference's undamped AMG_parallel_Jacobi_smoother
