@@ -522,16 +522,83 @@ __global__ __launch_bounds__(TPB) void k_slice_columns(int ns, int lt, SliceHead
     }
 }
 
+// put(q, value) for every place q of slice s, U loads in flight a lane; the
+// lanes past its rows put zeros; get(p): the CSR's entry p
+template <typename VT, typename G, typename F>
+__device__ __forceinline__ void slice_places(const Slices<VT>& S, int s, const int* __restrict__ rp, G&& get,
+                                             F&& put) {
+    using IT = decltype(get(0));
+    constexpr int U = 8;
+    const SliceLane L = slice_lane(S, s, rp);
+    const int steps = S.head[s].steps;
+    for (int j = 0; j < steps; j += U) {
+        IT a[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int e = (j + u) * L.T + L.t;
+            a[u] = e < L.len ? get(L.p0 + e) : (IT)0;
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (j + u < steps) put(L.base + (size_t)(j + u) * WAVE, a[u]);
+    }
+}
+
 template <typename VT>
 __global__ __launch_bounds__(TPB) void k_slice_values(const Slices<VT> S, const int* __restrict__ rp,
                                                       const VT* __restrict__ v, VT* __restrict__ out) {
     const int s = blockIdx.x * SLICES_PER_BLOCK + threadIdx.x / WAVE;
-    if (s >= S.ns) return;
-    const SliceLane L = slice_lane(S, s, rp);
-    const int steps = S.head[s].steps;
-    for (int j = 0; j < steps; j++) {
-        const int e = j * L.T + L.t;
-        out[L.base + (size_t)j * WAVE] = e < L.len ? v[L.p0 + e] : (VT)0;
+    if (s < S.ns) slice_places(S, s, rp, [&](int p) { return v[p]; }, [&](size_t q, VT a) { out[q] = a; });
+}
+
+// What a matrix's copies derive from FP64 values v, in one launch (a recompute
+// is little else on the small levels, at 2.6 us a launch): workgroups [0, b64)
+// the FP64 slices, with the FP32 slices where both have one layout, [b64, b64 +
+// b32) the FP32 slices of a layout of their own, the rest the CSR values (FP64
+// ones with a map).  map: entry p is v[map[p]].  l1: also the row sums of |v|
+// and |(float) v|, which a lane with a row of its own adds in row order.
+// Bytes bound it above 1M entries, launches below.  A recompute with gather,
+// conversion, two packings and two norms as launches -> with this (without
+// slices): Poisson 257^2 0.63 -> 0.57 ms (0.57), damage 513^2 0.64 -> 0.54 (0.52),
+// 1025^2 1.37 -> 1.25 (1.18), elasticity 129^2 2.13 -> 1.90 (1.95).
+__global__ __launch_bounds__(TPB) void k_pair_values(const Slices<double> S, const Slices<float> F, bool shared,
+                                                     const int* __restrict__ rp, const double* __restrict__ v,
+                                                     const int* __restrict__ map, int nnz, int b64, int b32,
+                                                     double* __restrict__ out, float* __restrict__ out32,
+                                                     double* __restrict__ v64, float* __restrict__ v32,
+                                                     double* __restrict__ l1, float* __restrict__ l132) {
+    const int wave = threadIdx.x / WAVE;
+    auto get = [&](int p) { return v[map ? map[p] : p]; };
+    int b = blockIdx.x;
+    if (b < b64) {
+        const int s = b * SLICES_PER_BLOCK + wave;
+        if (s >= S.ns) return;
+        double sum = 0;
+        float sum32 = 0;
+        slice_places(S, s, rp, get, [&](size_t q, double a) {
+            out[q] = a;
+            if (shared) out32[q] = (float)a;
+            sum += fabs(a);
+            sum32 += fabsf((float)a);
+        });
+        const int row = S.head[s].row0 + threadIdx.x % WAVE;
+        if (l1 && row < S.head[s].row1) {
+            l1[row] = sum;
+            l132[row] = sum32;
+        }
+        return;
+    }
+    b -= b64;
+    if (b < b32) {
+        const int s = b * SLICES_PER_BLOCK + wave;
+        if (s < F.ns) slice_places(F, s, rp, get, [&](size_t q, double a) { out32[q] = (float)a; });
+        return;
+    }
+    b -= b32;
+    for (int p = b * TPB + threadIdx.x; p < nnz; p += (gridDim.x - b64 - b32) * TPB) {
+        const double a = get(p);
+        v32[p] = (float)a;
+        if (map) v64[p] = a;
     }
 }
 
@@ -1902,12 +1969,19 @@ __global__ void k_plan_scatter(int ne, const double* __restrict__ val, const int
     }
 }
 
-template <typename VT>
-__global__ void k_row_l1(int n, const int* __restrict__ rp, const double* __restrict__ v, VT* __restrict__ out) {
+// row sums of |v| in FP64 and of |(float) v| in FP32, in row order
+__global__ void k_row_l1(int n, const int* __restrict__ rp, const double* __restrict__ v, double* __restrict__ out,
+                         float* __restrict__ out32) {
     for (int r = blockIdx.x * blockDim.x + threadIdx.x; r < n; r += gridDim.x * blockDim.x) {
-        VT s = 0;
-        for (int p = rp[r]; p < rp[r + 1]; p++) s += fabs((VT)v[p]);
+        double s = 0;
+        float f = 0;
+        for (int p = rp[r]; p < rp[r + 1]; p++) {
+            const double a = v[p];
+            s += fabs(a);
+            f += fabsf((float)a);
+        }
         out[r] = s;
+        out32[r] = f;
     }
 }
 
@@ -1916,6 +1990,15 @@ __global__ void k_gather(int n, const int* __restrict__ idx, const T* __restrict
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const int k = idx[i];
         dst[i] = k >= 0 ? src[k] : (T)0;
+    }
+}
+
+__global__ void k_gather2(int n, const int* __restrict__ idx, const double* __restrict__ src, double* __restrict__ dst,
+                          const float* __restrict__ src32, float* __restrict__ dst32) {
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+        const int k = idx[i];
+        dst[i] = src[k];
+        dst32[i] = src32[k];
     }
 }
 
@@ -2685,6 +2768,16 @@ void slice_values(hipStream_t st, const DMat<VT>& D) {
 template void slice_values<double>(hipStream_t, const DMat<double>&);
 template void slice_values<float>(hipStream_t, const DMat<float>&);
 
+bool pair_values(hipStream_t st, const DMat<double>& D, const DMat<float>& F, const double* from, const int* map) {
+    if (D.nnz <= 0) return false;
+    const bool shared = D.sl.ns > 0 && D.sl.head == F.sl.head, sums = D.sl.ns > 0 && D.sl.lt == 0;
+    const int b64 = slice_blocks(D.sl.ns), b32 = shared ? 0 : slice_blocks(F.sl.ns), bc = grid_for(D.nnz, 2048);
+    hipLaunchKernelGGL(k_pair_values, dim3(b64 + b32 + bc), dim3(TPB), 0, st, D.sl, F.sl, shared, D.rp,
+                       map ? from : D.v, map, D.nnz, b64, b32, D.sl.v, F.sl.v, D.v, F.v, sums ? D.l1 : nullptr,
+                       F.l1);
+    return sums;
+}
+
 // workgroups of a row-kernel launch: one per row block, or a persistent grid
 // of at most LINA_SPMV_GRID workgroups (rounded down to a multiple of 8; read
 // from the environment once, 0: off)
@@ -3346,19 +3439,19 @@ void negate_rows(hipStream_t st, int m, const int* rows, const int* rp, double* 
     if (m > 0) hipLaunchKernelGGL(k_negate_rows, dim3(std::min(m, 4096)), dim3(64), 0, st, m, rows, rp, v);
 }
 
-template <typename VT>
-void row_l1(hipStream_t st, int n, const int* rp, const double* v, VT* out) {
-    if (n > 0) hipLaunchKernelGGL((k_row_l1<VT>), dim3(grid_for(n)), dim3(TPB), 0, st, n, rp, v, out);
+void row_l1(hipStream_t st, int n, const int* rp, const double* v, double* out, float* out32) {
+    if (n > 0) hipLaunchKernelGGL(k_row_l1, dim3(grid_for(n)), dim3(TPB), 0, st, n, rp, v, out, out32);
 }
-template void row_l1<double>(hipStream_t, int, const int*, const double*, double*);
-template void row_l1<float>(hipStream_t, int, const int*, const double*, float*);
 
 template <typename T>
 void gather(hipStream_t st, int n, const int* idx, const T* src, T* dst) {
     if (n > 0) hipLaunchKernelGGL((k_gather<T>), dim3(grid_for(n)), dim3(TPB), 0, st, n, idx, src, dst);
 }
 template void gather<double>(hipStream_t, int, const int*, const double*, double*);
-template void gather<float>(hipStream_t, int, const int*, const float*, float*);
+
+void gather2(hipStream_t st, int n, const int* idx, const double* src, double* dst, const float* src32, float* dst32) {
+    if (n > 0) hipLaunchKernelGGL(k_gather2, dim3(grid_for(n)), dim3(TPB), 0, st, n, idx, src, dst, src32, dst32);
+}
 
 void scatter(hipStream_t st, int n, const int* idx, const double* src, double* dst) {
     if (n > 0) hipLaunchKernelGGL(k_scatter, dim3(grid_for(n)), dim3(TPB), 0, st, n, idx, src, dst);

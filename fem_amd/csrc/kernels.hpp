@@ -150,6 +150,12 @@ void slice_columns(hipStream_t st, const DMat<VT>& D);
 template <typename VT>
 void slice_values(hipStream_t st, const DMat<VT>& D);
 
+// everything that D's and its FP32 copy F's forms derive from D.v (after every
+// change of D.v): F's values and both sliced copies.  map: D.v[p] = from[map[p]]
+// first.  True when it also formed both l1 norms.
+bool pair_values(hipStream_t st, const DMat<double>& D, const DMat<float>& F, const double* from = nullptr,
+                 const int* map = nullptr);
+
 // the larger workgroup count of a row kernel over A's forms
 template <typename VT>
 inline int row_blocks(const DMat<VT>& A) {
@@ -493,12 +499,13 @@ void dirichlet_rows(hipStream_t st, int n, const int* rp, const int* ci, const u
                     double* val, double* b);
 // val = -val on the m listed rows
 void negate_rows(hipStream_t st, int m, const int* rows, const int* rp, double* v);
-// out[r] = sum_p |(VT) v[p]| over row r, in VT arithmetic and column order
-template <typename VT>
-void row_l1(hipStream_t st, int n, const int* rp, const double* v, VT* out);
+// out[r] = sum_p |v[p]| over row r in column order, out32[r] the same of (float) v[p] in FP32
+void row_l1(hipStream_t st, int n, const int* rp, const double* v, double* out, float* out32);
 // dst[i] = idx[i] >= 0 ? src[idx[i]] : 0
 template <typename T>
 void gather(hipStream_t st, int n, const int* idx, const T* src, T* dst);
+// the same for an FP64 and an FP32 array, every idx >= 0
+void gather2(hipStream_t st, int n, const int* idx, const double* src, double* dst, const float* src32, float* dst32);
 // dst[idx[i]] = src[i] where idx[i] >= 0
 void scatter(hipStream_t st, int n, const int* idx, const double* src, double* dst);
 

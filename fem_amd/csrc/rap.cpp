@@ -338,16 +338,10 @@ bool Solver::recompute_device_core() {
     // norms, the colour-permuted copies
     for (int l = 0; l < depth; l++) {
         DevLevel& d = L_[l];
-        dev::convert<double, float>(st, d.A.nnz, d.A.v, d.Af.v);
-        slice_pair(st, d.A, d.Af);
-        dev::row_l1<double>(st, d.n, d.A.rp, d.A.v, d.A.l1);
-        dev::row_l1<float>(st, d.n, d.A.rp, d.A.v, d.Af.l1);
+        if (!dev::pair_values(st, d.A, d.Af)) dev::row_l1(st, d.n, d.A.rp, d.A.v, d.A.l1, d.Af.l1);
         if (l == 0) continue;
-        dev::gather<double>(st, d.A.nnz, R.acmap[l], d.A.v, d.Ac.v);
-        dev::convert<double, float>(st, d.A.nnz, d.Ac.v, d.Acf.v);
-        slice_pair(st, d.Ac, d.Acf);
-        dev::gather<double>(st, d.n, d.perm, d.A.l1, d.Ac.l1);
-        dev::gather<float>(st, d.n, d.perm, d.Af.l1, d.Acf.l1);
+        if (!dev::pair_values(st, d.Ac, d.Acf, d.A.v, R.acmap[l]))
+            dev::gather2(st, d.n, d.perm, d.A.l1, d.Ac.l1, d.Af.l1, d.Acf.l1);
     }
     // the coarsest direct solve: the dense rows' matrix, inverted in place
     dev::fill<double>(st, nd_ * nd_, inv_, 0.0);

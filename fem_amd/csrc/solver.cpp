@@ -1230,8 +1230,7 @@ bool Solver::refresh_values() {
         const Csr& A = H_.lv[l].A;
         DevLevel& d = L_[l];
         put(d.A.v, A.v);
-        dev::convert<double, float>(st, d.A.nnz, d.A.v, d.Af.v);
-        slice_pair(st, d.A, d.Af);
+        dev::pair_values(st, d.A, d.Af);
         put(d.A.l1, row_l1<double>(A));
         putf(d.Af.l1, row_l1<float>(A));
         if (l == 0) continue;
@@ -1247,10 +1246,8 @@ bool Solver::refresh_values() {
         }
         put(d.Ac.l1, row_l1<double>(Ac));
         putf(d.Acf.l1, row_l1<float>(Ac));
-        const int nnz = (int)Ac.v.size();
         put(d.Ac.v, std::move(Ac.v));
-        dev::convert<double, float>(st, nnz, d.Ac.v, d.Acf.v);
-        slice_pair(st, d.Ac, d.Acf);
+        dev::pair_values(st, d.Ac, d.Acf);
         if (d.sor_packed) {
             hip_check(hipStreamSynchronize(st), "sync");
             build_sor_packs(l, *bufs_, true);  // the packs hold values: rewritten in place
@@ -2162,8 +2159,7 @@ bool DevMatrix::update_values(const Csr& A0) {
     const Csr A = drop_outside_zeros(A0);
     if (A.nnz() != A_.nnz) return false;
     hip_check(hipMemcpyAsync(A_.v, A.v.data(), A.v.size() * sizeof(double), hipMemcpyHostToDevice, stream_), "h2d");
-    dev::convert<double, float>(stream_, A_.nnz, A_.v, Af_.v);
-    slice_pair(stream_, A_, Af_);
+    dev::pair_values(stream_, A_, Af_);
     hip_check(hipStreamSynchronize(stream_), "update");
     return true;
 }
@@ -2171,8 +2167,7 @@ bool DevMatrix::update_values(const Csr& A0) {
 bool DevMatrix::update_values_device(const double* d_val, long nnz) {
     if (nnz != (long)A_.nnz || nnz_ != nnz) return false;
     hip_check(hipMemcpyAsync(A_.v, d_val, nnz * sizeof(double), hipMemcpyDeviceToDevice, stream_), "d2d");
-    dev::convert<double, float>(stream_, A_.nnz, A_.v, Af_.v);
-    slice_pair(stream_, A_, Af_);
+    dev::pair_values(stream_, A_, Af_);
     hip_check(hipStreamSynchronize(stream_), "update");
     return true;
 }

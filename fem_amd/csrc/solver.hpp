@@ -173,11 +173,6 @@ std::vector<dev::SliceHead> slice_layout(const Csr& A, const int* colours, bool 
                                          int* lt, size_t* steps);
 // a sliced copy of D (CSR of A uploaded) where worthwhile; false: none
 bool slice_matrix(const Csr& A, dev::DMat<double>& D, DevBuffers& B, hipStream_t st);
-// both precisions' sliced values from their CSR values
-inline void slice_pair(hipStream_t st, const dev::DMat<double>& D, const dev::DMat<float>& F) {
-    dev::slice_values<double>(st, D);
-    dev::slice_values<float>(st, F);
-}
 void build_blocks(const Csr& A, int begin, int end, int max_nnz, std::vector<int>& starts,
                   int max_rows = dev::BLOCK_ROWS);
 std::vector<int2> block_pairs(const Csr& A, const std::vector<int>& starts_with_end);

@@ -135,3 +135,37 @@ def test_operator_with_longer_rows_than_the_hierarchy(gpu, irregular):
     op.close()
     amg.close()
     assert np.linalg.norm(A @ got["x"] - b) <= 1e-8 * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("kind,coarsening", [("damage", 1), ("damage", 2), ("elastic", 1), ("elastic", 2)])
+@pytest.mark.parametrize("smoother,coarse", [("mc_ssor", "l1_jacobi"), ("jacobi", "mc_sor"), ("l1_jacobi", "mc_ssor")])
+def test_recomputed_copies_are_those_of_a_fresh_upload(gpu, kind, coarsening, smoother, coarse):
+    """every copy that a device recompute rewrites (both precisions' values,
+    slices, colour order, l1 norms) against a hierarchy that reaches the same
+    values through full uploads (its pattern changes on the way)"""
+    from fem_amd import problems as P
+    s = P.damage_system(129)[0] if kind == "damage" else P.degraded_elasticity(65)
+    row = np.repeat(np.arange(s.n), np.diff(s.rowptr))
+    scale = 1.0 + 0.1 * np.random.default_rng(3).random(s.n)
+    new = s.val * scale[row] * scale[s.col]
+    mid = new.copy()
+    mid[np.flatnonzero(s.col != row)[::3]] = 0.0
+    kw = dict(smoother=smoother, coarse_smoother=coarse, coarsening=coarsening)
+    prm = {p: gpu.params("vcycle", s.dof, 4, precision=p, **kw) for p in ("fp64", "mixed")}
+    a, b = (gpu.AMG(s.rowptr, s.col, s.val, prm["fp64"]) for _ in range(2))
+    a.recompute(new)
+    b.recompute(mid)
+    b.recompute(new)
+    rng = np.random.default_rng(4)
+    for l in range(a.depth):
+        assert np.array_equal(a.level(l)["A"][2], b.level(l)["A"][2])
+        x = rng.standard_normal(a.level_sizes(l)["fine"])
+        for p in prm:
+            assert np.array_equal(a.spmv(x, l, p), b.spmv(x, l, p)), (l, p)
+    for p in ("fp64", "mixed", "fp64"):
+        for h in (a, b):
+            h.set_params(prm[p])
+        u, v = (h.pcg(s.b, tol=1e-300, max_iter=5, stop="relres") for h in (a, b))
+        assert np.array_equal(u["x"], v["x"]), p
+    a.close()
+    b.close()
