@@ -321,6 +321,36 @@ SlicePlan plan_slices(const Csr& A, const std::vector<int>& groups, bool free_or
     return p;
 }
 
+// Whether the row kernels take a matrix faster from slices than from row
+// blocks, by launch (a group each), in us.  A slice is a chain of its longest
+// row's steps, 8 in flight; row blocks spread a long row over a workgroup.
+// Measured (blocks, slices; FP32): 116k entries, 50 steps, 4.9, 6.9; 248k, 108,
+// 7.7, 12.4; 638k, 407, 16.2, 37.1; 1.5M, 148, 11.3, 15.6; the other side 506k,
+// 26 steps, 8.5, 4.9; 986k, 65, 12.1, 8.2.  FP64 streams of long rows are a
+// little faster in blocks: 6.4M entries in rows of 95, 17.0, 19.5; 39M, 159,
+// 82, 97; but 1.7M, 95, 14.8, 7.1 and 7.8M, 53, 19.2, 19.6.
+static bool slices_pay(const Csr& A, const SlicePlan& p, bool fp64) {
+    double slices = 0, blocks = 0;
+    for (size_t g = 0; g + 1 < p.group.size(); g++) {
+        int steps = 0;
+        double ent = 0;
+        for (int k = p.group[g]; k < p.group[g + 1]; k++) {
+            steps = std::max(steps, p.head[k].steps);
+            ent += A.rp[p.head[k].row1] - A.rp[p.head[k].row0];
+        }
+        slices += 2.0 + 0.72 * ((steps + 7) / 8);
+        blocks += 4.0 + std::min(ent / 1e5, 8.0);
+    }
+    if (slices > blocks) return false;
+    return !(fp64 && A.nnz() >= 4000000 && A.nnz() >= 90.0 * A.n);
+}
+
+// the slices of a matrix's copy by the rules, or none
+static SlicePlan rule_slices(const Csr& A, const std::vector<int>& groups, bool free_order, bool fp64) {
+    SlicePlan p = plan_slices(A, groups, free_order);
+    return slices_pay(A, p, fp64) ? p : SlicePlan();
+}
+
 static bool same_rows(const SlicePlan& a, const SlicePlan& b) {
     auto eq = [](const dev::SliceHead& x, const dev::SliceHead& y) {
         return x.row0 == y.row0 && x.row1 == y.row1 && x.step0 == y.step0 && x.steps == y.steps;
@@ -392,7 +422,7 @@ static void make_slices(const SlicePlan& p, dev::DMat<VT>& D, DevBuffers& B, hip
 
 // slices of a matrix without groups and systems (krylov.cpp's operators)
 bool slice_matrix(const Csr& A, dev::DMat<double>& D, DevBuffers& B, hipStream_t st) {
-    const SlicePlan p = plan_slices(A, {}, false);  // the ILU's Krylov loops take no partials from it
+    const SlicePlan p = rule_slices(A, {}, false, true);  // the ILU's Krylov loops take no partials from it
     make_slices<double, double>(p, D, B, st, nullptr);
     return D.sl.ns > 0;
 }
@@ -496,8 +526,8 @@ struct PairPlan {
 static PairPlan plan_pair(const Csr& A, bool batch, bool free32, bool partials) {
     PairPlan q;
     // the FP64 finest matrix (partials) keeps a row's column order
-    q.p64 = plan_slices(A, {}, !partials);
-    q.p32 = plan_slices(A, {}, free32);
+    q.p64 = rule_slices(A, {}, !partials, true);
+    q.p32 = rule_slices(A, {}, free32, false);
     if (partials && !free32 && !batch && !q.p64.head.empty() && q.p64.lt == 0) {
         // slices by row block where they fill their wavefronts (1.05M rows x
         // 7: 256-row blocks), else the block form beside them (2.1M x 14, 146
@@ -558,8 +588,8 @@ static Csr colour_permuted(const Csr& A, const std::vector<int>& col, int nc, st
 // the slices of a colour-permuted copy's two precisions
 static PairPlan plan_colours(const Csr& Ac, const std::vector<int>& rows, bool free32) {
     PairPlan q;
-    q.p64 = plan_slices(Ac, rows, true);
-    q.p32 = plan_slices(Ac, rows, free32);
+    q.p64 = rule_slices(Ac, rows, true, true);
+    q.p32 = rule_slices(Ac, rows, free32, false);
     q.shared = same_rows(q.p64, q.p32);
     return q;
 }

@@ -48,14 +48,15 @@ def lengths_of(kind, seed):
         m = np.ones(256 * 20 - 50, np.int64)
         first = 256 * rng.integers(1, 8) + rng.integers(50, 64)
         m[first:first + 12] = 4
-    else:  # P1 mesh rows in blocks of 2,048 entries, two hubs
+    else:  # P1 mesh rows in blocks of 2,048 entries, two patches of longer rows
         m = np.full(256 * 2500 - 63, 7)
-        m[rng.integers(0, 400_000, 2)] = 256 + 28
+        for first in rng.integers(0, 400_000, 2):
+            m[first - first % 256 + 100:first - first % 256 + 120] = 21
     return m
 
 
 @pytest.mark.parametrize("seed", range(8))
-@pytest.mark.parametrize("kind", ["short", "patch", "hubs"])
+@pytest.mark.parametrize("kind", ["short", "patch", "mesh"])
 def test_copies_of_a_finest_matrix_are_stored_as_they_are_read(kind, seed):
     m = lengths_of(kind, seed)
     rp, ci = rows_with(m, seed)
@@ -82,7 +83,7 @@ def test_layouts_over_row_counts_and_lengths(n, mean, free32, partials):
 
 
 @pytest.mark.parametrize("free32", [True, False])
-@pytest.mark.parametrize("clique,sliced", [(40, True), (700, False)])
+@pytest.mark.parametrize("clique,sliced", [(8, True), (700, False)])
 def test_small_colours_of_long_rows_do_not_fill_memory(clique, sliced, free32):
     """a clique's rows have a colour each: a slice of one row stores 64 / lanes
     times the row"""
@@ -97,3 +98,22 @@ def test_small_colours_of_long_rows_do_not_fill_memory(clique, sliced, free32):
         assert (len(heads) > 0) == sliced
         assert 64 * steps <= 4 * len(ci) + 2 ** 20
         check_layout(np.append(0, np.cumsum(m[np.argsort(colours, kind="stable")])), heads, lanes, steps)
+
+
+@pytest.mark.parametrize("n,mean,longest,sliced", [
+    (1200, 90, 90, True), (1200, 90, 800, False), (8000, 80, 3200, False), (9400, 104, 1000, True),
+    (40_000, 7, 40, True), (40_000, 7, 300, False), (3000, 16, 16, True)])
+def test_a_few_long_rows_take_row_blocks(n, mean, longest, sliced):
+    """a slice runs its longest row's steps one after another"""
+    m = np.full(n, mean)
+    m[n // 3] = longest
+    rp, ci = rows_with(m, n)
+    for precision in ("fp64", "mixed"):
+        assert (len(lina.slice_layout(rp, ci, precision=precision)[0]) > 0) == sliced
+
+
+@pytest.mark.parametrize("n,mean,sliced64", [(70_000, 95, False), (18_000, 95, True), (120_000, 53, True)])
+def test_large_fp64_matrices_of_long_rows_take_row_blocks(n, mean, sliced64):
+    rp, ci = rows_with(np.full(n, mean), n)
+    assert (len(lina.slice_layout(rp, ci, precision="fp64")[0]) > 0) == sliced64
+    assert len(lina.slice_layout(rp, ci, precision="mixed")[0]) > 0
