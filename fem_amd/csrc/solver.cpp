@@ -267,22 +267,36 @@ struct SlicePlan {
     size_t steps = 0;
 };
 
-SlicePlan plan_slices(const Csr& A, const std::vector<int>& groups, bool free_order,
-                      const std::vector<int>* blocks = nullptr) {
-    SlicePlan p;
-    const long nnz = A.nnz();
-    if (A.n == 0 || nnz == 0) return p;
-    const double mean = (double)nnz / A.n;
+static int log2_of(int lanes) {
+    int t = 0;
+    while ((1 << t) < lanes) t++;
+    return t;
+}
+
+static int slice_lanes(const Csr& A, const std::vector<int>& groups, bool free_order) {
+    if (A.n == 0) return 0;
+    const double mean = (double)A.nnz() / A.n;
+    int lt = 0;
     if (free_order) {
         const double waves = (double)A.n / std::max((int)groups.size() - 1, 1) / 64;
-        auto more = [&]() { p.lt = p.lt == 0 ? 2 : p.lt + 1; };  // 1, 4, 8, 16 as in the block form
+        auto more = [&]() { lt = lt == 0 ? 2 : lt + 1; };  // 1, 4, 8, 16 as in the block form
         if (mean > 24)
-            while (p.lt < 4 && waves * (1 << p.lt) < 4096 && mean >= (p.lt == 0 ? 24 : 6 << (p.lt + 1))) more();
+            while (lt < 4 && waves * (1 << lt) < 4096 && mean >= (lt == 0 ? 24 : 6 << (lt + 1))) more();
         else if (waves < 1024 && mean >= 12)
             more();
     } else {
-        while ((1 << p.lt) < dev::lanes_per_row(mean)) p.lt++;
+        while ((1 << lt) < dev::lanes_per_row(mean)) lt++;
     }
+    return lt;
+}
+
+// lt: log2 of the lanes a row
+static SlicePlan plan_slices(const Csr& A, const std::vector<int>& groups, int lt,
+                             const std::vector<int>* blocks = nullptr) {
+    SlicePlan p;
+    p.lt = lt;
+    const long nnz = A.nnz();
+    if (A.n == 0 || nnz == 0) return p;
     const std::vector<int> whole = {0, A.n};
     const bool per_block = blocks && p.lt == 0;
     const std::vector<int>& g = per_block ? *blocks : groups.empty() ? whole : groups;
@@ -347,7 +361,7 @@ static bool slices_pay(const Csr& A, const SlicePlan& p, bool fp64) {
 
 // the slices of a matrix's copy by the rules, or none
 static SlicePlan rule_slices(const Csr& A, const std::vector<int>& groups, bool free_order, bool fp64) {
-    SlicePlan p = plan_slices(A, groups, free_order);
+    SlicePlan p = plan_slices(A, groups, slice_lanes(A, groups, free_order));
     return slices_pay(A, p, fp64) ? p : SlicePlan();
 }
 
@@ -522,18 +536,24 @@ struct PairPlan {
 
 // free32: the FP32 rows may be summed in any order (see Solver::fixed_order);
 // partials: the FP64 product's block partials are summed by a Krylov method
-// (its row order is kept then, and its partials' too without free32)
-static PairPlan plan_pair(const Csr& A, bool batch, bool free32, bool partials) {
+// (its row order is kept then, and its partials' too without free32); tuned:
+// the autotuner's lanes
+static PairPlan plan_pair(const Csr& A, bool batch, bool free32, bool partials, const TunedLanes* tuned = nullptr) {
     PairPlan q;
     // the FP64 finest matrix (partials) keeps a row's column order
-    q.p64 = rule_slices(A, {}, !partials, true);
-    q.p32 = rule_slices(A, {}, free32, false);
+    if (!tuned) {
+        q.p64 = rule_slices(A, {}, !partials, true);
+        q.p32 = rule_slices(A, {}, free32, false);
+    } else {
+        if (tuned->s64) q.p64 = plan_slices(A, {}, log2_of(tuned->l64));
+        if (tuned->s32) q.p32 = plan_slices(A, {}, log2_of(tuned->l32));
+    }
     if (partials && !free32 && !batch && !q.p64.head.empty() && q.p64.lt == 0) {
         // slices by row block where they fill their wavefronts (1.05M rows x
         // 7: 256-row blocks), else the block form beside them (2.1M x 14, 146
         // rows a block: 76 us, 87 us as slices of 64, 64 and 18 rows)
         q.s64 = schedule<double>(A);
-        SlicePlan b = plan_slices(A, {}, false, &q.s64);
+        SlicePlan b = plan_slices(A, {}, 0, &q.s64);
         if (!b.head.empty() && A.n >= 0.9 * 64 * b.head.size()) {
             q.p64 = std::move(b);
             q.s64.clear();
@@ -551,11 +571,15 @@ static PairPlan plan_pair(const Csr& A, bool batch, bool free32, bool partials) 
 // plan_pair); returns the largest workgroup count of a row kernel over either
 // copy in either form
 int upload_pair(const Csr& A0, dev::DMat<double>& D, dev::DMat<float>& F, DevBuffers& B, hipStream_t st,
-                const std::vector<int>* seg, bool free32, bool partials) {
+                const std::vector<int>* seg, bool free32, bool partials, const TunedLanes* tuned) {
     Csr A = drop_outside_zeros(A0);
-    const PairPlan q = plan_pair(A, seg != nullptr, free32, partials);
+    const PairPlan q = plan_pair(A, seg != nullptr, free32, partials, tuned);
     upload_mat<double, double>(A, q.p64, q.s64, D, B, st, nullptr, false, nullptr, nullptr, seg);
     upload_mat(A, q.p32, q.s32, F, B, st, &D, q.shared, &q.s64, nullptr, seg);
+    if (tuned) {
+        if (!D.sl.ns) D.lpr = tuned->l64;
+        if (!F.sl.ns) F.lpr = tuned->l32;
+    }
     const int blocks = std::max((int)schedule<double>(A).size(), (int)schedule<float>(A).size()) - 1;
     return std::max({dev::row_blocks(D), dev::row_blocks(F), blocks});
 }
@@ -586,10 +610,16 @@ static Csr colour_permuted(const Csr& A, const std::vector<int>& col, int nc, st
 }
 
 // the slices of a colour-permuted copy's two precisions
-static PairPlan plan_colours(const Csr& Ac, const std::vector<int>& rows, bool free32) {
+static PairPlan plan_colours(const Csr& Ac, const std::vector<int>& rows, bool free32,
+                             const TunedLanes* tuned = nullptr) {
     PairPlan q;
-    q.p64 = rule_slices(Ac, rows, true, true);
-    q.p32 = rule_slices(Ac, rows, free32, false);
+    if (!tuned) {
+        q.p64 = rule_slices(Ac, rows, true, true);
+        q.p32 = rule_slices(Ac, rows, free32, false);
+    } else {
+        if (tuned->s64) q.p64 = plan_slices(Ac, rows, log2_of(tuned->l64));
+        if (tuned->s32) q.p32 = plan_slices(Ac, rows, log2_of(tuned->l32));
+    }
     q.shared = same_rows(q.p64, q.p32);
     return q;
 }
@@ -670,6 +700,7 @@ void Solver::setup_host(const Csr& A, const lina_amg_params& p) {
     sp.eps_plus = p.eps_plus;
     sp.matrix_tol = p.matrix_tol;
     amg_setup(A, sp, H_);
+    tuned_.clear();
     n_ = A.n;
     colours_.assign(H_.lv.size(), std::vector<int>());
     ncolours_.assign(H_.lv.size(), 0);
@@ -679,89 +710,136 @@ void Solver::setup_host(const Csr& A, const lina_amg_params& p) {
 // ------------------------------------------------------- autotuning
 
 namespace {
-constexpr int kLprCandidates[] = {1, 4, 8, 16, 32};
+constexpr int kLaneCandidates[] = {1, 4, 8, 16, 32};
 }
 
-template <typename VT, typename XT>
-int Solver::tune_spmv(dev::DMat<VT>& M, const XT* x, XT* y) {
-    if (M.n == 0 || M.sl.ns) return M.lpr;  // slices: their lanes follow from the plan
-    float best = 1e30f;
-    int best_lpr = M.lpr;
-    for (int lpr : kLprCandidates) {
-        M.lpr = lpr;
-        dev::spmv<VT, XT>(stream_, M, x, nullptr, y, dev::MODE_SET, nullptr, nullptr);
-        hip_check(hipEventRecord(ev0_, stream_), "event");
-        for (int k = 0; k < 3; k++) dev::spmv<VT, XT>(stream_, M, x, nullptr, y, dev::MODE_SET, nullptr, nullptr);
-        hip_check(hipEventRecord(ev1_, stream_), "event");
-        hip_check(hipEventSynchronize(ev1_), "event sync");
-        float ms = 0;
-        hip_check(hipEventElapsedTime(&ms, ev0_, ev1_), "elapsed");
-        if (ms < best) {
-            best = ms;
-            best_lpr = lpr;
+// The form of M (rows: A's) whose launches are fastest: a sliced copy with each
+// lane count, laid out in scratch memory, and the row blocks with each where M
+// has them.  groups: a colour-permuted copy's (offsets: its sweep's offsets of
+// slices or blocks).  What M has stays unless another is 3 % faster.
+template <typename VT>
+Solver::Form Solver::tune_form(const Csr& A, const std::vector<int>& groups, const dev::DMat<VT>& M,
+                               const std::vector<int>& offsets,
+                               const std::function<void(const dev::DMat<VT>&, const std::vector<int>&)>& run) {
+    const Form have = {M.sl.ns ? 1 << M.sl.lt : M.lpr, M.sl.ns > 0};
+    if (M.n == 0 || M.nnz == 0) return have;
+    auto timed = [&](const dev::DMat<VT>& T, const std::vector<int>& off) {
+        run(T, off);
+        float t = 1e30f;
+        for (int rep = 0; rep < 2; rep++) {
+            hip_check(hipEventRecord(ev0_, stream_), "event");
+            for (int k = 0; k < 3; k++) run(T, off);
+            hip_check(hipEventRecord(ev1_, stream_), "event");
+            hip_check(hipEventSynchronize(ev1_), "event sync");
+            float ms = 0;
+            hip_check(hipEventElapsedTime(&ms, ev0_, ev1_), "elapsed");
+            t = std::min(t, ms);
         }
-    }
-    M.lpr = best_lpr;
-    return best_lpr;
-}
-
-template <typename VT, typename XT>
-int Solver::tune_mcsor(DevLevel& d, dev::DMat<VT>& Ac, const XT* f, XT* x) {
-    if (Ac.n == 0 || d.ncolours == 0 || Ac.sl.ns) return Ac.lpr;
-    float best = 1e30f;
-    int best_lpr = Ac.lpr;
-    const std::vector<int>& cb = sizeof(VT) == 8 ? d.colour_blk : d.colour_blk32;
-    auto sweep = [&]() {
-        for (int c = 0; c < d.ncolours; c++)
-            dev::mcsor_colour(stream_, Ac, cb[c], cb[c + 1] - cb[c], d.perm, f, x, (XT)1);
+        return t;
     };
-    for (int lpr : kLprCandidates) {
-        Ac.lpr = lpr;
-        sweep();
-        hip_check(hipEventRecord(ev0_, stream_), "event");
-        for (int k = 0; k < 2; k++) sweep();
-        hip_check(hipEventRecord(ev1_, stream_), "event");
-        hip_check(hipEventSynchronize(ev1_), "event sync");
-        float ms = 0;
-        hip_check(hipEventElapsedTime(&ms, ev0_, ev1_), "elapsed");
-        if (ms < best) {
-            best = ms;
-            best_lpr = lpr;
+    Form best = have;
+    float best_t = 0.97f * timed(M, offsets);
+    auto keep = [&](float t, Form f) {
+        if (t < best_t) {
+            best_t = t;
+            best = f;
         }
+    };
+    for (int lanes : kLaneCandidates) {
+        if (!have.sliced && lanes != have.lanes) {
+            dev::DMat<VT> T = M;
+            T.lpr = lanes;
+            keep(timed(T, offsets), {lanes, false});
+        }
+        if (have.sliced && lanes == have.lanes) continue;
+        const SlicePlan p = plan_slices(A, groups, log2_of(lanes));
+        if (p.head.empty()) continue;
+        validate(A, p);
+        DevBuffers scratch;
+        dev::DMat<VT> T = M;
+        T.bspec = nullptr;
+        make_slices<VT, VT>(p, T, scratch, stream_, nullptr);
+        keep(timed(T, p.group), {lanes, true});
+        hip_check(hipStreamSynchronize(stream_), "autotune");  // the scratch slices die here
     }
-    Ac.lpr = best_lpr;
-    return best_lpr;
+    return best;
 }
 
-// The row partition (lanes per row in the LDS reduction phase) of every
-// matrix of the hierarchy, chosen by timing each candidate on the device:
-// the SpMV-shaped kernels (residual, restriction, prolongation, Jacobi) take
-// their matrix's choice, the multicolour sweeps the colour-permuted copy's.
-void Solver::autotune() {
+// The row partition (slices or row blocks, lanes per row) of every matrix of the
+// hierarchy, chosen by timing each candidate on the device: the SpMV-shaped kernels (residual,
+// restriction, prolongation, Jacobi) take their matrix's choice, the
+// multicolour sweeps the colour-permuted copy's.  True when a matrix should
+// have another than it has.
+bool Solver::autotune() {
     hipStream_t st = stream_;
     tuned_.clear();
+    bool other = false;
+    auto differs = [](const auto& M, Form f) {
+        return f.sliced != (M.sl.ns > 0) || f.lanes != (M.sl.ns ? 1 << M.sl.lt : M.lpr);
+    };
+    auto note = [&](int l, char which, const dev::DMat<double>& D, const dev::DMat<float>& F, Form a, Form b) {
+        tuned_.push_back({l, which, a.lanes, b.lanes, a.sliced, b.sliced});
+        other = other || differs(D, a) || differs(F, b);
+    };
+    auto product = [&](int l, char which, const Csr& M0, const dev::DMat<double>& D, const dev::DMat<float>& F,
+                       const double* x, double* y, const float* xf, float* yf) {
+        const Csr M = which == 'A' ? Csr() : drop_outside_zeros(M0);  // A has none
+        const Csr& A = which == 'A' ? M0 : M;
+        const Form a = tune_form<double>(A, {}, D, {}, [&](const dev::DMat<double>& T, const std::vector<int>&) {
+            dev::spmv<double, double>(st, T, x, nullptr, y, dev::MODE_SET, nullptr, nullptr);
+        });
+        const Form b = tune_form<float>(A, {}, F, {}, [&](const dev::DMat<float>& T, const std::vector<int>&) {
+            dev::spmv<float, float>(st, T, xf, nullptr, yf, dev::MODE_SET, nullptr, nullptr);
+        });
+        note(l, which, D, F, a, b);
+    };
     for (size_t l = 0; l < L_.size(); l++) {
         DevLevel& d = L_[l];
+        const HostLevel& h = H_.lv[l];
         for (double* v : {d.x, d.f, d.r, d.xo}) dev::fill<double>(st, d.n, v, 1.0);
         for (float* v : {d.xf, d.ff, d.rf, d.xof}) dev::fill<float>(st, d.n, v, 1.0f);
-        tuned_.push_back({(int)l, 'A', tune_spmv<double, double>(d.A, d.x, d.r), tune_spmv<float, float>(d.Af, d.xf, d.rf)});
+        product((int)l, 'A', h.A, d.A, d.Af, d.x, d.r, d.xf, d.rf);
         if (l == 0) continue;
         DevLevel& c = L_[l - 1];
         for (double* v : {c.x, c.f}) dev::fill<double>(st, c.n, v, 1.0);
         for (float* v : {c.xf, c.ff}) dev::fill<float>(st, c.n, v, 1.0f);
-        tuned_.push_back({(int)l, 'P', tune_spmv<double, double>(d.P, c.x, d.r), tune_spmv<float, float>(d.Pf, c.xf, d.rf)});
-        tuned_.push_back({(int)l, 'R', tune_spmv<double, double>(d.R, d.r, c.f), tune_spmv<float, float>(d.Rf, d.rf, c.ff)});
+        product((int)l, 'P', h.P, d.P, d.Pf, c.x, d.r, c.xf, d.rf);
+        product((int)l, 'R', h.R, d.R, d.Rf, d.r, c.f, d.rf, c.ff);
         dev::fill<double>(st, d.n, d.f, 0.0);
         dev::fill<float>(st, d.n, d.ff, 0.0f);
-        tuned_.push_back({(int)l, 'C', tune_mcsor<double, double>(d, d.Ac, d.f, d.x),
-                          tune_mcsor<float, float>(d, d.Acf, d.ff, d.xf)});
+        if (d.ncolours == 0) continue;
+        std::vector<int> perm, rows;
+        const Csr Ac = colour_permuted(h.A, colours_[l], ncolours_[l], perm, rows);
+        const Form a = tune_form<double>(Ac, rows, d.Ac, d.colour_blk,
+                                         [&](const dev::DMat<double>& T, const std::vector<int>& cb) {
+            for (int c = 0; c < d.ncolours; c++)
+                dev::mcsor_colour(st, T, cb[c], cb[c + 1] - cb[c], d.perm, (const double*)d.f, d.x, 1.0);
+        });
+        const Form b = tune_form<float>(Ac, rows, d.Acf, d.colour_blk32,
+                                        [&](const dev::DMat<float>& T, const std::vector<int>& cb) {
+            for (int c = 0; c < d.ncolours; c++)
+                dev::mcsor_colour(st, T, cb[c], cb[c + 1] - cb[c], d.perm, (const float*)d.ff, d.xf, 1.0f);
+        });
+        note((int)l, 'C', d.Ac, d.Acf, a, b);
     }
     hip_check(hipStreamSynchronize(st), "autotune");
+    return other;
+}
+
+// the autotuner's lanes of a matrix, or nullptr before it has run
+const TunedLanes* Solver::tuned_lanes(int l, char which, TunedLanes& t) const {
+    for (const Tuned& q : tuned_)
+        if (q.level == l && q.which == which) {
+            t = {q.lpr64, q.lpr32, q.s64, q.s32};
+            return &t;
+        }
+    return nullptr;
 }
 
 void Solver::set_hierarchy(HostHierarchy&& H, const lina_amg_params& p) {
     prm_ = p;
     H_ = std::move(H);
+    tuned_.clear();
     n_ = H_.lv.back().A.n;
     colours_.assign(H_.lv.size(), std::vector<int>());
     ncolours_.assign(H_.lv.size(), 0);
@@ -804,7 +882,9 @@ void Solver::upload() {
         d.n = h.A.n;
         maxn = std::max(maxn, d.n);
         const std::vector<int>* segl = seg_off_.empty() ? nullptr : &seg_off_[l];
-        maxblk = std::max(maxblk, upload_pair(h.A, d.A, d.Af, B, st, segl, !fixed_order(), l == depth - 1));
+        TunedLanes tl;
+        maxblk = std::max(maxblk, upload_pair(h.A, d.A, d.Af, B, st, segl, !fixed_order(), l == depth - 1,
+                                              tuned_lanes(l, 'A', tl)));
         d.x = dalloc<double>(d.n, B);
         d.f = dalloc<double>(d.n, B);
         d.r = dalloc<double>(d.n, B);
@@ -819,9 +899,10 @@ void Solver::upload() {
             up_[l].ci = h.A.ci;
         }
         if (l == 0) continue;
-        maxblk = std::max(maxblk, upload_pair(h.P, d.P, d.Pf, B, st, segl, !fixed_order(), false));
+        maxblk = std::max(maxblk, upload_pair(h.P, d.P, d.Pf, B, st, segl, !fixed_order(), false,
+                                              tuned_lanes(l, 'P', tl)));
         maxblk = std::max(maxblk, upload_pair(h.R, d.R, d.Rf, B, st, seg_off_.empty() ? nullptr : &seg_off_[l - 1],
-                                              !fixed_order(), false));
+                                              !fixed_order(), false, tuned_lanes(l, 'R', tl)));
         // colour-permuted copy for the multicolour sweeps
         const std::vector<int>& col = colours_[l];
         int nc = ncolours_[l];
@@ -839,13 +920,16 @@ void Solver::upload() {
             starts.push_back(d.n);
             return starts;
         };
-        PairPlan q = plan_colours(Ac, d.colour_rows, !fixed_order());
+        const TunedLanes* tuned = tuned_lanes(l, 'C', tl);
+        PairPlan q = plan_colours(Ac, d.colour_rows, !fixed_order(), tuned);
         if (q.p64.head.empty()) q.s64 = colour_schedule(dev::block_nnz<double>(), d.colour_blk);
         else d.colour_blk = q.p64.group;
         if (q.p32.head.empty()) q.s32 = colour_schedule(dev::block_nnz<float>(), d.colour_blk32);
         else d.colour_blk32 = q.p32.group;
         upload_mat<double, double>(Ac, q.p64, q.s64, d.Ac, B, st, nullptr, false, nullptr, perm.data(), segl);
         upload_mat(Ac, q.p32, q.s32, d.Acf, B, st, &d.Ac, q.shared, &q.s64, perm.data(), segl);
+        if (tuned && !d.Ac.sl.ns) d.Ac.lpr = tuned->l64;
+        if (tuned && !d.Acf.sl.ns) d.Acf.lpr = tuned->l32;
         d.perm = dupload(perm, B, st);
         d.ncolours = nc;
         if (track_) {
@@ -977,7 +1061,8 @@ void Solver::upload() {
     dev::fill(st, dev::S_COUNT, scal_, 0.0);
     hip_check(hipStreamSynchronize(st), "upload sync");
     ensure_ctiles();
-    if (prm_.autotune) autotune();
+    // the tuner's layouts take a second upload; later uploads keep its choices
+    if (prm_.autotune && tuned_.empty() && autotune()) upload();
 }
 
 void Solver::set_params(const lina_amg_params& p) { prm_ = p; }
@@ -1846,7 +1931,7 @@ static bool same_cycle(const lina_amg_params& a, const lina_amg_params& b) {
     auto key = [](const lina_amg_params& p) {
         return std::make_tuple(p.dof, p.depth, p.smoothing_iterations, p.aggr_smoothing_iterations, p.coarsening,
                                p.smoother, p.omega, p.amg_eps, p.amg_max_iter, p.zero_init, p.precision,
-                               p.coarse_smoother, p.coarse_sweeps, p.cycle, p.skip_levels);
+                               p.coarse_smoother, p.coarse_sweeps, p.autotune, p.cycle, p.skip_levels);
     };
     return key(a) == key(b);
 }

@@ -164,8 +164,14 @@ struct DevLevel {
     float *xf = nullptr, *ff = nullptr, *rf = nullptr, *xof = nullptr;
 };
 
+// lanes a row of a matrix's FP64 and FP32 copies as the autotuner chose them, and
+// whether they are those of slices (else of row blocks)
+struct TunedLanes {
+    int l64 = 1, l32 = 1;
+    bool s64 = false, s32 = false;
+};
 int upload_pair(const Csr& A0, dev::DMat<double>& D, dev::DMat<float>& F, DevBuffers& B, hipStream_t st,
-                const std::vector<int>* seg, bool free32, bool partials);
+                const std::vector<int>* seg, bool free32, bool partials, const TunedLanes* tuned = nullptr);
 // the slices that upload_pair's FP64 or FP32 copy of A (colours: of A with its
 // rows colour by colour) reads (none: row blocks), log2 of the lanes a row and
 // the steps its values are stored for; no device needed
@@ -236,11 +242,12 @@ class Solver {
     // a hierarchy built elsewhere (the block-diagonal union of a batch)
     void set_hierarchy(HostHierarchy&& H, const lina_amg_params& p);
     // row-partition autotuning (run by upload when params.autotune != 0)
-    void autotune();
+    bool autotune();
     struct Tuned {
         int level;
         char which;  // A, P, R, C (colour-permuted copy of A)
         int lpr64, lpr32;
+        bool s64, s32;  // lanes of slices (else of row blocks)
     };
     const std::vector<Tuned>& tuned() const { return tuned_; }
     void upload();
@@ -267,7 +274,8 @@ class Solver {
     // 403 iterations and 1e-10 to 1e-8 of the solution over orders of one dot
     // product).  Those hierarchies keep one order of every FP32 row sum and of
     // the outer product's partials, whatever form the matrices have.
-    bool fixed_order() const { return prm_.coarsening == LINA_COARSEN_AGGRESSIVE; }
+    // Not with autotune, whose caller has freed the order.
+    bool fixed_order() const { return prm_.coarsening == LINA_COARSEN_AGGRESSIVE && !prm_.autotune; }
     const std::vector<int>& colours(int l) const { return colours_.at(l); }
     bool uploaded() const { return bufs_ != nullptr; }
     int n() const { return n_; }
@@ -359,10 +367,15 @@ class Solver {
     double* cpiv_ = nullptr;
     bool fused_gather() const;
     void ensure_ctiles();
-    template <typename VT, typename XT>
-    int tune_spmv(dev::DMat<VT>& M, const XT* x, XT* y);
-    template <typename VT, typename XT>
-    int tune_mcsor(DevLevel& d, dev::DMat<VT>& Ac, const XT* f, XT* x);
+    struct Form {
+        int lanes;
+        bool sliced;
+    };
+    template <typename VT>
+    Form tune_form(const Csr& A, const std::vector<int>& groups, const dev::DMat<VT>& M,
+                   const std::vector<int>& offsets,
+                   const std::function<void(const dev::DMat<VT>&, const std::vector<int>&)>& run);
+    const TunedLanes* tuned_lanes(int l, char which, TunedLanes& t) const;
     std::vector<Tuned> tuned_;
     std::vector<std::vector<int>> seg_off_;
     const double* seg_active_ = nullptr;

@@ -169,3 +169,37 @@ def test_recomputed_copies_are_those_of_a_fresh_upload(gpu, kind, coarsening, sm
     a.close()
     b.close()
 
+
+@pytest.mark.parametrize("prec", ["fp64", "mixed"])
+def test_autotuned_forms(gpu, prec):
+    """autotune times the lanes of sliced copies too: on coarse levels with a few
+    hundred long rows others than the rule's (8 or 16) are twice as fast.  What it
+    chooses multiplies, smooths and follows a recompute like any other form."""
+    from fem_amd import problems as P
+    s = P.degraded_elasticity(129)
+    prm = gpu.params("vcycle", 2, 5, precision=prec, autotune=1)
+    amg = gpu.AMG(s.rowptr, s.col, s.val, prm)
+    tuned = amg.tuned()
+    print("tuned", prec, tuned, flush=True)
+    assert len(tuned) == 4 * amg.depth - 3 and all(t[2] in (1, 4, 8, 16, 32) and t[3] in (1, 4, 8, 16, 32) for t in tuned)
+    rng = np.random.default_rng(12)
+    other = 0
+    for l in range(amg.depth):
+        rp, ci, v = amg.level(l)["A"]
+        m = np.diff(rp)
+        rule = [1, 4, 8, 16, 32][int(np.searchsorted([24, 48, 96, 192], m.mean()))]
+        other += sum(t[3] != rule for t in tuned if t[0] == l and t[1] in "AC")
+        x = rng.standard_normal(len(m))
+        prod = v * x[ci]
+        ref, bound = np.add.reduceat(prod, rp[:-1]), np.add.reduceat(np.abs(prod), rp[:-1])
+        assert np.all(np.abs(amg.spmv(x, l) - ref) <= 2 * (m + 1) * 2.0 ** -53 * bound)
+        assert np.all(np.abs(amg.spmv(x, l, "mixed") - ref) <= (m + 4) * 2.0 ** -24 * bound)
+    assert other > 0
+    b = rng.standard_normal(s.n)
+    A = s.scipy().tocsr()
+    for scale in (1.0, 1.7):
+        got = amg.pcg(b, tol=1e-9, max_iter=3000, stop="relres")
+        assert np.linalg.norm(scale * (A @ got["x"]) - b) <= 1e-7 * np.linalg.norm(b)
+        assert amg.tuned() == tuned
+        amg.recompute(1.7 * s.val)
+    amg.close()
