@@ -117,6 +117,21 @@ DevBuffers::~DevBuffers() {
     for (void* p : ptrs) (void)hipFree(p);
 }
 
+DevBuffers& DevBuffers::operator=(DevBuffers&& o) {
+    std::swap(ptrs, o.ptrs);
+    std::swap(chunk, o.chunk);
+    std::swap(left, o.left);
+    return *this;
+}
+
+void DevBuffers::drop(void* p, size_t bytes) {
+    if (bytes <= SHARED_MAX) return;  // part of a shared allocation
+    const auto it = std::find(ptrs.begin(), ptrs.end(), p);
+    if (it == ptrs.end()) return;
+    (void)hipFree(p);
+    ptrs.erase(it);
+}
+
 // row-block schedule over rows [begin, end): at most max_nnz products and
 // max_rows rows per block; a row longer than max_nnz gets a block alone.
 // (Blocks of up to 1024 rows for the prolongations, a few entries a row,
@@ -401,23 +416,29 @@ static int slice_unroll(double mean_steps) {
     return (w + 6) / 7 * 7 < (w + 7) / 8 * 8 ? 7 : 8;
 }
 
+// D.sl's fields from the plan.  Large streams are loaded nontemporally: FP64
+// from 64 MB (read once per Krylov iteration; 2.1M rows x 14, 79 -> 69 us, 1.05M
+// x 7, 22.0 -> 20.4 us), FP32 from 128 MB (2.1M x 14, 40 -> 37 us; smaller ones
+// stay in the last-level cache between sweeps and lose: 403k x 14, 8.6 -> 9.1 us).
+template <typename VT>
+static dev::Slices<VT> slice_shape(const SlicePlan& p) {
+    dev::Slices<VT> S;
+    S.ns = (int)p.head.size();
+    S.lt = p.lt;
+    S.steps = p.steps;
+    S.unroll = slice_unroll((double)S.steps / std::max(S.ns, 1));
+    S.nt = S.steps * 64 * (sizeof(VT) + 2) >= (sizeof(VT) == 8 ? 64u << 20 : 128u << 20);
+    return S;
+}
+
 // D.sl from the plan (D's CSR uploaded); share: the other precision's copy of
-// the same plan (same_rows), whose heads and codes are reused.  Large streams are loaded nontemporally:
-// FP64 from 64 MB (read once per Krylov iteration; 2.1M rows x 14, 79 -> 69
-// us, 1.05M x 7, 22.0 -> 20.4 us), FP32 from 128 MB (2.1M x 14, 40 -> 37 us;
-// smaller ones stay in the last-level cache between sweeps and lose: 403k x
-// 14, 8.6 -> 9.1 us).
+// the same plan (same_rows), whose heads and codes are reused.
 template <typename VT, typename OT>
 static void make_slices(const SlicePlan& p, dev::DMat<VT>& D, DevBuffers& B, hipStream_t st,
                         const dev::DMat<OT>* share) {
     dev::Slices<VT>& S = D.sl;
-    S = dev::Slices<VT>();
+    S = slice_shape<VT>(p);
     if (p.head.empty()) return;
-    S.ns = (int)p.head.size();
-    S.lt = p.lt;
-    S.steps = p.steps;
-    S.unroll = slice_unroll((double)S.steps / S.ns);
-    S.nt = S.steps * 64 * (sizeof(VT) + 2) >= (sizeof(VT) == 8 ? 64u << 20 : 128u << 20);
     if (share && (share->sl.ns != S.ns || share->sl.lt != S.lt || share->sl.steps != S.steps))
         throw std::logic_error("slices shared between different plans");
     S.v = dalloc<VT>(S.steps * 64, B);
@@ -439,6 +460,14 @@ bool slice_matrix(const Csr& A, dev::DMat<double>& D, DevBuffers& B, hipStream_t
     const SlicePlan p = rule_slices(A, {}, false, true);  // the ILU's Krylov loops take no partials from it
     make_slices<double, double>(p, D, B, st, nullptr);
     return D.sl.ns > 0;
+}
+
+// the slices' first rows, ending with A.n
+static std::vector<int> slice_starts(const Csr& A, const SlicePlan& p) {
+    std::vector<int> first;
+    for (const dev::SliceHead& k : p.head) first.push_back(k.row0);
+    first.push_back(A.n);
+    return first;
 }
 
 // plan: the slices (none: empty), starts_with_end: the row blocks (none:
@@ -486,12 +515,8 @@ static void upload_mat(const Csr& A, const SlicePlan& plan, const std::vector<in
         D.lpr = dev::lanes_per_row(A.n > 0 ? (double)A.nnz() / A.n : 0.0);
     }
     if (!plan.head.empty()) make_slices<VT, OT>(plan, D, B, st, share_slices ? share : nullptr);
-    if (seg) {  // the systems of each slice, or of each block where there are no slices
-        std::vector<int> first;
-        for (const dev::SliceHead& k : plan.head) first.push_back(k.row0);
-        if (!first.empty()) first.push_back(A.n);
-        D.bspec = dupload(block_systems(first.empty() ? starts_with_end : first, *seg, row_ids), B, st);
-    }
+    if (seg)  // the systems of each slice, or of each block where there are no slices
+        D.bspec = dupload(block_systems(plan.head.empty() ? starts_with_end : slice_starts(A, plan), *seg, row_ids), B, st);
     // diagonal positions (row r's own index: row_ids == nullptr) and l1 norms
     std::vector<int> dpos(A.n, -1);
     std::vector<VT> l1(A.n, (VT)0);
@@ -713,15 +738,33 @@ namespace {
 constexpr int kLaneCandidates[] = {1, 4, 8, 16, 32};
 }
 
+// device arrays that the candidates of one tuning are laid out in, one after another
+struct Solver::SliceScratch {
+    DevBuffers bufs;
+    size_t heads = 0, entries = 0;
+    dev::SliceHead* head = nullptr;
+    uint16_t* cs = nullptr;
+    double* v = nullptr;  // or as many floats
+    void hold(size_t nh, size_t ne) {
+        if (nh <= heads && ne <= entries) return;
+        heads = std::max(nh, 2 * heads);
+        entries = std::max(ne, 2 * entries);
+        bufs = DevBuffers();  // the last candidate's timing has ended
+        head = dalloc<dev::SliceHead>(heads, bufs);
+        cs = dalloc<uint16_t>(entries, bufs);
+        v = dalloc<double>(entries, bufs);
+    }
+};
+
 // The form of M (rows: A's) whose launches are fastest: a sliced copy with each
 // lane count, laid out in scratch memory, and the row blocks with each where M
 // has them.  groups: a colour-permuted copy's (offsets: its sweep's offsets of
 // slices or blocks).  What M has stays unless another is 3 % faster.
 template <typename VT>
 Solver::Form Solver::tune_form(const Csr& A, const std::vector<int>& groups, const dev::DMat<VT>& M,
-                               const std::vector<int>& offsets,
+                               const std::vector<int>& offsets, SliceScratch& scratch,
                                const std::function<void(const dev::DMat<VT>&, const std::vector<int>&)>& run) {
-    const Form have = {M.sl.ns ? 1 << M.sl.lt : M.lpr, M.sl.ns > 0};
+    const Form have = form_of(M);
     if (M.n == 0 || M.nnz == 0) return have;
     auto timed = [&](const dev::DMat<VT>& T, const std::vector<int>& off) {
         run(T, off);
@@ -746,6 +789,7 @@ Solver::Form Solver::tune_form(const Csr& A, const std::vector<int>& groups, con
         }
     };
     for (int lanes : kLaneCandidates) {
+        if (lanes > 4 && (double)lanes * M.n > M.nnz) break;  // less than an entry a lane
         if (!have.sliced && lanes != have.lanes) {
             dev::DMat<VT> T = M;
             T.lpr = lanes;
@@ -755,75 +799,118 @@ Solver::Form Solver::tune_form(const Csr& A, const std::vector<int>& groups, con
         const SlicePlan p = plan_slices(A, groups, log2_of(lanes));
         if (p.head.empty()) continue;
         validate(A, p);
-        DevBuffers scratch;
+        scratch.hold(p.head.size(), p.steps * 64);
         dev::DMat<VT> T = M;
         T.bspec = nullptr;
-        make_slices<VT, VT>(p, T, scratch, stream_, nullptr);
+        T.sl = slice_shape<VT>(p);
+        T.sl.head = scratch.head;
+        T.sl.cs = scratch.cs;
+        T.sl.v = (VT*)scratch.v;
+        hip_check(hipMemcpyAsync(T.sl.head, p.head.data(), p.head.size() * sizeof(dev::SliceHead),
+                                 hipMemcpyHostToDevice, stream_), "h2d");
+        dev::slice_columns<VT>(stream_, T);
+        dev::slice_values<VT>(stream_, T);
         keep(timed(T, p.group), {lanes, true});
-        hip_check(hipStreamSynchronize(stream_), "autotune");  // the scratch slices die here
     }
     return best;
+}
+
+// M in another form; share: the other precision's copy where it has that form
+template <typename VT, typename OT>
+void Solver::adopt_form(const Csr& A, const std::vector<int>& groups, dev::DMat<VT>& M, Form f,
+                        const dev::DMat<OT>* share, std::vector<int>* offsets, const std::vector<int>* seg,
+                        const int* row_ids) {
+    if (!f.sliced) {  // only where M has row blocks already
+        M.lpr = f.lanes;
+        return;
+    }
+    const SlicePlan p = plan_slices(A, groups, log2_of(f.lanes));
+    make_slices<VT, OT>(p, M, *bufs_, stream_, share);
+    if (offsets) *offsets = p.group;
+    if (seg) M.bspec = dupload(block_systems(slice_starts(A, p), *seg, row_ids), *bufs_, stream_);
+    hip_check(hipStreamSynchronize(stream_), "adopt");  // the host plan dies here
+}
+
+// both copies of a matrix in the forms timed fastest; the slices that neither
+// reads any more are freed
+void Solver::adopt_forms(const Csr& A, const std::vector<int>& groups, dev::DMat<double>& D, dev::DMat<float>& F,
+                         Form a, Form b, std::vector<int>* off64, std::vector<int>* off32,
+                         const std::vector<int>* seg, const int* row_ids) {
+    const dev::Slices<double> d0 = D.sl;
+    const dev::Slices<float> f0 = F.sl;
+    auto same = [](Form x, Form y) { return x.sliced == y.sliced && x.lanes == y.lanes; };
+    if (!same(a, form_of(D))) adopt_form<double, double>(A, groups, D, a, nullptr, off64, seg, row_ids);
+    if (!same(b, form_of(F)))
+        adopt_form<float, double>(A, groups, F, b, same(a, b) && a.sliced ? &D : nullptr, off32, seg, row_ids);
+    auto drop = [&](void* p, size_t bytes) {
+        if (p) bufs_->drop(p, bytes);
+    };
+    if (D.sl.head != d0.head && F.sl.head != d0.head) drop(d0.head, d0.ns * sizeof(dev::SliceHead));
+    if (f0.head != d0.head && F.sl.head != f0.head) drop(f0.head, f0.ns * sizeof(dev::SliceHead));
+    if (D.sl.v != d0.v) drop(d0.v, d0.steps * 64 * sizeof(double));
+    if (F.sl.v != f0.v) drop(f0.v, f0.steps * 64 * sizeof(float));
+    if (D.sl.cs != d0.cs && F.sl.cs != d0.cs) drop(d0.cs, d0.steps * 64 * sizeof(uint16_t));
+    if (f0.cs != d0.cs && F.sl.cs != f0.cs) drop(f0.cs, f0.steps * 64 * sizeof(uint16_t));
 }
 
 // The row partition (slices or row blocks, lanes per row) of every matrix of the
 // hierarchy, chosen by timing each candidate on the device: the SpMV-shaped kernels (residual,
 // restriction, prolongation, Jacobi) take their matrix's choice, the
-// multicolour sweeps the colour-permuted copy's.  True when a matrix should
-// have another than it has.
-bool Solver::autotune() {
+// multicolour sweeps the colour-permuted copy's.
+void Solver::autotune() {
     hipStream_t st = stream_;
     tuned_.clear();
-    bool other = false;
-    auto differs = [](const auto& M, Form f) {
-        return f.sliced != (M.sl.ns > 0) || f.lanes != (M.sl.ns ? 1 << M.sl.lt : M.lpr);
-    };
-    auto note = [&](int l, char which, const dev::DMat<double>& D, const dev::DMat<float>& F, Form a, Form b) {
+    SliceScratch scratch;
+    auto note = [&](int l, char which, Form a, Form b) {
         tuned_.push_back({l, which, a.lanes, b.lanes, a.sliced, b.sliced});
-        other = other || differs(D, a) || differs(F, b);
     };
-    auto product = [&](int l, char which, const Csr& M0, const dev::DMat<double>& D, const dev::DMat<float>& F,
-                       const double* x, double* y, const float* xf, float* yf) {
+    auto product = [&](int l, char which, const Csr& M0, dev::DMat<double>& D, dev::DMat<float>& F, const double* x,
+                       double* y, const float* xf, float* yf, const std::vector<int>* seg) {
         const Csr M = which == 'A' ? Csr() : drop_outside_zeros(M0);  // A has none
         const Csr& A = which == 'A' ? M0 : M;
-        const Form a = tune_form<double>(A, {}, D, {}, [&](const dev::DMat<double>& T, const std::vector<int>&) {
+        const Form a = tune_form<double>(A, {}, D, {}, scratch,
+                                         [&](const dev::DMat<double>& T, const std::vector<int>&) {
             dev::spmv<double, double>(st, T, x, nullptr, y, dev::MODE_SET, nullptr, nullptr);
         });
-        const Form b = tune_form<float>(A, {}, F, {}, [&](const dev::DMat<float>& T, const std::vector<int>&) {
+        const Form b = tune_form<float>(A, {}, F, {}, scratch,
+                                        [&](const dev::DMat<float>& T, const std::vector<int>&) {
             dev::spmv<float, float>(st, T, xf, nullptr, yf, dev::MODE_SET, nullptr, nullptr);
         });
-        note(l, which, D, F, a, b);
+        adopt_forms(A, {}, D, F, a, b, nullptr, nullptr, seg, nullptr);
+        note(l, which, a, b);
     };
+    auto segs = [&](size_t l) { return seg_off_.empty() ? nullptr : &seg_off_[l]; };
     for (size_t l = 0; l < L_.size(); l++) {
         DevLevel& d = L_[l];
         const HostLevel& h = H_.lv[l];
         for (double* v : {d.x, d.f, d.r, d.xo}) dev::fill<double>(st, d.n, v, 1.0);
         for (float* v : {d.xf, d.ff, d.rf, d.xof}) dev::fill<float>(st, d.n, v, 1.0f);
-        product((int)l, 'A', h.A, d.A, d.Af, d.x, d.r, d.xf, d.rf);
+        product((int)l, 'A', h.A, d.A, d.Af, d.x, d.r, d.xf, d.rf, segs(l));
         if (l == 0) continue;
         DevLevel& c = L_[l - 1];
         for (double* v : {c.x, c.f}) dev::fill<double>(st, c.n, v, 1.0);
         for (float* v : {c.xf, c.ff}) dev::fill<float>(st, c.n, v, 1.0f);
-        product((int)l, 'P', h.P, d.P, d.Pf, c.x, d.r, c.xf, d.rf);
-        product((int)l, 'R', h.R, d.R, d.Rf, d.r, c.f, d.rf, c.ff);
+        product((int)l, 'P', h.P, d.P, d.Pf, c.x, d.r, c.xf, d.rf, segs(l));
+        product((int)l, 'R', h.R, d.R, d.Rf, d.r, c.f, d.rf, c.ff, segs(l - 1));
         dev::fill<double>(st, d.n, d.f, 0.0);
         dev::fill<float>(st, d.n, d.ff, 0.0f);
         if (d.ncolours == 0) continue;
         std::vector<int> perm, rows;
         const Csr Ac = colour_permuted(h.A, colours_[l], ncolours_[l], perm, rows);
-        const Form a = tune_form<double>(Ac, rows, d.Ac, d.colour_blk,
+        const Form a = tune_form<double>(Ac, rows, d.Ac, d.colour_blk, scratch,
                                          [&](const dev::DMat<double>& T, const std::vector<int>& cb) {
             for (int c = 0; c < d.ncolours; c++)
                 dev::mcsor_colour(st, T, cb[c], cb[c + 1] - cb[c], d.perm, (const double*)d.f, d.x, 1.0);
         });
-        const Form b = tune_form<float>(Ac, rows, d.Acf, d.colour_blk32,
+        const Form b = tune_form<float>(Ac, rows, d.Acf, d.colour_blk32, scratch,
                                         [&](const dev::DMat<float>& T, const std::vector<int>& cb) {
             for (int c = 0; c < d.ncolours; c++)
                 dev::mcsor_colour(st, T, cb[c], cb[c + 1] - cb[c], d.perm, (const float*)d.ff, d.xf, 1.0f);
         });
-        note((int)l, 'C', d.Ac, d.Acf, a, b);
+        adopt_forms(Ac, rows, d.Ac, d.Acf, a, b, &d.colour_blk, &d.colour_blk32, segs(l), perm.data());
+        note((int)l, 'C', a, b);
     }
     hip_check(hipStreamSynchronize(st), "autotune");
-    return other;
 }
 
 // the autotuner's lanes of a matrix, or nullptr before it has run
@@ -1061,8 +1148,7 @@ void Solver::upload() {
     dev::fill(st, dev::S_COUNT, scal_, 0.0);
     hip_check(hipStreamSynchronize(st), "upload sync");
     ensure_ctiles();
-    // the tuner's layouts take a second upload; later uploads keep its choices
-    if (prm_.autotune && tuned_.empty() && autotune()) upload();
+    if (prm_.autotune && tuned_.empty()) autotune();  // later uploads keep its choices
 }
 
 void Solver::set_params(const lina_amg_params& p) { prm_ = p; }

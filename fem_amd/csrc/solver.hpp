@@ -75,10 +75,17 @@ class Captured {
 };
 
 struct DevBuffers {
+    static constexpr size_t SHARED_MAX = 64 << 10;  // larger arrays have an allocation each
     std::vector<void*> ptrs;
     char* chunk = nullptr;  // the rest of the last shared allocation of small arrays
     size_t left = 0;
+    DevBuffers() = default;
+    DevBuffers(const DevBuffers&) = delete;
+    DevBuffers& operator=(const DevBuffers&) = delete;
+    DevBuffers& operator=(DevBuffers&& o);
     ~DevBuffers();
+    // frees an array of dalloc's that nothing uses any more (a small one stays)
+    void drop(void* p, size_t bytes);
 };
 
 // device arrays owned by a DevBuffers (freed with it).  Arrays up to 64 KB
@@ -88,7 +95,7 @@ template <typename T>
 T* dalloc(size_t n, DevBuffers& owner) {
     if (n == 0) n = 1;
     const size_t bytes = n * sizeof(T), shared = 1 << 20;
-    if (bytes > (64u << 10)) {
+    if (bytes > DevBuffers::SHARED_MAX) {
         void* p = nullptr;
         hip_check(hipMalloc(&p, bytes), "hipMalloc");
         owner.ptrs.push_back(p);
@@ -242,7 +249,7 @@ class Solver {
     // a hierarchy built elsewhere (the block-diagonal union of a batch)
     void set_hierarchy(HostHierarchy&& H, const lina_amg_params& p);
     // row-partition autotuning (run by upload when params.autotune != 0)
-    bool autotune();
+    void autotune();
     struct Tuned {
         int level;
         char which;  // A, P, R, C (colour-permuted copy of A)
@@ -372,9 +379,21 @@ class Solver {
         bool sliced;
     };
     template <typename VT>
+    static Form form_of(const dev::DMat<VT>& M) {
+        return {M.sl.ns ? 1 << M.sl.lt : M.lpr, M.sl.ns > 0};
+    }
+    struct SliceScratch;
+    template <typename VT>
     Form tune_form(const Csr& A, const std::vector<int>& groups, const dev::DMat<VT>& M,
-                   const std::vector<int>& offsets,
+                   const std::vector<int>& offsets, SliceScratch& scratch,
                    const std::function<void(const dev::DMat<VT>&, const std::vector<int>&)>& run);
+    template <typename VT, typename OT>
+    void adopt_form(const Csr& A, const std::vector<int>& groups, dev::DMat<VT>& M, Form f,
+                    const dev::DMat<OT>* share, std::vector<int>* offsets, const std::vector<int>* seg,
+                    const int* row_ids);
+    void adopt_forms(const Csr& A, const std::vector<int>& groups, dev::DMat<double>& D, dev::DMat<float>& F, Form a,
+                     Form b, std::vector<int>* off64, std::vector<int>* off32, const std::vector<int>* seg,
+                     const int* row_ids);
     const TunedLanes* tuned_lanes(int l, char which, TunedLanes& t) const;
     std::vector<Tuned> tuned_;
     std::vector<std::vector<int>> seg_off_;
