@@ -1788,10 +1788,15 @@ __global__ __launch_bounds__(TPB) void k_tri_level(const TriLevel L, const doubl
     }
 }
 
-__global__ void k_tri_gather(long n, const int* __restrict__ map, const double* __restrict__ v,
-                             double* __restrict__ val) {
-    for (long q = blockIdx.x * blockDim.x + threadIdx.x; q < n; q += gridDim.x * blockDim.x)
-        val[q] = map[q] >= 0 ? v[map[q]] : 0.0;
+__global__ void k_tri_gather(const TriFills fills) {
+#pragma unroll
+    for (int k = 0; k < TRI_FILLS; k++) {
+        const TriFill& f = fills.f[k];
+        for (long q = blockIdx.x * blockDim.x + threadIdx.x; q < f.n; q += gridDim.x * blockDim.x) {
+            const int p = f.map[q];
+            f.val[q] = p >= 0 ? f.v[p] : 0.0;
+        }
+    }
 }
 
 __global__ __launch_bounds__(TPB) void k_ipcg_p(int n, int first, double* __restrict__ P, const double* __restrict__ Z,
@@ -3312,10 +3317,11 @@ void tri_level(hipStream_t st, const TriLevel& L, const double* in, double* out,
         hipLaunchKernelGGL(k_tri_level, dim3(tri_level_blocks(L)), dim3(TPB), 0, st, L, in, out, ud, w, r, part);
 }
 
-void tri_values(hipStream_t st, long n, const int* map, const double* v, double* val) {
+void tri_values(hipStream_t st, const TriFills& fills) {
+    long n = 0;
+    for (const TriFill& f : fills.f) n = std::max(n, f.n);
     if (n <= 0) return;
-    const int g = grid_for((int)std::min(n, 1L << 30));
-    hipLaunchKernelGGL(k_tri_gather, dim3(g), dim3(TPB), 0, st, n, map, v, val);
+    hipLaunchKernelGGL(k_tri_gather, dim3(grid_for((int)std::min(n, 1L << 30))), dim3(TPB), 0, st, fills);
 }
 
 void ipcg_p(hipStream_t st, int n, int first, double* P, const double* Z, double* scal, const double* rz, int nrz,

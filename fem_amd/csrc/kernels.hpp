@@ -429,8 +429,19 @@ int tri_level_blocks(const TriLevel& L);
 // partials of r_i times the rows' final results (w_i, or out_i without w).
 void tri_level(hipStream_t st, const TriLevel& L, const double* in, double* out, const double* ud, double* w,
                const double* r, double* part);
-// val[q] = v[map[q]] (map < 0: 0) for the padded entries and diagonals of a factor
-void tri_values(hipStream_t st, long n, const int* map, const double* v, double* val);
+// val[q] = v[map[q]] (map < 0: 0), q < n, for the padded entries and diagonals of
+// both factors, in one launch
+struct TriFill {
+    long n = 0;
+    const int* map = nullptr;
+    const double* v = nullptr;
+    double* val = nullptr;
+};
+constexpr int TRI_FILLS = 5;
+struct TriFills {
+    TriFill f[TRI_FILLS];
+};
+void tri_values(hipStream_t st, const TriFills& fills);
 
 // ILU-pcg on the device (IluSystem::pcg_core), its sums as in pcg_direction
 enum { IS_S = 0, IS_RZ = 1, IS_PQ = 2, IS_RR = 3, IS_STOP = 4, IS_IT = 5, IS_R = 6, IS_R0 = 7, IS_TOL = 8,

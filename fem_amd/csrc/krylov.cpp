@@ -616,13 +616,12 @@ void IluSystem::upload(bool pattern_levels_in) {
 }
 
 void IluSystem::pack_values() {
-    if (wide_) {
-        dev::tri_values(stream_, wl_.nval, wl_.vmap, dL_.v, wl_.val);
-        dev::tri_values(stream_, n_, wl_.dmap, dL_.v, wl_.diag);
-        dev::tri_values(stream_, wu_.nval, wu_.vmap, dU_.v, wu_.val);
-        dev::tri_values(stream_, n_, wu_.dmap, dU_.v, wu_.diag);
-        dev::tri_values(stream_, n_, udmap_, dU_.v, ud_);
-    }
+    if (wide_)
+        dev::tri_values(stream_, {{{(long)wl_.nval, wl_.vmap, dL_.v, wl_.val},
+                                   {n_, wl_.dmap, dL_.v, wl_.diag},
+                                   {(long)wu_.nval, wu_.vmap, dU_.v, wu_.val},
+                                   {n_, wu_.dmap, dU_.v, wu_.diag},
+                                   {n_, udmap_, dU_.v, ud_}}});
     if (!packed_) return;
     dev::tri_pack_values(stream_, n_, tf_.p.maxp, tf_.vmap, tf_.dmap, tf_.nov, tf_.ovmap, dL_.v, tf_.rec, tf_.ovval);
     dev::tri_pack_values(stream_, n_, tb_.p.maxp, tb_.vmap, tb_.dmap, tb_.nov, tb_.ovmap, dU_.v, tb_.rec, tb_.ovval);

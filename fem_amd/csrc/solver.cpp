@@ -357,8 +357,10 @@ static SlicePlan plan_slices(const Csr& A, const std::vector<int>& groups, int l
 // 7.7, 12.4; 638k, 407, 16.2, 37.1; 1.5M, 148, 11.3, 15.6; the other side 506k,
 // 26 steps, 8.5, 4.9; 986k, 65, 12.1, 8.2.  FP64 streams of long rows are a
 // little faster in blocks: 6.4M entries in rows of 95, 17.0, 19.5; 39M, 159,
-// 82, 97; but 1.7M, 95, 14.8, 7.1 and 7.8M, 53, 19.2, 19.6.
+// 82, 97; but 1.7M, 95, 14.8, 7.1 and 7.8M, 53, 19.2, 19.6.  A colour's sweep
+// loads its rows' places, then their right-hand sides first (base).
 static bool slices_pay(const Csr& A, const SlicePlan& p, bool fp64) {
+    const double base = p.group.size() > 2 ? 3.0 : 2.0;
     double slices = 0, blocks = 0;
     for (size_t g = 0; g + 1 < p.group.size(); g++) {
         int steps = 0;
@@ -367,7 +369,7 @@ static bool slices_pay(const Csr& A, const SlicePlan& p, bool fp64) {
             steps = std::max(steps, p.head[k].steps);
             ent += A.rp[p.head[k].row1] - A.rp[p.head[k].row0];
         }
-        slices += 2.0 + 0.72 * ((steps + 7) / 8);
+        slices += base + 0.72 * ((steps + 7) / 8);
         blocks += 4.0 + std::min(ent / 1e5, 8.0);
     }
     if (slices > blocks) return false;
