@@ -203,3 +203,65 @@ def test_autotuned_forms(gpu, prec):
         assert amg.tuned() == tuned
         amg.recompute(1.7 * s.val)
     amg.close()
+
+
+def spd(n, per_row, seed):
+    import scipy.sparse as sp
+    rng = np.random.default_rng(seed)
+    i, j = rng.integers(0, n, n * per_row // 2), rng.integers(0, n, n * per_row // 2)
+    A = sp.coo_matrix((-rng.uniform(0.1, 1.0, len(i)), (i, j)), shape=(n, n)).tocsr()
+    A = (A + A.T).tolil()
+    A.setdiag(0)
+    A = A.tocsr()
+    A = (A + sp.diags(np.asarray(abs(A).sum(axis=1)).ravel() + 0.5)).tocsr()
+    A.sort_indices()
+    return A
+
+
+def sweep(A, colours, smoother, x, f, backward):
+    d = A.diagonal()
+    if smoother == "jacobi":
+        return (f - (A @ x - d * x)) / d
+    if smoother == "l1_jacobi":
+        return x + (f - A @ x) / np.asarray(abs(A).sum(axis=1)).ravel()
+    x = x.copy()
+    order = range(colours.max() + 1)
+    for c in reversed(order) if backward else order:
+        r = np.flatnonzero(colours == c)
+        x[r] = (f[r] - (A[r] @ x - d[r] * x[r])) / d[r]
+    return x
+
+
+@pytest.mark.parametrize("system", [("damage", 8), ("damage", 9), ("damage", 16), ("damage", 17), ("damage", 129),
+                                    ("spd", 63, 10), ("spd", 65, 30), ("spd", 257, 40), ("spd", 700, 130),
+                                    ("spd", 1500, 260)])
+@pytest.mark.parametrize("smoother", ["jacobi", "l1_jacobi", "mc_sor", "mc_ssor"])
+def test_sliced_sweeps_match_numpy(gpu, system, smoother):
+    """a two-level V(1,1) cycle whose finest level is swept by slices of one and of
+    several lanes a row, against the same cycle in numpy on the hierarchy's own
+    matrices.  About 4 (m + 2) roundings an entry (m the longest row) in either
+    precision; the coarse solve multiplies them by its condition, below 1e3 here."""
+    import scipy.sparse as sp
+    from fem_amd import problems as P
+    print("sweeps", system, smoother, flush=True)
+    A = spd(*system[1:], seed=system[1]) if system[0] == "spd" else P.damage_system(system[1])[0].scipy().tocsr()
+    A.sort_indices()
+    n = A.shape[0]
+    amg = gpu.AMG(A.indptr, A.indices, A.data, gpu.params("vcycle", 1, 2))
+    lev, top = amg.level(0), amg.level(1)
+    csr = lambda m, shape: sp.csr_matrix((m[2], m[1], m[0]), shape=shape)
+    nc = lev["fine"]
+    keep = top["P"][1] < nc  # zero seeds of rows the reference leaves empty
+    Pm = sp.csr_matrix((top["P"][2] * keep, np.where(keep, top["P"][1], 0), top["P"][0]), shape=(n, nc))
+    Rm, Ac = csr(top["R"], (nc, n)), csr(lev["A"], (nc, nc)).toarray()
+    f = np.random.default_rng(1).standard_normal(n)
+    x = sweep(A, top["colours"], smoother, np.zeros(n), f, False)
+    x = x + Pm @ np.linalg.solve(Ac, Rm @ (f - A @ x))
+    x = sweep(A, top["colours"], smoother, x, f, smoother == "mc_ssor")
+    m = int(np.diff(A.indptr).max())
+    for prec, eps in (("fp64", 2.0 ** -53), ("mixed", 2.0 ** -24)):
+        amg.set_params(gpu.params("vcycle", 1, 2, smoother=smoother, coarse_smoother=-1, precision=prec))
+        it, got = amg.amg_solve(f, np.zeros(n))
+        assert it == 1
+        assert np.linalg.norm(got - x) <= 4e3 * (m + 2) * eps * np.linalg.norm(x), prec
+    amg.close()
