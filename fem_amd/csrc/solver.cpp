@@ -358,21 +358,26 @@ static SlicePlan plan_slices(const Csr& A, const std::vector<int>& groups, int l
 // 26 steps, 8.5, 4.9; 986k, 65, 12.1, 8.2.  FP64 streams of long rows are a
 // little faster in blocks: 6.4M entries in rows of 95, 17.0, 19.5; 39M, 159,
 // 82, 97; but 1.7M, 95, 14.8, 7.1 and 7.8M, 53, 19.2, 19.6.  A colour's sweep
-// loads its rows' places, then their right-hand sides first (base).
+// loads its rows' places, then their right-hand sides first (base).  Padding
+// costs where it is much: a prolongation of 2.1M rows, 9.4M entries, 1.47 read
+// an entry, FP64 35.5, 50.1, FP32 23.3, 24.7; 525k, 2.7M, 1.69, 12.4, 15.8; but
+// 1.05M, 2.5M, 1.49, 15.9, 10.7.
 static bool slices_pay(const Csr& A, const SlicePlan& p, bool fp64) {
     const double base = p.group.size() > 2 ? 3.0 : 2.0;
-    double slices = 0, blocks = 0;
+    double slices = 0, blocks = 0, read = 0;
     for (size_t g = 0; g + 1 < p.group.size(); g++) {
         int steps = 0;
         double ent = 0;
         for (int k = p.group[g]; k < p.group[g + 1]; k++) {
-            steps = std::max(steps, p.head[k].steps);
-            ent += A.rp[p.head[k].row1] - A.rp[p.head[k].row0];
+            const dev::SliceHead& h = p.head[k];
+            steps = std::max(steps, h.steps);
+            ent += A.rp[h.row1] - A.rp[h.row0];
+            read += ((double)h.steps * (h.row1 - h.row0)) * (1 << p.lt);
         }
         slices += base + 0.72 * ((steps + 7) / 8);
         blocks += 4.0 + std::min(ent / 1e5, 8.0);
     }
-    if (slices > blocks) return false;
+    if (slices > blocks || (read > 1.4 * A.nnz() && read - A.nnz() > 1.5e6)) return false;
     return !(fp64 && A.nnz() >= 4000000 && A.nnz() >= 90.0 * A.n);
 }
 

@@ -117,3 +117,13 @@ def test_large_fp64_matrices_of_long_rows_take_row_blocks(n, mean, sliced64):
     rp, ci = rows_with(np.full(n, mean), n)
     assert (len(lina.slice_layout(rp, ci, precision="fp64")[0]) > 0) == sliced64
     assert len(lina.slice_layout(rp, ci, precision="mixed")[0]) > 0
+
+
+@pytest.mark.parametrize("n,sliced", [(100_000, True), (1_000_000, False)])
+def test_large_padding_takes_row_blocks(n, sliced):
+    """prolongation-like rows of 2 to 8 entries: 1.6 entries read for one"""
+    m = np.random.default_rng(n).integers(2, 9, n)
+    rp, ci = rows_with(m, 1)
+    for precision in ("fp64", "mixed"):
+        heads, lanes, _ = lina.slice_layout(rp, ci, precision=precision)
+        assert (len(heads) > 0) == sliced
