@@ -172,7 +172,7 @@ def copy_gbs(lina, n=1 << 27, reps=5):
 def kernels_only(s, lina):
     """The launches the counter runs read: one copy of known size (the
     calibration of FETCH_SIZE / WRITE_SIZE) and the finest-level SpMVs, on a
-    device matrix handle (the same kernel and row blocks as the solver's)."""
+    device matrix handle (the same kernel and slices as the autotuned solver's)."""
     gbs = copy_gbs(lina, reps=3)
     m = lina.Matrix(s.rowptr, s.col, s.val)
     ms64 = m.time_spmv("fp64", reps=5)
@@ -619,6 +619,9 @@ def main():
     tuned = amg.tuned()
     lpr_top = [t for t in tuned if t[0] == amg.depth - 1 and t[1] == "A"]
     lpr64 = lpr_top[0][2] if lpr_top else 1
+    sliced = len(lina.slice_layout(s.rowptr, s.col, free32=True, partials=True)[0]) > 0
+    outer = f"k_sell_spmv<double, double, 3> (sliced copy, lanes a row: {lpr64})" if sliced \
+        else f"k_spmv<double, double, 3, {lpr64}>"
     log(f"AMG setup + upload {t_setup:.1f}s, level sizes {sizes}, autotuned row partitions {tuned}")
     prm32 = lina.params("vcycle", 2, args.depth, precision="mixed", coarse_sweeps=args.coarse_sweeps, autotune=1,
                         skip_levels=mask)
@@ -751,7 +754,7 @@ def main():
         "setup_s": t_setup,
         "roofline": {"bound": "hbm", "achieved": spmv_gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": spmv_gbs / HBM_PEAK_GBS, "traffic": measured_traffic(),
-                     "kernel": f"k_spmv<double, double, 3, {lpr64}> (finest-level A*p of the outer CG)",
+                     "kernel": f"{outer}: finest-level A*p of the outer CG",
                      "bytes_per_launch": spmv_bytes, "stored_bytes_per_launch": stored_bytes, "avg_ms": spmv_ms,
                      "launches": res["mixed"]["spmv_launches"],
                      "back_to_back_ms": b2b_ms, "back_to_back_gbs": spmv_bytes / (b2b_ms * 1e-3) / 1e9,
