@@ -136,10 +136,11 @@ def test_ilu_replays_keep_the_bits(gpu, m, ordering):
     f.close()
 
 
-@pytest.mark.parametrize("solver", ["amg", "ilu"])
-def test_an_iteration_more_costs_an_iteration(gpu, solver):
-    """no replays past the end where an iteration takes long: 49 iterations
-    against 48 (a solve of 49 took 8 % and 16 % longer when they started there)"""
+@pytest.mark.parametrize("solver,most", [("amg", 1.245), ("ilu", 1.3)])
+def test_iterations_past_the_end_are_not_paid_for(gpu, solver, most):
+    """49 iterations against 40, 1.22 times the work, took 1.27 and 1.38 times the
+    time when replays started at 48 wherever an iteration takes long; 1.21 and 1.22
+    without. The bounds lie between, the best of each length taken in turn"""
     if solver == "amg":
         s = P.poisson(513)
         h = gpu.AMG(s.rowptr, s.col, s.val, gpu.params("vcycle", 1, 6, precision="mixed"))
@@ -147,17 +148,14 @@ def test_an_iteration_more_costs_an_iteration(gpu, solver):
         s = P.poisson(257)
         h = gpu.ILU(s.rowptr, s.col, s.val)
     b = np.random.default_rng(1).standard_normal(s.n)
-
-    def run(limit):
-        best = 1e9
-        for _ in range(9):
+    best = {40: 1e9, 49: 1e9}
+    h.pcg(b, tol=0.0, max_iter=49, stop="relres")
+    for _ in range(15):
+        for limit in best:
             t = time.perf_counter()
             h.pcg(b, tol=0.0, max_iter=limit, stop="relres")
-            best = min(best, time.perf_counter() - t)
-        return best
-
-    run(48)
-    t48, t49 = run(48), run(49)
+            best[limit] = min(best[limit], time.perf_counter() - t)
     h.close()
-    print(solver, "48: %.2f ms, 49: %.2f ms" % (t48 * 1e3, t49 * 1e3), flush=True)
-    assert t49 <= 1.05 * t48
+    t40, t49 = best[40], best[49]
+    print(solver, "40: %.2f ms, 49: %.2f ms, %.3f" % (t40 * 1e3, t49 * 1e3, t49 / t40), flush=True)
+    assert t49 <= most * t40
